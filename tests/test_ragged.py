@@ -1,0 +1,88 @@
+"""Sizes and alignments that are nobody's choice: rows of odd length, views that start in the middle of a
+vector, edge tiles one element wide.  The elementwise results are IEEE operations on the same operands, so
+numpy gives the same bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [np.float32, np.float64]
+IDS = ["f32", "f64"]
+
+
+def same(got, exp, what):
+    assert got.shape == exp.shape and np.array_equal(got, exp), what
+
+
+def offset_matrix(hip, a, off):
+    """`a` in device memory `off` elements behind a 256-byte boundary"""
+    flat = np.concatenate([np.zeros(off, a.dtype), a.reshape(-1)])
+    m = hip.Matrix.from_numpy(flat)
+    return hip.Matrix(m.buf, off, a.shape, hip.default_stride(a.shape), a.dtype)
+
+
+# one element, around one vector, around the 32 / 64 tile edges and one row piece, a last tile of 1, 3, 4 and 63
+EDGES = [(1, 1), (1, 5), (3, 2), (4, 4), (5, 3), (31, 33), (33, 31), (63, 65), (64, 64), (65, 129), (127, 68), (196, 130), (67, 1025)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", EDGES, ids=str)
+def test_broadcast_and_transposed_operands(hip, dtype, shape):
+    r = np.random.default_rng(shape[0] * 7 + shape[1])
+    rows, cols = shape
+    for off in (0, 1, 3):
+        a, b = r.standard_normal(shape).astype(dtype), r.standard_normal((cols, rows)).astype(dtype)
+        row, col = r.standard_normal(cols).astype(dtype), r.standard_normal((rows, 1)).astype(dtype)
+        A, B, Row, Col = (offset_matrix(hip, t, o) for t, o in ((a, off), (b, 3 - off), (row, off // 2), (col, 1)))
+        out = offset_matrix(hip, np.zeros(shape, dtype), 2 if off else 0)
+        what = (shape, off)
+        out.add_array(A, Row)
+        same(out.to_numpy(), a + row, ("row", what))
+        out.sub_array(Row, A)
+        same(out.to_numpy(), row - a, ("row first", what))
+        out.mul_array(A, Col)
+        same(out.to_numpy(), a * col, ("column", what))
+        out.add_array(A, B.transpose())
+        same(out.to_numpy(), a + b.T, ("transposed", what))
+        out.copy_from(B.transpose())
+        same(out.to_numpy(), b.T, ("transposed copy", what))
+        out.mul_scalar(A, 0.5)
+        same(out.to_numpy(), a * dtype(0.5), ("scalar", what))
+        A.add_assign(B.transpose())                        # in place: every element is added to once
+        same(A.to_numpy(), a + b.T, ("transposed, in place", what))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 15, 16, 17, 255, 1027])
+def test_rows_of_a_wider_matrix(hip, dtype, cols):
+    """row slices: neither the row starts nor the row length are multiples of a vector, and nothing outside is written"""
+    r = np.random.default_rng(cols)
+    wide = r.standard_normal((37, cols + 6)).astype(dtype)
+    row = r.standard_normal(cols).astype(dtype)
+    W, D, Row = hip.Matrix.from_numpy(wide), hip.Matrix.from_numpy(wide), hip.Matrix.from_numpy(row)
+    at = (slice(None), slice(3, 3 + cols))
+    D.slice(*at).add_array(W.slice(*at), Row)
+    exp = wide.copy()
+    exp[at] = wide[at] + row
+    same(D.to_numpy(), exp, "slice + row")
+    D.slice(*at).copy_from(W.slice(slice(None), slice(1, 1 + cols)))
+    exp[at] = wide[:, 1:1 + cols]
+    same(D.to_numpy(), exp, "slice copy")
+
+
+def test_streaming_sizes(hip):
+    """beyond the caches (streaming accesses), every operand starting in the middle of a vector"""
+    r = np.random.default_rng(3)
+    rows, cols = 2051, 2047
+    a, b = r.standard_normal((rows, cols), dtype=np.float32), r.standard_normal((cols, rows), dtype=np.float32)
+    row = r.standard_normal(cols, dtype=np.float32)
+    A, B, Row = offset_matrix(hip, a, 1), offset_matrix(hip, b, 2), offset_matrix(hip, row, 3)
+    out = offset_matrix(hip, np.zeros((rows, cols), np.float32), 1)
+    out.add_array(A, Row)
+    same(out.to_numpy(), a + row, "row")
+    out.add_array(A, B.transpose())
+    same(out.to_numpy(), a + b.T, "transposed")
+    out.copy_from(B.transpose())
+    same(out.to_numpy(), b.T, "transposed copy")
+    out.relu(A, 0.0)
+    same(out.to_numpy(), np.maximum(a, 0), "relu")

@@ -318,16 +318,22 @@ __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *ou
             if constexpr (NT && ContigShape<F>::kSmall && VEC > 1) store_pack_wt<T, VEC>(out + i, r);
             else store_pack<T, VEC, NT>(out + i, r);
         }
-    } else {
+    } else {   // the last tile: whole vectors while they last, then the remaining elements one by one
         f.init();
+#pragma unroll
         for (int u = 0; u < kUnroll; u++) {
             int64_t i = base + ((int64_t)u * kBlock + tid) * VEC;
-#pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                if (i + j < n) {
-                    T x = a[i + j];
-                    T y = (F::NIN == 2) ? b[i + j] : x;
-                    out[i + j] = f(x, y);
+            if (i + VEC <= n) {
+                const Pack<T, VEC> x = load_pack<T, VEC, false>(a + i);
+                const Pack<T, VEC> y = (F::NIN == 2) ? load_pack<T, VEC, false>(b + i) : x;
+                store_pack<T, VEC, false>(out + i, apply_pack<T, VEC, F>(f, x, y));
+            } else {
+                for (int j = 0; j < VEC; j++) {
+                    if (i + j < n) {
+                        T x = a[i + j];
+                        T y = (F::NIN == 2) ? b[i + j] : x;
+                        out[i + j] = f(x, y);
+                    }
                 }
             }
         }
@@ -340,7 +346,10 @@ __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *ou
 // [m,n], a column [m,1] on [m,n].  Flat index i reads y[(i / inner) % mid].  Indices are 32-bit
 // (checked at launch).  With a one-input functor there is no x: the output is f(y) spread over the
 // other dims (broadcast of a row, a column, a bias).  MODE 0: inner == 1 and mid % VEC == 0, y is read as vectors; MODE 1:
-// inner % VEC == 0, one y per vector; MODE 2: inner >= VEC, a vector spans at most two y.
+// inner % VEC == 0, one y per vector; MODE 2: inner >= VEC, a vector spans at most two y; MODE 3: inner == 1 and
+// any mid, y is read as vectors except where one runs past the end of the period.  (MODE 3 keeps x and the output
+// flat and aligned however long the row is: [3001,2047] + [2047] f32 takes 9.9 us (5.0 TB/s), 24.4 us when rows of
+// odd length were walked one by one with scalar accesses.)
 
 template <typename T, int VEC, bool NT, typename F, bool Y_FIRST, int MODE, int kBlock, int kUnroll>
 __global__ __launch_bounds__(kBlock) void ew_periodic_kernel(T *out, const T *x, const T *y, uint32_t n,
@@ -354,6 +363,18 @@ __global__ __launch_bounds__(kBlock) void ew_periodic_kernel(T *out, const T *x,
             yv = load_pack<T, VEC, false>(y + i0 % mid);
         } else if constexpr (MODE == 1) {
             yv = splat<T, VEC>(y[(i0 / inner) % mid]);
+        } else if constexpr (MODE == 3) {
+            const uint32_t c = i0 % mid;
+            if (c + VEC <= mid) {
+                yv = load_pack<T, VEC, false>(y + c);
+            } else {
+                uint32_t cj = c;
+#pragma unroll
+                for (int j = 0; j < VEC; j++) {
+                    yv.v[j] = y[cj];
+                    cj = cj + 1 == mid ? 0 : cj + 1;
+                }
+            }
         } else {
             const uint32_t q0 = i0 / inner, rem = i0 - q0 * inner, c0 = q0 % mid;
             const uint32_t c1 = c0 + 1 == mid ? 0 : c0 + 1;
@@ -558,6 +579,7 @@ __global__ __launch_bounds__(kBlock) void ew_rows_kernel(T *out, const T *a, con
 // SMALL halves the edge (32 / 16): few tiles of a small matrix leave most CUs idle and make each workgroup a
 // long chain; with a quarter of the tile per workgroup a transposed copy of [256,512] f32 takes 2.8 us
 // against 3.3 us, of [784,512] 3.4 against 3.6 (the MLP step of a 512-wide layer issues eleven of them).
+// Operands that stay in the caches take them at every size, see launch_ew.
 template <typename T, bool SMALL = false> struct TileOf { static constexpr int N = (sizeof(T) == 4 ? 64 : 32) / (SMALL ? 2 : 1); };
 // With two inputs (three streams, a + b^T) two vectors per thread and operand at 512 threads are the
 // fastest (stand-alone probe: 36.2 us with four at 256 threads, 35.5 us with two at 512, 35.7 us with
@@ -567,7 +589,7 @@ template <typename T, typename F, bool SMALL = false> struct TileThreads {
     static constexpr int value = (F::NIN == 1 || kVecs < 512) ? kVecs : 512;
 };
 
-enum { kWalkRows = 0, kWalkCols = 1, kWalkDiagonal = 2 };
+enum { kWalkRows = 0, kWalkCols = 1, kWalkDiagonal = 2, kWalkBands = 3 };
 
 struct TileParams {
     OuterDesc outer;      // batch dims (everything except the two tile dims)
@@ -576,9 +598,9 @@ struct TileParams {
     int64_t ldr[kMaxOperands];  // stride along R per operand
     int64_t ldc[kMaxOperands];  // stride along C per operand (1 for out; 0/1 direct; ld for transposed)
     int trans_a, trans_b;       // input goes through LDS
-    int vec_ok;                 // alignment allows 128-bit accesses on full tiles
+    int vec_ok;                 // every operand can be read as vectors
     int grid3d;                 // the grid is (tiles_c, tiles_r, nbatch); else linear, tiles_c fastest
-    int walk;                   // order of the tiles: kWalkRows, kWalkCols (3-d grids only) or kWalkDiagonal
+    int walk;                   // order of the tiles: kWalkRows, kWalkDiagonal, or (3-d grids only) kWalkCols, kWalkBands
     int64_t tiles_r, tiles_c;
     uint32_t tiles_r_magic;     // min(floor(2^32 / tiles_r), 2^32 - 1): x mod tiles_r from one high multiply and a fix-up
 };
@@ -652,23 +674,43 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         const uint32_t r = x - q * ntr;
         tr32 = r >= ntr ? r - ntr : r;
     }
+    if (walk == kWalkBands) {
+        // Workgroup i runs on XCD i mod 8; each XCD gets one run of consecutive tiles, row by row.  Where the
+        // output's rows do not start at cache lines, neighbouring tiles share the lines at their border, and
+        // with the neighbours on one XCD its L2 puts the two halves together.
+        const uint32_t gx = gridDim.x, gxy = gx * gridDim.y, total = gxy * gridDim.z;
+        const uint32_t wg = batch32 * gxy + tr32 * gx + tc32;
+        const uint32_t share = total >> 3, rest = total & 7, xcd = wg & 7;
+        uint32_t t = xcd * share + (xcd < rest ? xcd : rest) + (wg >> 3);
+        batch32 = t / gxy;
+        t -= batch32 * gxy;
+        tr32 = t / gx;
+        tc32 = t - tr32 * gx;
+    }
     const int64_t tc = tc32, tr = tr32;
     int64_t oo = 0, oa = 0, ob = 0;
     if (nouter > 0) decompose32(p.outer, batch32, oo, oa, ob);
     const int64_t r0 = tr * kTile, c0 = tc * kTile;
     const int64_t nr = (R - r0 < kTile) ? R - r0 : kTile;
     const int64_t nc = (C - c0 < kTile) ? C - c0 : kTile;
-    const bool full = (nr == kTile) & (nc == kTile) & (vec_ok != 0);
+    const bool full = (nr == kTile) & (nc == kTile);
     const int tid = threadIdx.x;
 
     T *obase = out + oo + r0 * ldr0 + c0;
     const T *abase = a + oa + r0 * ldr1 + c0 * ldc1;
     const T *bbase = (F::NIN == 2) ? b + ob + r0 * ldr2 + c0 * ldc2 : abase;
 
-    if (full) {
-        // All global loads of the tile are issued first -- the transposed inputs along R (their
-        // contiguous dim), the others along C -- so both streams are in flight together; then the
-        // transposed ones are turned through LDS.
+    // All global loads of the tile are issued first -- the transposed inputs along R (their
+    // contiguous dim), the others along C -- so both streams are in flight together; then the
+    // transposed ones are turned through LDS.
+    // EDGE: a tile that the matrix ends in.  The vectors that would run past the end are moved back to end with
+    // it (two lanes then load, and scatter to LDS, the same elements) and positions past the end of the other
+    // dim repeat its last one, so the loads stay vectors without a branch between them; every element is stored
+    // by one thread only, the moved-back vectors element by element.  a + b^T of [3001,2047] f32 15.6 us,
+    // 19.2 us when operands of odd pitch were accessed element by element; the transposed copies of a [1000,999]
+    // head and of [1500,1433] weights 4.6 - 4.9 / 6.6 us, 5.2 - 5.8 / 8.4 us before.
+    auto tile_by_vectors = [&](auto edge_c) {
+        constexpr bool EDGE = decltype(edge_c)::value;
         // vector e = k * kBlock + tid of the tile: eight consecutive ones form a segment, the segments
         // of one segment column follow each other along the other dim
         constexpr int K = kTile * SEG * VPS / kBlock;   // vectors per thread and operand (1 or 4)
@@ -677,6 +719,9 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         auto vec_of = [&](int k) { return seg_v + (((k * kBlock + tid) / VPS) / kTile) * VPS * VEC; };  // element position along the vector dim
         const bool ta = trans_a != 0;
         const bool tb = (F::NIN == 2) && trans_b != 0;
+        // where the vectors of an input, or of the output, start and lie in an edge tile
+        auto clip_vec = [&](int v, bool t) { return EDGE ? min(v, (int)(t ? nr : nc) - VEC) : v; };
+        auto clip_other = [&](int o, bool t) { return EDGE ? min(o, (int)(t ? nc : nr) - 1) : o; };
         // A transposed input is read along R with its pitch ldc between the vectors, any other along C
         // with its pitch ldr: the same expression with the pitch selected, so the loads of one thread
         // follow each other without a branch between them.  (With a branch per load the compiler put a
@@ -688,14 +733,14 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         for (int k = 0; k < K; k++) {
             const int o = other_of(k);
             const int lane_v = vec_of(k);
-            xa[k] = load_pack<T, VEC, NT>(abase + lane_v + (int64_t)o * pitch_a);
-            if constexpr (F::NIN == 2) xb[k] = load_pack<T, VEC, NT>(bbase + lane_v + (int64_t)o * pitch_b);
+            xa[k] = load_pack<T, VEC, NT>(abase + clip_vec(lane_v, ta) + (int64_t)clip_other(o, ta) * pitch_a);
+            if constexpr (F::NIN == 2) xb[k] = load_pack<T, VEC, NT>(bbase + clip_vec(lane_v, tb) + (int64_t)clip_other(o, tb) * pitch_b);
         }
         if (ta) {
 #pragma unroll
             for (int k = 0; k < K; k++) {
-                const int c = other_of(k);               // the loaded vector holds rows lane_v.. of column c
-                const int lane_v = vec_of(k);
+                const int c = clip_other(other_of(k), true);        // the loaded vector holds rows lane_v.. of column c
+                const int lane_v = clip_vec(vec_of(k), true);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) lds_a[(lane_v + j) * kPitch + c] = xa[k].v[j];
             }
@@ -704,8 +749,8 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
             if (tb) {
 #pragma unroll
                 for (int k = 0; k < K; k++) {
-                    const int c = other_of(k);
-                    const int lane_v = vec_of(k);
+                    const int c = clip_other(other_of(k), true);
+                    const int lane_v = clip_vec(vec_of(k), true);
 #pragma unroll
                     for (int j = 0; j < VEC; j++) lds_b[(lane_v + j) * kPitch + c] = xb[k].v[j];
                 }
@@ -715,8 +760,8 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         if (ta) {
 #pragma unroll
             for (int k = 0; k < K; k++) {
-                const int r = other_of(k);
-                const int lane_v = vec_of(k);
+                const int r = clip_other(other_of(k), false);
+                const int lane_v = clip_vec(vec_of(k), false);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) xa[k].v[j] = lds_a[r * kPitch + lane_v + j];
             }
@@ -725,8 +770,8 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
             if (tb) {
 #pragma unroll
                 for (int k = 0; k < K; k++) {
-                    const int r = other_of(k);
-                    const int lane_v = vec_of(k);
+                    const int r = clip_other(other_of(k), false);
+                    const int lane_v = clip_vec(vec_of(k), false);
 #pragma unroll
                     for (int j = 0; j < VEC; j++) xb[k].v[j] = lds_b[r * kPitch + lane_v + j];
                 }
@@ -738,10 +783,31 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
             const int lane_v = vec_of(k);
             Pack<T, VEC> y = xa[k];
             if constexpr (F::NIN == 2) y = xb[k];
-            store_pack<T, VEC, NT>(obase + (int64_t)r * ldr0 + lane_v, apply_pack<T, VEC, F>(f, xa[k], y));
+            const Pack<T, VEC> z = apply_pack<T, VEC, F>(f, xa[k], y);
+            if constexpr (EDGE) {
+                if ((r < nr) & (lane_v < nc)) {
+                    T *const orow = obase + (int64_t)r * ldr0;
+                    if (lane_v + VEC <= nc) {
+                        store_pack<T, VEC, NT>(orow + lane_v, z);
+                    } else {
+                        const int c = clip_vec(lane_v, false);
+#pragma unroll
+                        for (int j = 0; j < VEC; j++)
+                            if (c + j >= lane_v) orow[c + j] = z.v[j];
+                    }
+                }
+            } else {
+                store_pack<T, VEC, NT>(obase + (int64_t)r * ldr0 + lane_v, z);
+            }
         }
+    };
+
+    if (vec_ok && full) {
+        tile_by_vectors(std::false_type());
+    } else if (vec_ok && nr >= VEC && nc >= VEC) {
+        tile_by_vectors(std::true_type());
     } else {
-        // Edge tiles and unaligned operands: element by element with bounds checks.  All loads of a
+        // Tiles narrower than a vector, and inputs broadcast along the row: element by element with bounds checks.  All loads of a
         // phase are issued before the first use (an element outside the tile reads the tile's first
         // one again and is dropped): with the loads inside the bounds check the compiler waits for each
         // before it issues the next, and a small matrix made of edge tiles only (the [512,10] weights of a
@@ -908,28 +974,19 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
         if (p.stride[o][0] != 1) all_unit = false;
     if (all_unit) {
         const int64_t n = p.numel;
-        bool vec = aligned16(out) && aligned16(a) && aligned16(b);
-        if (vec) {
-            constexpr int cb = ContigShape<F>::kBlock, cu = ContigShape<F>::kUnroll;
-            int64_t tile = (int64_t)cb * VEC * cu;
-            int64_t grid = (n + tile - 1) / tile;
-            if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
-            if (nt) ew_contig_kernel<T, VEC, true, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
-            else    ew_contig_kernel<T, VEC, false, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
-        } else {
-            constexpr int cb = ContigShape<F>::kBlock, cu = ContigShape<F>::kUnroll;
-            int64_t tile = (int64_t)cb * cu;
-            int64_t grid = (n + tile - 1) / tile;
-            if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
-            ew_contig_kernel<T, 1, false, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
-        }
+        constexpr int cb = ContigShape<F>::kBlock, cu = ContigShape<F>::kUnroll;
+        int64_t tile = (int64_t)cb * VEC * cu;
+        int64_t grid = (n + tile - 1) / tile;
+        if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
+        if (nt) ew_contig_kernel<T, VEC, true, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
+        else    ew_contig_kernel<T, VEC, false, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
         ZENU_LAUNCH_CHECK();
         return ZENU_OK;
     }
 
     // flat with one periodic operand (bias over channels, a row or a column over a matrix)
     {
-        if (p.numel < ((int64_t)1 << 32) - 65536 && aligned16(out)) {
+        if (p.numel < ((int64_t)1 << 32) - 65536) {
             auto flat = [&](int o) {
                 int64_t want = 1;
                 for (int d = p.ndim - 1; d >= 0; d--) {
@@ -957,10 +1014,8 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                 int64_t inner = 1;
                 for (int d = m + 1; d < p.ndim; d++) inner *= p.shape[d];
                 const int64_t mid = p.shape[m];
-                const int mode = (inner == 1 && mid % VEC == 0 && aligned16(y)) ? 0
-                                 : (inner % VEC == 0)                           ? 1
-                                 : (inner >= VEC)                               ? 2 : -1;
-                if (mode >= 0 && aligned16(x)) {
+                const int mode = inner == 1 ? (mid % VEC == 0 ? 0 : 3) : inner % VEC == 0 ? 1 : inner >= VEC ? 2 : -1;
+                if (mode >= 0) {
                     // one load and one store stream: the small workgroup shape of the unary ops when y comes as
                     // vectors (22.4 against 23.5 us on [4096,4096] + [1,4096]); with the index divisions of
                     // the other modes the larger shape is the better one (16.4 against 17.0 us on a
@@ -970,7 +1025,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                         constexpr bool YF = decltype(yfirst_c)::value;
                         constexpr int MODE = decltype(mode_c)::value;
                         // a lone store stream (one-input functor) keeps the larger shape, like the fill kernel
-                        constexpr bool small = MODE == 0 && !IsValuBound<F>::value && F::NIN == 2;
+                        constexpr bool small = (MODE == 0 || MODE == 3) && !IsValuBound<F>::value && F::NIN == 2;
                         constexpr int B = small ? ZENU_EW1_BLOCK : 256, U = small ? ZENU_EW1_UNROLL : 2;
                         const int64_t tile = (int64_t)B * VEC * U;
                         const unsigned grid = (unsigned)((p.numel + tile - 1) / tile);
@@ -980,7 +1035,8 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                     auto by_mode = [&](auto yfirst_c) {
                         if (mode == 0) go(yfirst_c, std::integral_constant<int, 0>());
                         else if (mode == 1) go(yfirst_c, std::integral_constant<int, 1>());
-                        else go(yfirst_c, std::integral_constant<int, 2>());
+                        else if (mode == 2) go(yfirst_c, std::integral_constant<int, 2>());
+                        else go(yfirst_c, std::integral_constant<int, 3>());
                     };
                     if (yo == 1) by_mode(std::true_type());
                     else by_mode(std::false_type());
@@ -1013,16 +1069,11 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
             if (p.stride[1][d] == 0) nta = false;   // re-read for every outer index: keep it cached
             if (nin == 2 && p.stride[2][d] == 0) ntb = false;
         }
-        bool vec = aligned16(out) && (rp.ncols % VEC == 0);
-        for (int o = 1; o <= nin && vec; o++)
-            if (p.stride[o][last] == 1 && !aligned16(p.ptr[o])) vec = false;
-        for (int d = 0; d < p.ndim - 1 && vec; d++) {
-            if (p.stride[0][d] % VEC) vec = false;
-            for (int o = 1; o <= nin; o++)
-                if (p.stride[o][last] == 1 && p.stride[o][d] % VEC) vec = false;
-        }
+        // Vectors whatever the alignment; a short row that is no whole number of vectors leaves a lane with up to
+        // VEC - 1 single elements one after the other, so it takes one element per lane.
+        const bool vec = rp.ncols % VEC == 0 || rp.ncols >= 4 * VEC;
         const int v = vec ? VEC : 1;
-        int64_t vcols = (rp.ncols + v - 1) / v;
+        const int64_t vcols = (rp.ncols + v - 1) / v;
         // full-size streams of this launch: the output plus every input that is neither a scalar
         // per row nor re-read for every outer index; exactly two of them (one load, one store per
         // element) take the small workgroup shape.  A lone store stream (broadcast of a row) does
@@ -1099,23 +1150,34 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
             tp.trans_a = trans[1];
             tp.trans_b = nin == 2 ? trans[2] : 0;
             bool vec = true;
-            for (int o = 0; o <= nin && vec; o++) {
-                if (!aligned16(p.ptr[o])) vec = false;
-                // every stride that moves a vector's base address must keep 16 B alignment
-                for (int d = 0; d < p.ndim && vec; d++) {
-                    int64_t s = p.stride[o][d];
-                    if (s == 1 || s == 0) continue;
-                    if (s % VEC) vec = false;
-                }
-            }
             // the vector path reads whole vectors along C from the inputs that are not transposed: one
             // that is broadcast along C (a column beside a transposed operand) takes the element path
             for (int o = 1; o <= nin; o++)
                 if (!trans[o] && tp.ldc[o] == 0) vec = false;
             tp.vec_ok = vec ? 1 : 0;
-            // tile edge: halved when the full-size tiles would not give every CU two workgroups
-            auto launch_tiles = [&](auto small_c) -> int {
+            // Rows of the output that do not start at 128-byte lines: every border between two column tiles
+            // is a line that both write in part.  Streaming accesses then cost a second transfer of that line
+            // and are not used; small tiles in one band per XCD are the fastest (us of the four combinations
+            // of tile edge 64 / 32 and walk rows / bands, without the hint, and of 64 / rows with it): a + b^T
+            // [3001,2047] f32 20.9 / 17.7 / 21.7 / 16.8, 21.7; [4099,4097] 53.8 / 47.4 / 60.2 / 46.3, 64.0;
+            // transposed copy [1500,1433] 6.2 / 5.9 / 6.1 / 4.8, 7.6.
+            bool rows_split_lines = reinterpret_cast<uintptr_t>(out) % 128 != 0;
+            for (int d = 0; d < last; d++)
+                if (p.stride[0][d] * (int64_t)sizeof(T) % 128) rows_split_lines = true;
+            // Otherwise: two inputs stream from kStreamBytes on, as the other kernels do; one input (us with the
+            // small tiles and no hint / large tiles and hint: NCHW -> NHWC of [64,512,14,14] f32, 51 MB,
+            // 10.5 / 13.7; transposed [2048,2048], 34 MB, 6.0 / 8.2; [4096,4096], 134 MB, 27.4 / 23.9) from three
+            // times that.  The large tiles' longer row pieces pay only when streaming, with enough tiles and
+            // little padding ([64,256,28,28] NCHW -> NHWC, 784 = 12.25 tiles: 19.2 small, 21.4 large).
+            const int64_t bytes = p.numel * (int64_t)sizeof(T) * (nin + 1);
+            const bool stream_tiles = nt && !rows_split_lines && (nin == 2 || bytes >= 3 * kStreamBytes);
+            constexpr int kFullTile = TileOf<T>::N;
+            const int64_t full_tiles = tp.nbatch * ((tp.R + kFullTile - 1) / kFullTile) * ((tp.C + kFullTile - 1) / kFullTile);
+            const bool large = stream_tiles && full_tiles >= 2 * (int64_t)device_info().num_cus &&
+                               full_tiles * (kFullTile * kFullTile) <= p.numel + p.numel / 25;
+            auto launch_tiles = [&](auto small_c, auto nt_c) -> int {
                 constexpr bool SMALL = decltype(small_c)::value;
+                constexpr bool NT = decltype(nt_c)::value;
                 constexpr int kTile = TileOf<T, SMALL>::N;
                 tp.tiles_r = (tp.R + kTile - 1) / kTile;
                 tp.tiles_c = (tp.C + kTile - 1) / kTile;
@@ -1137,7 +1199,8 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                     if (trans[o]) trans_near = trans_near || near_4k(tp.ldc[o]);
                     else if (tp.ldc[o] == 1) direct_near = direct_near || near_4k(tp.ldr[o]);
                 }
-                tp.walk = !trans_near ? kWalkRows
+                tp.walk = (rows_split_lines && tp.grid3d && tp.tiles_c > 1) ? kWalkBands
+                          : !trans_near                                     ? kWalkRows
                           : (!direct_near && tp.grid3d && tp.tiles_c <= 65535) ? kWalkCols : kWalkDiagonal;
                 const bool by_cols = tp.walk == kWalkCols;
                 const dim3 g = !tp.grid3d ? dim3((unsigned)grid)
@@ -1145,14 +1208,12 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                                          : dim3((unsigned)tp.tiles_c, (unsigned)tp.tiles_r, (unsigned)tp.nbatch);
                 const size_t lds = (size_t)(tp.trans_a + tp.trans_b) * kTile * (kTile + 1) * sizeof(T);
                 constexpr int kThreads = TileThreads<T, F, SMALL>::value;
-                if (nt) ew_tile_kernel<T, true, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
-                else    ew_tile_kernel<T, false, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
+                ew_tile_kernel<T, NT, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
                 return ZENU_OK;
             };
-            constexpr int kFullTile = TileOf<T>::N;
-            const int64_t full_tiles = tp.nbatch * ((tp.R + kFullTile - 1) / kFullTile) * ((tp.C + kFullTile - 1) / kFullTile);
-            const int rc_tiles = full_tiles < 2 * (int64_t)device_info().num_cus ? launch_tiles(std::true_type())
-                                                                                  : launch_tiles(std::false_type());
+            const int rc_tiles = large          ? launch_tiles(std::false_type(), std::true_type())
+                                 : stream_tiles ? launch_tiles(std::true_type(), std::true_type())
+                                                : launch_tiles(std::true_type(), std::false_type());
             if (rc_tiles) return rc_tiles;
             ZENU_LAUNCH_CHECK();
             return ZENU_OK;
