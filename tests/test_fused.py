@@ -179,6 +179,73 @@ def test_softmax_rows_divide_like_the_chain(hip):
             assert matched, f"R={R} row {i}: no single divisor near {s0!r} reproduces the row"
 
 
+# Rows of a wavefront, of 256, 512 and 1024 threads and beyond their registers (f32 32768 elements, f64
+# 16384), one element around each limit; lines of 8, 16 and 32 elements per thread on one and several wavefronts;
+# totals below and above the 32 MiB from which rows are cut at cache lines
+ROW_SHAPES = [(5, 65), (3, 511), (9, 513), (3, 1023), (2, 1025), (2, 4095), (2, 4097), (3, 8193), (2, 16383), (3, 16385),
+              (2, 32767), (3, 32769), (2, 40003), (9001, 481), (4400, 993), (1100, 4065), (150, 32735), (131, 32737), (110, 40001)]
+LINE_SHAPES = [(3, 1, 5), (2, 8, 65), (2, 9, 63), (1, 17, 129), (5, 33, 7), (1, 128, 3), (1, 129, 70), (2, 257, 2), (1, 513, 9),
+               (16, 21, 16384), (40, 16, 4099), (70, 33, 2048), (300, 17, 1), (70, 64, 1), (140000, 23, 1)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", ROW_SHAPES + LINE_SHAPES, ids=str)
+def test_softmax_kernel_edges(hip, dtype, shape):
+    """Every kernel of the dispatch at its edges, the operands at odd offsets, against 80-bit sums.  n terms added in
+    any order are off by less than (n - 1) eps of the sum of their magnitudes; a term and the quotient by an eps each."""
+    print(f"[case] softmax {shape} {np.dtype(dtype).name}", flush=True)
+    n = shape[1]
+    r = np.random.default_rng(n)
+    x = (r.standard_normal(shape, dtype=np.float32) * 3).astype(dtype)
+    gy = r.standard_normal(shape, dtype=np.float32).astype(dtype)
+
+    def at_offset(a, off):
+        m = hip.Matrix.from_numpy(np.concatenate([np.zeros(off, dtype), a.reshape(-1), np.full(5, 7, dtype)]))
+        return hip.Matrix(m.buf, off, shape, hip.default_stride(shape), dtype), m
+
+    out, whole = at_offset(np.zeros_like(x), 3)
+    out.softmax_assign(at_offset(x, 1)[0], 1)
+    y = out.to_numpy()
+    e = np.exp(x.astype(np.longdouble) - x.max(axis=1, keepdims=True))
+    exact = e / e.sum(axis=1, keepdims=True)
+    eps = np.finfo(dtype).eps
+    assert np.all(np.abs(y - exact) <= (n + 3 + 2 * np.abs(x - x.max(axis=1, keepdims=True))) * eps * exact + np.finfo(dtype).tiny)
+    ends = hip.Matrix(whole.buf, 0, (x.size + 8,), (1,), dtype).to_numpy()
+    assert np.all(ends[:3] == 0) and np.all(ends[-5:] == 7)
+
+    gx, whole = at_offset(np.zeros_like(x), 2)
+    hip._lib.check(hip.lib().zenu_hip_softmax_backward(hip._lib.F32 if dtype == np.float32 else hip._lib.F64, C.byref(gx.desc()),
+                   C.byref(out.desc()), C.byref(at_offset(gy, 1)[0].desc()), 1, None), "softmax_backward")
+    got = gx.to_numpy()
+    t = y.astype(np.longdouble) * gy
+    exact = t - y * t.sum(axis=1, keepdims=True)
+    bound = (n + 2) * eps * np.abs(t).sum(axis=1, keepdims=True) * y + 3 * eps * np.abs(t)
+    assert np.all(np.abs(got - exact) <= bound + np.finfo(dtype).tiny)
+    ends = hip.Matrix(whole.buf, 0, (x.size + 7,), (1,), dtype).to_numpy()
+    assert np.all(ends[:2] == 0) and np.all(ends[-5:] == 7)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("n,c", [(193, 40), (130, 64), (257, 63), (31, 513), (1000, 999), (700, 4099), (2, 32769)])
+def test_cross_entropy_kernel_edges(hip, dtype, n, c):
+    """loss and gradient where the workgroup's shape changes; bounds as above, the loss a sum of n logarithms"""
+    print(f"[case] cross_entropy {n}x{c} {np.dtype(dtype).name}", flush=True)
+    r = np.random.default_rng(n + c)
+    pred = r.standard_normal((n, c)).astype(dtype)
+    ans = np.zeros((n, c), dtype=dtype)
+    ans[np.arange(n), r.integers(0, c, n)] = 1
+    loss, prob = hip.cross_entropy(hip.Matrix.from_numpy(pred), hip.Matrix.from_numpy(ans))
+    p = prob.to_numpy()
+    e = np.exp(pred.astype(np.longdouble))
+    exact = e / e.sum(axis=1, keepdims=True)
+    eps = np.finfo(dtype).eps
+    assert np.all(np.abs(p - exact) <= (c + 20) * eps * exact)
+    want = -np.sum(np.log(p[ans == 1].astype(np.longdouble))) / n
+    assert abs(float(loss.to_numpy()) - want) <= (n + 4) * eps * want
+    g = hip.cross_entropy_backward(prob, hip.Matrix.from_numpy(ans)).to_numpy()
+    assert np.all(np.abs(g - (p - ans) / n) <= (c + 6) * eps * (p + ans) / n)
+
+
 def test_softmax_special_rows(hip):
     """NaN in position 0 / elsewhere and an all -inf row poison the row exactly as in the chain; a row
     with +inf gives NaN at the inf (inf - inf) and 0 elsewhere... all NaN after the division"""

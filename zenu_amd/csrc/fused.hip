@@ -28,7 +28,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kLineMaxR = 64;   // rows up to this length: one thread per row
-constexpr int kRegPacks = 4;    // workgroup-per-row: vectors a thread keeps in registers
 
 // ---- workgroup reductions in a fixed order ------------------------------------------------------------
 
@@ -55,83 +54,138 @@ template <typename T, bool MAX, int BLOCK = kBlock> __device__ __forceinline__ T
 // ---- forward ---------------------------------------------------------------------------------------------
 // CE: additionally rowloss[line] = sum_r target * log(softmax)   (inner == 1 only)
 
-constexpr int kLineRegs = 16;   // lines up to this length are kept in registers by the lines kernel
+constexpr int kLineRegs = 16;   // classes of the one-workgroup classifier head kernels below
+constexpr int kLineWaves = 16;  // wavefronts that can share the lines of a workgroup
 
-template <typename T, bool CE>
-__device__ __forceinline__ T softmax_line(const zmath::ExpLog<T> &ml, const T *x, T *y, int64_t line, int64_t R,
-                                          int64_t inner, const T *target, T *rowloss);
+// Where a wavefront of the two lines kernels stands: a workgroup has `waves` wavefronts along R for every 64
+// lines, wavefront w of them holds elements [w OWN, (w + 1) OWN) of each of its lines in registers.
+struct LineSpot {
+    int64_t line, base;   // base: offset of the line's element 0 (of line 0 past the end)
+    int w, group;
+    bool active;
+    __device__ __forceinline__ LineSpot(int64_t lines, int64_t R, int64_t inner, int waves)
+    {
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        group = wave / waves;
+        w = wave - group * waves;
+        const int groups = (int)(blockDim.x >> 6) / waves;
+        line = ((int64_t)blockIdx.x * groups + group) * 64 + (threadIdx.x & 63);
+        active = line < lines;
+        const int64_t l = active ? line : 0;
+        if (inner == 1) {
+            base = l * R;
+        } else {
+            const int64_t q = l / inner;
+            base = q * R * inner + (l - q * inner);
+        }
+    }
+};
 
+// `x[i]`, i = 0 .. valid - 1, added to a running sum in index order over the wavefronts of a line: each takes the
+// sum over from the one before it.  carry: one value per line of the workgroup.  Every thread calls it.
+template <typename T, int OWN>
+__device__ __forceinline__ T sum_in_order(const T (&x)[OWN], int valid, const LineSpot &at, int waves, T *carry)
+{
+    T *const mine = carry + at.group * 64 + (threadIdx.x & 63);
+    T sum = (T)0;
+    for (int turn = 0; turn < waves; turn++) {
+        if (at.w == turn) {
+            if (turn) sum = *mine;
+#pragma unroll
+            for (int i = 0; i < OWN; i++)
+                if (i < valid) sum = sum + x[i];
+            if (waves > 1) *mine = sum;
+        }
+        if (waves > 1) __syncthreads();
+    }
+    return waves > 1 ? *mine : sum;
+}
+
+// The softmax axis is not the last one, or is short: a lane per line, and as many wavefronts along the line as it
+// takes to hold it in registers, so that it is read and written once with all its loads in flight together.  The
+// sums run over the line in index order exactly as sum.rs:20-25 adds (they are handed from wavefront to wavefront).
+// Bound by the passes over memory: [16,21,16384] f32 (22 MB each way, cached) 17.0 us, 26.1 when one thread
+// walked a line three times, one load in flight; its backward pass 11.9 us, 20.5.
 // With `loss` set (cross-entropy, every line in this one workgroup) the kernel also folds the row
 // terms and divides by -N, in the order of ce_finalize_kernel: the whole loss in one launch.
-template <typename T, bool CE>
-__global__ __launch_bounds__(kBlock) void softmax_lines_kernel(const T *x, T *y, int64_t lines, int64_t R,
-                                                                int64_t inner, const T *target, T *rowloss,
-                                                                T *loss, T neg_n)
+template <typename T, bool CE, int OWN>
+__global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T *x, T *y, int64_t lines, int R,
+                                                                         int64_t inner, int waves, const T *target,
+                                                                         T *rowloss, T *loss, T neg_n)
 {
+    __shared__ T shared[kLineWaves * 64];
+    const LineSpot at(lines, R, inner, waves);
+    const int lane = threadIdx.x & 63;
+    const int r0 = at.w * OWN;
+    const int valid = R - r0;              // uniform; at least 1
+    const T *const xl = x + at.base + r0 * inner;
+    T *const yl = y + at.base + r0 * inner;
+    T v[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; i += 4) {
+        if (i < valid) {
+#pragma unroll
+            for (int j = i; j < i + 4; j++) v[j] = xl[(j < valid ? j : 0) * inner];
+        }
+    }
+    const T x0 = waves > 1 ? x[at.base] : v[0];
     zmath::ExpLog<T> ml;
     ml.init(true, CE);
-    const int64_t line = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    T row_term = (T)0;
-    if (line < lines) row_term = softmax_line<T, CE>(ml, x, y, line, R, inner, target, rowloss);
+    // max_axis: strict '>' from element 0 (max.rs:19-34): a NaN there stays, a NaN elsewhere never replaces
+    T m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < OWN; i++)
+        if (i < valid) m = combine<T, true>(m, v[i]);
+    if (waves > 1) {
+        shared[threadIdx.x] = m;
+        __syncthreads();
+        for (int w = 0; w < waves; w++) m = combine<T, true>(m, shared[(at.group * waves + w) * 64 + lane]);
+        __syncthreads();
+    }
+    m = combine<T, true>(x0, m);
+#pragma unroll
+    for (int i = 0; i < OWN; i++)
+        if (i < valid) v[i] = ml.exp(v[i] - m);
+    const T sum = sum_in_order<T, OWN>(v, valid, at, waves, shared);
+#pragma unroll
+    for (int i = 0; i < OWN; i++) {
+        if (i < valid) {
+            const T s = v[i] / sum;
+            if (at.active) yl[i * inner] = s;
+            if constexpr (CE) v[i] = target[at.base + r0 + i] * ml.log(s);
+        }
+    }
     if constexpr (CE) {
-        if (loss) {     // uniform: every thread of the workgroup gets here
-            __shared__ T lds[kWaves];
-            T acc = (T)0;
-            if (line < lines) acc = acc + row_term;
-            acc = block_red<T, false>(acc, lds);
-            if (threadIdx.x == 0) *loss = acc / neg_n;
+        if (waves > 1) __syncthreads();        // the sum of the exponentials has been read
+        const T term = sum_in_order<T, OWN>(v, valid, at, waves, shared);
+        if (loss) {     // uniform; one workgroup of at most four groups of 64 lines
+            __shared__ T lds[4];
+            T acc = at.active ? (T)0 + term : (T)0;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) acc = acc + __shfl_xor(acc, o);
+            if (threadIdx.x < 4) lds[threadIdx.x] = (T)0;
+            __syncthreads();
+            if (at.w == 0 && lane == 0) lds[at.group] = acc;
+            __syncthreads();
+            if (threadIdx.x == 0) *loss = (((lds[0] + lds[1]) + lds[2]) + lds[3]) / neg_n;
+        } else if (at.active && at.w == 0) {
+            rowloss[at.line] = term;
         }
     }
 }
 
-// one softmax line by one thread; returns the line's cross-entropy term (also stored to rowloss when set)
-template <typename T, bool CE>
-__device__ __forceinline__ T softmax_line(const zmath::ExpLog<T> &ml, const T *x, T *y, int64_t line, int64_t R,
-                                          int64_t inner, const T *target, T *rowloss)
+// lines longer than kLineWaves wavefronts hold, the softmax axis not the last one: one thread walks its line
+template <typename T>
+__global__ __launch_bounds__(kBlock) void softmax_long_lines_kernel(const T *x, T *y, int64_t lines, int64_t R, int64_t inner)
 {
-    int64_t q = line, c = 0;
-    if (inner != 1) {
-        q = line / inner;
-        c = line - q * inner;
-    }
-    const int64_t base = q * R * inner + c;
+    zmath::ExpLog<T> ml;
+    ml.init(true, false);
+    const int64_t line = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (line >= lines) return;
+    const int64_t q = line / inner;
+    const int64_t base = q * R * inner + (line - q * inner);
     const T *xl = x + base;
     T *yl = y + base;
-    if (R <= kLineRegs) {
-        // a short line (the classes of a classifier head) stays in registers: its loads, and those of
-        // the targets, are issued together instead of one per loop iteration, and nothing is read
-        // back.  The operations and their order are those of the loops below.
-        T v[kLineRegs], tg[kLineRegs];
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            const int64_t rl = r < R ? r : 0;
-            v[r] = xl[rl * inner];
-            if (CE) tg[r] = target[base + rl * inner];
-        }
-        T m = v[0];
-#pragma unroll
-        for (int r = 1; r < kLineRegs; r++)
-            if (r < R && v[r] > m) m = v[r];
-        T sum = (T)0;
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            if (r < R) {
-                v[r] = ml.exp(v[r] - m);
-                sum = sum + v[r];
-            }
-        }
-        T acc = (T)0;
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            if (r < R) {
-                const T s = v[r] / sum;
-                yl[r * inner] = s;
-                if (CE) acc = acc + tg[r] * ml.log(s);
-            }
-        }
-        if (CE && rowloss) rowloss[line] = acc;
-        return acc;
-    }
     // max_axis: strict '>' from element 0 (max.rs:19-34)
     T m = xl[0];
     for (int64_t r = 1; r < R; r++) {
@@ -145,148 +199,233 @@ __device__ __forceinline__ T softmax_line(const zmath::ExpLog<T> &ml, const T *x
         yl[r * inner] = e;
         sum = sum + e;
     }
-    T acc = (T)0;
-    for (int64_t r = 0; r < R; r++) {
-        const T s = yl[r * inner] / sum;
-        yl[r * inner] = s;
-        if (CE) acc = acc + target[base + r * inner] * ml.log(s);
-    }
-    if (CE && rowloss) rowloss[line] = acc;
-    return acc;
+    for (int64_t r = 0; r < R; r++) yl[r * inner] = yl[r * inner] / sum;
 }
 
-template <typename T, int VEC, bool CE, bool REG, bool NT, int kBlock = 256, int kRegPacks = 4>
-__global__ __launch_bounds__(kBlock) void softmax_rows_kernel(const T *x, T *y, int64_t R, const T *target,
-                                                               T *rowloss, zmath::ExpLog<T> ml)
+// A row in vectors of any alignment.  Slot k of a thread is the vector at r = tid VEC + k step - head; a slot that
+// sticks out of the row at either end loads the nearest whole vector instead (the load needs no branch) and owns
+// only those of its elements that lie in the slot.
+template <int VEC> struct RowSlot {
+    int at;      // first element loaded
+    int lo, hi;  // elements [lo, hi) of the loaded vector are the slot's own; lo >= VEC or hi <= 0: none
+    __device__ __forceinline__ RowSlot(int r, int R)
+    {
+        at = min(max(r, 0), R - VEC);
+        lo = r - at;
+        hi = VEC + r - at;
+    }
+    __device__ __forceinline__ bool any() const { return lo < VEC && hi > 0; }
+    __device__ __forceinline__ bool own(int j) const { return j >= lo && j < hi; }
+    __device__ __forceinline__ bool full() const { return lo == 0; }
+};
+template <typename T, int VEC, typename Store>
+__device__ __forceinline__ void store_slot(T *row, const RowSlot<VEC> &s, const Pack<T, VEC> &v, Store store)
+{
+    if (s.full()) {
+        store(row, s.at, v);
+    } else {
+#pragma unroll
+        for (int j = 0; j < VEC; j++)
+            if (s.own(j)) row[s.at + j] = v.v[j];
+    }
+}
+// Elements from the row's start to the 128-byte line that it starts in.  Streaming rows are cut into vectors
+// there: wavefronts then write whole lines.
+template <typename T> __device__ __forceinline__ int line_head(const T *row)
+{
+    return (int)((reinterpret_cast<uintptr_t>(row) & 127) / sizeof(T));
+}
+constexpr int kMaxHead = 32;   // elements, at most
+
+// the vectors of a row from element `from` on, `step` apart, four loads in flight; the row's last, partial
+// vector comes as single elements.  fn(r, n, load): n elements at r
+template <typename T, int VEC, typename Fn> __device__ __forceinline__ void stream_row(int64_t from, int64_t step, int64_t R, Fn fn)
+{
+    int64_t r = from;
+    for (; r + 3 * step + VEC <= R; r += 4 * step) fn(r, std::integral_constant<int, 4>(), VEC);
+    for (; r + VEC <= R; r += step) fn(r, std::integral_constant<int, 1>(), VEC);
+    if (r < R) fn(r, std::integral_constant<int, 1>(), (int)(R - r));
+}
+template <typename T, int VEC> __device__ __forceinline__ Pack<T, VEC> load_some(const T *p, int n, T fill)
+{
+    if (n == VEC) return load_pack<T, VEC, false>(p);
+    Pack<T, VEC> v = splat<T, VEC>(fill);
+#pragma unroll
+    for (int j = 0; j < VEC; j++)
+        if (j < n) v.v[j] = p[j];
+    return v;
+}
+template <typename T, int VEC> __device__ __forceinline__ void store_some(T *p, int n, const Pack<T, VEC> &v)
+{
+    if (n == VEC) {
+        store_pack<T, VEC, false>(p, v);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; j++)
+        if (j < n) p[j] = v.v[j];
+}
+
+// The softmax axis is the last one: LANES threads hold a row in registers, EPT elements each, and read and write
+// it once (a wavefront takes a row of its own when LANES == 64).  LONG: the row is longer than that; what is
+// beyond the registers is read three times and its exponentials are computed twice, from and into the same place.
+// Bound by memory and, f32, by the 11 f64 operations of an exp: [2048,32003] f32 108 us (524 MB, 4.8 TB/s), 329 when
+// the row was walked three times with scalar accesses.  One workgroup of 1024 threads per CU takes 146 us: loading,
+// exp and storing follow each other; two of 512 threads with 64 elements each overlap theirs.
+template <typename T, bool CE, bool NT, bool LONG, int LANES, int EPT>
+__global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void softmax_rows_kernel(const T *x, T *y, int64_t rows, int64_t R,
+                                                                                  const T *target, T *rowloss,
+                                                                                  zmath::ExpLog<T> ml)
 {
     // (ml arrives as an argument so that the f64 constants of exp / log sit in scalar registers; written
     // as literals each is copied into a register pair per use, and this kernel is bound by its scalar
     // instructions: the branch-free exp for the same reason)
-    __shared__ T lds[4];
-    if (!REG) ml.init(true, CE);
-    const int64_t row = blockIdx.x;
+    constexpr int VEC = VecOf<T>::N;
+    constexpr int kPacks = EPT / VEC;
+    constexpr int kRows = LANES < 256 ? 256 / LANES : 1;
+    constexpr int step = LANES * VEC;
+    __shared__ T lds[LANES / 64];
+    const int tid = threadIdx.x % LANES;
+    const int64_t row0 = (int64_t)blockIdx.x * kRows + (kRows > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / LANES)) : 0);
+    const bool active = kRows == 1 || row0 < rows;     // uniform per wavefront
+    const int64_t row = active ? row0 : 0;
     const T *xr = x + row * R;
     T *yr = y + row * R;
     const T *tr = CE ? target + row * R : nullptr;
-    const int64_t first = (int64_t)threadIdx.x * VEC;
-    constexpr int64_t step = (int64_t)kBlock * VEC;
+    const int head = (NT && !LONG && R + kMaxHead <= LANES * EPT) ? line_head(yr) : 0;
+    int first = tid * VEC - head;
+    const int Rr = LONG ? LANES * EPT : (int)R;        // the part in registers
     const T x0 = xr[0];
     T acc = (T)0;
 
-    if (REG) {   // R <= kRegPacks * step: the row lives in registers, one read and one write
-        Pack<T, VEC> v[kRegPacks];
-        T m = -INFINITY;
+    Pack<T, VEC> v[kPacks];
 #pragma unroll
-        for (int k = 0; k < kRegPacks; k++) {
-            const int64_t r = first + k * step;
-            v[k] = r < R ? load_pack<T, VEC, NT>(xr + r) : splat<T, VEC>(-INFINITY);
+    for (int k = 0; k < kPacks; k++) v[k] = load_pack<T, VEC, NT>(xr + RowSlot<VEC>(first + k * step, Rr).at);
+    // the targets of the cross-entropy terms travel with the row: loaded where they are used, each
+    // pack cost the end of the kernel a round trip of its own
+    Pack<T, VEC> tg[kPacks];
+    if (CE) {
 #pragma unroll
-            for (int j = 0; j < VEC; j++) m = combine<T, true>(m, v[k].v[j]);
-        }
-        // the targets of the cross-entropy terms travel with the row: loaded where they are used, each
-        // pack cost the end of the kernel a round trip of its own
-        Pack<T, VEC> tg[kRegPacks];
-        if (CE) {
+        for (int k = 0; k < kPacks; k++) tg[k] = load_pack<T, VEC, NT>(tr + RowSlot<VEC>(first + k * step, Rr).at);
+    }
+    ml.init(true, CE);      // after the row's loads are issued: the table fetch overlaps them
+    asm volatile("" : "+v"(first));   // the slots are computed anew in every phase: kept, they take more registers than the row
+    T m = -INFINITY;
 #pragma unroll
-            for (int k = 0; k < kRegPacks; k++) {
-                const int64_t r = first + k * step;
-                tg[k] = load_pack<T, VEC, NT>(tr + (r < R ? r : 0));
-            }
-        }
-        ml.init(true, CE);      // after the row's loads are issued: the table fetch overlaps them
-        m = block_red<T, true, kBlock>(m, lds);
-        if (x0 != x0) m = x0;   // a NaN in position 0 is never replaced
-        T sum = (T)0;
-        T least = INFINITY;     // the smallest of this thread's terms
+    for (int k = 0; k < kPacks; k++) {
+        const RowSlot<VEC> s(first + k * step, Rr);
 #pragma unroll
-        for (int k = 0; k < kRegPacks; k++) {
-            if (first + k * step < R) {
-#pragma unroll
-                for (int j = 0; j < VEC; j++) {
-                    v[k].v[j] = ml.exp_flat(v[k].v[j] - m);
-                    sum = sum + v[k].v[j];
-                    least = v[k].v[j] < least ? v[k].v[j] : least;
-                }
-            }
-        }
-        sum = block_red<T, false, kBlock>(sum, lds);
-        // Every quotient of the row has the same divisor.  With r = RN(1 / sum): q0 = RN(a r), the
-        // exact remainder a - sum q0 (one fma) and q = fma(remainder, r, q0) is the correctly rounded
-        // a / sum (Markstein) unless the divisor's mantissa is all ones, as long as nothing underflows:
-        // three instructions per element instead of the division's eleven.  The thread takes that road
-        // when its terms are at least 2^-64 and the sum lies in [1, 2^23) (quotient and remainder stay
-        // normal); otherwise it divides.  On 9.6e9 random pairs from those ranges (terms down to 2^-80)
-        // the host finds no quotient that differs from the division's.
-        bool shared_divisor = false;
-        if constexpr (sizeof(T) == 4) {
-            uint32_t sb;
-            __builtin_memcpy(&sb, &sum, 4);
-            shared_divisor = least >= (T)0x1p-64f && sum >= (T)1 && sum < (T)0x1p23f && (sb & 0x7fffffu) != 0x7fffffu;
-        }
-        auto finish = [&](auto by_reciprocal) {
-            const T rcp = decltype(by_reciprocal)::value ? (T)1 / sum : (T)0;
-#pragma unroll
-            for (int k = 0; k < kRegPacks; k++) {
-                const int64_t r = first + k * step;
-                if (r < R) {
-                    const Pack<T, VEC> t = tg[k];
-#pragma unroll
-                    for (int j = 0; j < VEC; j++) {
-                        T s;
-                        if constexpr (decltype(by_reciprocal)::value && sizeof(T) == 4) {
-                            const float a = v[k].v[j];
-                            const float q0 = a * rcp;
-                            s = __builtin_fmaf(__builtin_fmaf(-sum, q0, a), rcp, q0);
-                        } else {
-                            s = v[k].v[j] / sum;
-                        }
-                        v[k].v[j] = s;
-                        if (CE) acc = acc + t.v[j] * ml.log(s);
-                    }
-                    // the CE output is read again by the backward pass; plain softmax is one stream in, one out
-                    if constexpr (NT && !CE && VEC > 1) store_pack_wt<T, VEC>(yr + r, v[k]);
-                    else store_pack<T, VEC, false>(yr + r, v[k]);
-                }
-            }
-        };
-        if (shared_divisor) finish(std::true_type());
-        else finish(std::false_type());
-    } else {     // long rows: three passes; the second and third find the row in cache
-        T m = -INFINITY;
-        for (int64_t r = first; r < R; r += step) {
-            const Pack<T, VEC> v = load_pack<T, VEC, false>(xr + r);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) m = combine<T, true>(m, v.v[j]);
-        }
-        m = block_red<T, true, kBlock>(m, lds);
-        if (x0 != x0) m = x0;
-        T sum = (T)0;
-        for (int64_t r = first; r < R; r += step) {
-            Pack<T, VEC> v = load_pack<T, VEC, false>(xr + r);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                v.v[j] = ml.exp_flat(v.v[j] - m);
-                sum = sum + v.v[j];
-            }
-            store_pack<T, VEC, false>(yr + r, v);
-        }
-        sum = block_red<T, false, kBlock>(sum, lds);
-        for (int64_t r = first; r < R; r += step) {   // each thread re-reads what it wrote itself
-            Pack<T, VEC> v = load_pack<T, VEC, false>(yr + r);
-            Pack<T, VEC> t;
-            if (CE) t = load_pack<T, VEC, false>(tr + r);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                const T s = v.v[j] / sum;
-                v.v[j] = s;
-                if (CE) acc = acc + t.v[j] * ml.log(s);
-            }
-            store_pack<T, VEC, false>(yr + r, v);
+        for (int j = 0; j < VEC; j++) {
+            if (!LONG) v[k].v[j] = s.own(j) ? v[k].v[j] : -(T)INFINITY;
+            m = combine<T, true>(m, v[k].v[j]);
         }
     }
+    if constexpr (LONG) {
+        stream_row<T, VEC>(Rr + first, step, R, [&](int64_t r, auto count, int n) {
+            constexpr int U = decltype(count)::value;
+            Pack<T, VEC> p[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) p[u] = load_some<T, VEC>(xr + r + u * step, n, -(T)INFINITY);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int j = 0; j < VEC; j++) m = combine<T, true>(m, p[u].v[j]);
+        });
+    }
+    m = block_red<T, true, LANES>(m, lds);
+    if (x0 != x0) m = x0;   // a NaN in position 0 is never replaced
+    asm volatile("" : "+v"(first));
+    T sum = (T)0;
+    uint32_t least = ~0u;   // f32: the smallest of this thread's terms above zero, as its bits less one
+#pragma unroll
+    for (int k = 0; k < kPacks; k++) {
+        if (LONG || RowSlot<VEC>(first + k * step, Rr).any()) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) {      // an element that is not the slot's own is exp(-inf), zero
+                v[k].v[j] = ml.exp_flat(v[k].v[j] - m);
+                sum = sum + v[k].v[j];
+                if constexpr (sizeof(T) == 4) least = min(least, __float_as_uint(v[k].v[j]) - 1u);
+            }
+        }
+    }
+    if constexpr (LONG) {
+        stream_row<T, VEC>(Rr + first, step, R, [&](int64_t r, auto count, int n) {
+            constexpr int U = decltype(count)::value;
+            Pack<T, VEC> p[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) p[u] = load_some<T, VEC>(xr + r + u * step, n, -(T)INFINITY);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int j = 0; j < VEC; j++) sum = sum + ml.exp_flat(p[u].v[j] - m);
+        });
+    }
+    sum = block_red<T, false, LANES>(sum, lds);
+    // Every quotient of the row has the same divisor.  With r = RN(1 / sum): q0 = RN(a r), the
+    // exact remainder a - sum q0 (one fma) and q = fma(remainder, r, q0) is the correctly rounded
+    // a / sum (Markstein) unless the divisor's mantissa is all ones, as long as nothing underflows:
+    // three instructions per element instead of the division's eleven.  The thread takes that road
+    // when its terms are zero (the quotient is, too) or at least 2^-64 and the sum lies in [1, 2^23) (quotient
+    // and remainder stay normal); otherwise it divides.  On 9.6e9 random pairs from those ranges (terms down to
+    // 2^-80) the host finds no quotient that differs from the division's.
+    bool shared_divisor = false;
+    if constexpr (sizeof(T) == 4)
+        shared_divisor = least >= __float_as_uint(0x1p-64f) - 1u && sum >= (T)1 && sum < (T)0x1p23f &&
+                         (__float_as_uint(sum) & 0x7fffffu) != 0x7fffffu;
+    asm volatile("" : "+v"(first));
+    auto finish = [&](auto by_reciprocal) {
+        const T rcp = decltype(by_reciprocal)::value ? (T)1 / sum : (T)0;
+#pragma unroll
+        for (int k = 0; k < kPacks; k++) {
+            const RowSlot<VEC> slot(first + k * step, Rr);
+            if (LONG || slot.any()) {
+                const Pack<T, VEC> t = tg[k];
+#pragma unroll
+                for (int j = 0; j < VEC; j++) {
+                    T s;
+                    if constexpr (decltype(by_reciprocal)::value && sizeof(T) == 4) {
+                        const float a = v[k].v[j];
+                        const float q0 = a * rcp;
+                        s = __builtin_fmaf(__builtin_fmaf(-sum, q0, a), rcp, q0);
+                    } else {
+                        s = v[k].v[j] / sum;
+                    }
+                    v[k].v[j] = s;
+                    if (CE) acc = (LONG || slot.own(j)) ? acc + t.v[j] * ml.log(s) : acc;
+                }
+                // the CE output is read again by the backward pass; plain softmax is one stream in, one out
+                if (active)
+                    store_slot<T, VEC>(yr, slot, v[k], [](T *row, int at, const Pack<T, VEC> &z) {
+                        if constexpr (NT && !CE) store_pack_wt_at<T, VEC>(row, at, z);
+                        else store_pack<T, VEC, false>(row + at, z);
+                    });
+            }
+        }
+    };
+    if (shared_divisor) finish(std::true_type());
+    else finish(std::false_type());
+    if constexpr (LONG) {       // each thread re-reads the elements that it writes
+        stream_row<T, VEC>(Rr + first, step, R, [&](int64_t r, auto count, int n) {
+            constexpr int U = decltype(count)::value;
+            Pack<T, VEC> p[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) p[u] = load_some<T, VEC>(xr + r + u * step, n, -(T)INFINITY);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                Pack<T, VEC> t;
+                if (CE) t = load_some<T, VEC>(tr + r + u * step, n, (T)0);
+#pragma unroll
+                for (int j = 0; j < VEC; j++) {
+                    p[u].v[j] = ml.exp_flat(p[u].v[j] - m) / sum;
+                    if (CE) acc = j < n ? acc + t.v[j] * ml.log(p[u].v[j]) : acc;
+                }
+                store_some<T, VEC>(yr + r + u * step, n, p[u]);
+            }
+        });
+    }
     if (CE) {
-        acc = block_red<T, false, kBlock>(acc, lds);
-        if (threadIdx.x == 0) rowloss[row] = acc;
+        acc = block_red<T, false, LANES>(acc, lds);
+        if (active && tid == 0) rowloss[row] = acc;
     }
 }
 
@@ -313,183 +452,148 @@ __global__ __launch_bounds__(kBlock) void ce_finalize_kernel(const T *rowloss, i
 // gx = t - y * sum(t), t = y * gy.  CE: gy = (target * g_total) / y with g_total = gout / (-N), the
 // chain div -> sum_to -> mul -> log backward of cross_entropy.rs:18-22.
 
-template <typename T, bool CE> struct GySource {
-    const T *p;        // gy, or the target when CE
-    T g_total;
-    __device__ __forceinline__ T get(int64_t off, T yv) const
-    {
-        if (CE) return (p[off] * g_total) / yv;
-        return p[off];
+// lines in registers, as in softmax_lines_kernel; the sum of t in index order
+template <typename T, bool CE, int OWN>
+__global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(const T *y, const T *gy_or_target, T *gx,
+                                                                             int64_t lines, int R, int64_t inner,
+                                                                             int waves, const T *gout, T neg_n)
+{
+    __shared__ T carry[kLineWaves * 64];
+    const LineSpot at(lines, R, inner, waves);
+    const T g_total = CE ? (gout ? *gout : (T)1) / neg_n : (T)0;
+    const int r0 = at.w * OWN;
+    const int valid = R - r0;
+    const int64_t base = at.base + r0 * inner;
+    T yv[OWN], t[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; i += 4) {
+        if (i < valid) {
+#pragma unroll
+            for (int j = i; j < i + 4; j++) {
+                const int64_t off = base + (j < valid ? j : 0) * inner;
+                yv[j] = y[off];
+                t[j] = gy_or_target[off];
+            }
+        }
     }
-};
+#pragma unroll
+    for (int i = 0; i < OWN; i++)
+        if (i < valid) t[i] = yv[i] * (CE ? (t[i] * g_total) / yv[i] : t[i]);
+    const T sum = sum_in_order<T, OWN>(t, valid, at, waves, carry);
+    if (!at.active) return;
+#pragma unroll
+    for (int i = 0; i < OWN; i++)
+        if (i < valid) gx[base + i * inner] = t[i] - yv[i] * sum;
+}
 
-// With `colsum` set (every line in this one workgroup, lines of at most kLineRegs elements, inner == 1)
-// the kernel also writes the column sums of gx -- the bias gradient of the Linear layer that
-// produced the logits (zenu-layer/src/layers/linear.rs:27-31 through the `sum_to` of
-// zenu-autograd/src/lib.rs:466-486) -- each folded over the lines in the fixed order of block_red.
-template <typename T, bool CE>
-__global__ __launch_bounds__(kBlock) void softmax_bwd_lines_kernel(const T *y, const T *gy_or_target, T *gx,
-                                                                    int64_t lines, int64_t R, int64_t inner,
-                                                                    const T *gout, T neg_n, T *colsum)
+// lines longer than that, the softmax axis not the last one
+template <typename T>
+__global__ __launch_bounds__(kBlock) void softmax_bwd_long_lines_kernel(const T *y, const T *gy, T *gx, int64_t lines,
+                                                                         int64_t R, int64_t inner)
 {
     const int64_t line = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (colsum) {    // uniform; the host sends this only with R <= kLineRegs, inner == 1, one workgroup
-        __shared__ T lds[kLineRegs * kWaves];
-        const bool active = line < lines;
-        const T g_total = CE ? (gout ? *gout : (T)1) / neg_n : (T)0;
-        const int64_t base = (active ? line : 0) * R;
-        T yv[kLineRegs], pv[kLineRegs], t[kLineRegs];
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            const int64_t off = base + (r < R ? r : 0);
-            yv[r] = y[off];
-            pv[r] = gy_or_target[off];
-        }
-        T sum = (T)0;
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            if (r < R) {
-                t[r] = yv[r] * (CE ? (pv[r] * g_total) / yv[r] : pv[r]);
-                sum = sum + t[r];
-            }
-        }
-        // the column sums in the order of block_red (butterfly inside a wavefront, then the wavefronts
-        // in index order), all columns behind ONE barrier instead of two per column
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            if (r < R) {
-                const T g = t[r] - yv[r] * sum;
-                if (active) gx[base + r] = g;
-                T c = (T)0;
-                if (active) c = c + g;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) c = c + __shfl_xor(c, o);
-                if ((threadIdx.x & 63) == 0) lds[r * kWaves + (threadIdx.x >> 6)] = c;
-            }
-        }
-        __syncthreads();
-        if ((int64_t)threadIdx.x < R) {
-            T c = lds[threadIdx.x * kWaves];
-#pragma unroll
-            for (int w = 1; w < kWaves; w++) c = c + lds[threadIdx.x * kWaves + w];
-            colsum[threadIdx.x] = c;
-        }
-        return;
-    }
     if (line >= lines) return;
-    GySource<T, CE> src;
-    src.p = gy_or_target;
-    src.g_total = CE ? (gout ? *gout : (T)1) / neg_n : (T)0;
-    int64_t q = line, c = 0;
-    if (inner != 1) {
-        q = line / inner;
-        c = line - q * inner;
-    }
-    const int64_t base = q * R * inner + c;
-    if (R <= kLineRegs) {     // a short line in registers, as in the forward kernel: same operations, same order
-        T yv[kLineRegs], pv[kLineRegs], t[kLineRegs];
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            const int64_t off = base + (r < R ? r : 0) * inner;
-            yv[r] = y[off];
-            pv[r] = gy_or_target[off];
-        }
-        T sum = (T)0;
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++) {
-            if (r < R) {
-                t[r] = yv[r] * (CE ? (pv[r] * src.g_total) / yv[r] : pv[r]);
-                sum = sum + t[r];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < kLineRegs; r++)
-            if (r < R) gx[base + r * inner] = t[r] - yv[r] * sum;
-        return;
-    }
+    const int64_t q = line / inner;
+    const int64_t base = q * R * inner + (line - q * inner);
     T sum = (T)0;
+    for (int64_t r = 0; r < R; r++) {
+        const int64_t off = base + r * inner;
+        sum = sum + y[off] * gy[off];
+    }
     for (int64_t r = 0; r < R; r++) {
         const int64_t off = base + r * inner;
         const T yv = y[off];
-        const T t = yv * src.get(off, yv);
-        gx[off] = t;
-        sum = sum + t;
-    }
-    for (int64_t r = 0; r < R; r++) {
-        const int64_t off = base + r * inner;
-        gx[off] = gx[off] - y[off] * sum;
+        gx[off] = yv * gy[off] - yv * sum;
     }
 }
 
-template <typename T, int VEC, bool CE, bool REG, bool NT>
-__global__ __launch_bounds__(kBlock) void softmax_bwd_rows_kernel(const T *y, const T *gy_or_target, T *gx,
-                                                                   int64_t R, const T *gout, T neg_n)
+// Rows in registers, as in softmax_rows_kernel: y and y * gy are held, two reads and one write.  LONG: what is
+// beyond the registers is read twice.  [2048,32003] f32 134 us (787 MB, 5.9 TB/s), 311 with scalar accesses
+// and t written out and read back.
+template <typename T, bool CE, bool NT, bool LONG, int LANES, int EPT>
+__global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void softmax_bwd_rows_kernel(const T *y, const T *gy_or_target, T *gx,
+                                                                                      int64_t rows, int64_t R,
+                                                                                      const T *gout, T neg_n)
 {
-    __shared__ T lds[kWaves];
+    constexpr int VEC = VecOf<T>::N;
+    constexpr int kPacks = EPT / VEC;
+    constexpr int kRows = LANES < 256 ? 256 / LANES : 1;
+    constexpr int step = LANES * VEC;
+    __shared__ T lds[LANES / 64];
     const T g_total = CE ? (gout ? *gout : (T)1) / neg_n : (T)0;
-    const int64_t base = (int64_t)blockIdx.x * R;
+    const int tid = threadIdx.x % LANES;
+    const int64_t row = (int64_t)blockIdx.x * kRows + (kRows > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / LANES)) : 0);
+    if (kRows > 1 && row >= rows) return;      // a wavefront per row: no barrier follows
+    const int64_t base = row * R;
     const T *yr = y + base;
     const T *sr = gy_or_target + base;
     T *gr = gx + base;
-    const int64_t first = (int64_t)threadIdx.x * VEC;
-    constexpr int64_t step = (int64_t)kBlock * VEC;
+    const int head = (NT && !LONG && R + kMaxHead <= LANES * EPT) ? line_head(gr) : 0;
+    const int first = tid * VEC - head;
+    const int Rr = LONG ? LANES * EPT : (int)R;
+    auto product = [&](T yv, T g) { return yv * (CE ? (g * g_total) / yv : g); };
     T sum = (T)0;
-    if (REG) {   // the row of y and of t = y * gy stays in registers: two reads, one write
-        Pack<T, VEC> yv[kRegPacks], gv[kRegPacks], t[kRegPacks];
-        // all loads of the thread first (a pack past the end of the row reads the row's first one and
-        // is not used): with the loads inside the bounds check the compiler waits for each pair
-        // before it issues the next, because the running sum orders the blocks
+    Pack<T, VEC> yv[kPacks], t[kPacks];
+    // all loads of the thread first: with the loads inside a bounds check the compiler waits for each pair
+    // before it issues the next, because the running sum orders the blocks
 #pragma unroll
-        for (int k = 0; k < kRegPacks; k++) {
-            const int64_t r = first + k * step;
-            const int64_t rl = r < R ? r : 0;
-            yv[k] = load_pack<T, VEC, NT && !CE>(yr + rl);
-            gv[k] = load_pack<T, VEC, NT>(sr + rl);
-        }
+    for (int k = 0; k < kPacks; k++) {
+        const RowSlot<VEC> s(first + k * step, Rr);
+        yv[k] = load_pack<T, VEC, NT && !CE>(yr + s.at);
+        t[k] = load_pack<T, VEC, NT>(sr + s.at);
+    }
 #pragma unroll
-        for (int k = 0; k < kRegPacks; k++) {
-            const int64_t r = first + k * step;
-            if (r < R) {
-                const Pack<T, VEC> g = gv[k];
-#pragma unroll
-                for (int j = 0; j < VEC; j++) {
-                    const T gyv = CE ? (g.v[j] * g_total) / yv[k].v[j] : g.v[j];
-                    t[k].v[j] = yv[k].v[j] * gyv;
-                    sum = sum + t[k].v[j];
-                }
-            }
-        }
-        sum = block_red<T, false>(sum, lds);
-#pragma unroll
-        for (int k = 0; k < kRegPacks; k++) {
-            const int64_t r = first + k * step;
-            if (r < R) {
-#pragma unroll
-                for (int j = 0; j < VEC; j++) t[k].v[j] = t[k].v[j] - yv[k].v[j] * sum;
-                store_pack<T, VEC, NT>(gr + r, t[k]);
-            }
-        }
-    } else {     // long rows: t goes to gx first; the second pass finds both rows in cache
-        for (int64_t r = first; r < R; r += step) {
-            const Pack<T, VEC> yv = load_pack<T, VEC, false>(yr + r);
-            const Pack<T, VEC> g = load_pack<T, VEC, false>(sr + r);
-            Pack<T, VEC> t;
+    for (int k = 0; k < kPacks; k++) {
+        const RowSlot<VEC> s(first + k * step, Rr);
+        if (LONG || s.any()) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) {
-                const T gyv = CE ? (g.v[j] * g_total) / yv.v[j] : g.v[j];
-                t.v[j] = yv.v[j] * gyv;
-                sum = sum + t.v[j];
+                t[k].v[j] = product(yv[k].v[j], t[k].v[j]);
+                sum = (LONG || s.own(j)) ? sum + t[k].v[j] : sum;
             }
-            store_pack<T, VEC, false>(gr + r, t);
         }
-        sum = block_red<T, false>(sum, lds);
-        for (int64_t r = first; r < R; r += step) {
-            const Pack<T, VEC> yv = load_pack<T, VEC, false>(yr + r);
-            Pack<T, VEC> t = load_pack<T, VEC, false>(gr + r);
+    }
+    if constexpr (LONG) {
+        stream_row<T, VEC>(Rr + first, step, R, [&](int64_t r, auto count, int n) {
+            constexpr int U = decltype(count)::value;
+            Pack<T, VEC> a[U], b[U];
 #pragma unroll
-            for (int j = 0; j < VEC; j++) t.v[j] = t.v[j] - yv.v[j] * sum;
-            store_pack<T, VEC, false>(gr + r, t);
+            for (int u = 0; u < U; u++) {
+                a[u] = load_some<T, VEC>(yr + r + u * step, n, (T)1);
+                b[u] = load_some<T, VEC>(sr + r + u * step, n, (T)0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int j = 0; j < VEC; j++) sum = j < n ? sum + product(a[u].v[j], b[u].v[j]) : sum;
+        });
+    }
+    sum = block_red<T, false, LANES>(sum, lds);
+#pragma unroll
+    for (int k = 0; k < kPacks; k++) {
+        const RowSlot<VEC> s(first + k * step, Rr);
+        if (LONG || s.any()) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) t[k].v[j] = t[k].v[j] - yv[k].v[j] * sum;
+            store_slot<T, VEC>(gr, s, t[k], [](T *row, int at, const Pack<T, VEC> &z) { store_pack<T, VEC, NT>(row + at, z); });
         }
+    }
+    if constexpr (LONG) {       // each thread re-reads the elements that it writes
+        stream_row<T, VEC>(Rr + first, step, R, [&](int64_t r, auto count, int n) {
+            constexpr int U = decltype(count)::value;
+            Pack<T, VEC> a[U], b[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                a[u] = load_some<T, VEC>(yr + r + u * step, n, (T)1);
+                b[u] = load_some<T, VEC>(sr + r + u * step, n, (T)0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int j = 0; j < VEC; j++) b[u].v[j] = product(a[u].v[j], b[u].v[j]) - a[u].v[j] * sum;
+                store_some<T, VEC>(gr + r + u * step, n, b[u]);
+            }
+        });
     }
 }
 
@@ -747,11 +851,68 @@ inline bool ce_single_workgroup(const Geometry &g)
     return g.inner == 1 && g.R <= kLineMaxR && g.outer <= kBlock;
 }
 
+// How many elements of a line a thread of the lines kernels holds: as many as leave every SIMD two wavefronts, so
+// that a large tensor needs no hand-over of sums and a small one is not a single thread's long chain; never so few
+// that the line needs more than kLineWaves wavefronts.  0: the line is too long for them.
+inline int line_own(int64_t lines, int64_t R, int most)
+{
+    const int64_t groups = (lines + 63) / 64;
+    const int64_t want = 8 * (int64_t)device_info().num_cus;
+    for (int own = most; own >= 8; own /= 2) {
+        if (R > (int64_t)own * kLineWaves) return own == most ? 0 : 2 * own;
+        if (groups * ((R + own - 1) / own) >= want) return own;
+    }
+    return 8;
+}
+// calls go(own) with `own` as a constant
+template <int MOST, typename Go> int with_own(int own, Go go)
+{
+    if constexpr (MOST >= 32)
+        if (own == 32) return go(std::integral_constant<int, 32>());
+    if (own == 16) return go(std::integral_constant<int, 16>());
+    return go(std::integral_constant<int, 8>());
+}
+// wavefronts along a line, and lines in groups of 64 that fill a workgroup of about four wavefronts
+struct LineGrid {
+    int waves, groups;
+    int64_t blocks;
+    LineGrid(int64_t lines, int64_t R, int own, bool one_workgroup)
+    {
+        const int64_t all = (lines + 63) / 64;
+        waves = (int)((R + own - 1) / own);
+        groups = waves >= 4 ? 1 : 4 / waves;
+        if (one_workgroup || groups > all) groups = (int)all;
+        blocks = (all + groups - 1) / groups;
+    }
+    unsigned threads() const { return (unsigned)(64 * waves * groups); }
+};
+
+// elements per thread of the largest workgroups, which leave a thread 128 registers: y and t of the backward pass, or
+// the terms of the forward pass with the constants of exp, in 64 of them (f64 with 32 elements spills)
+template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
+
+// Threads per row and elements per thread of the rows kernels by row length; `spare` leaves
+// room for the alignment of a streaming row.  go(lanes, elements, long) gets constants.
+template <int EPT_LONG, typename Go> int with_row_shape(int64_t R, bool spare, Go go)
+{
+    const int64_t need = R + (spare ? kMaxHead : 0);
+    typedef std::integral_constant<int, 64> L64;
+    typedef std::integral_constant<int, 256> L256;
+    typedef std::integral_constant<int, 512> L512;
+    typedef std::integral_constant<int, 1024> L1024;
+    typedef std::integral_constant<int, EPT_LONG> Long;
+    if (need <= 512) return go(L64(), std::integral_constant<int, 8>(), std::false_type());
+    if (need <= 1024) return go(L256(), std::integral_constant<int, 4>(), std::false_type());
+    if (need <= 4096) return go(L256(), std::integral_constant<int, 16>(), std::false_type());
+    if (need <= 512 * EPT_LONG) return go(L512(), Long(), std::false_type());
+    if (R <= 1024 * EPT_LONG) return go(L1024(), Long(), std::false_type());
+    return go(L1024(), Long(), std::true_type());
+}
+
 template <typename T, bool CE>
 int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *rowloss, hipStream_t s,
                            T *loss = nullptr, T neg_n = (T)0)
 {
-    constexpr int VEC = VecOf<T>::N;
     const int64_t lines = g.outer * g.inner;
     if constexpr (CE) {
         if (loss && g.inner == 1 && g.R <= kLineRegs && lines <= kHeadLines) {   // a classifier head: four lanes per line
@@ -761,22 +922,37 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
         }
     }
     if (g.inner != 1 || g.R <= kLineMaxR) {
-        const int64_t blocks = (lines + kBlock - 1) / kBlock;
-        if (!grid_ok(blocks)) return ZENU_ERR_UNSUPPORTED;
-        T *fold = (CE && blocks == 1) ? loss : nullptr;
-        softmax_lines_kernel<T, CE><<<(unsigned)blocks, kBlock, 0, s>>>(x, y, lines, g.R, g.inner, target, rowloss, fold, neg_n);
+        // (16 elements at most where the whole loss is one workgroup: 16 wavefronts hold 256 lines of 64)
+        int own = line_own(lines, g.R, 32);
+        if (CE && loss && own < 16 && (lines + 63) / 64 * ((g.R + own - 1) / own) > kLineWaves) own = 16;
+        if (own == 0) {
+            const int64_t blocks = (lines + kBlock - 1) / kBlock;
+            if (!grid_ok(blocks)) return ZENU_ERR_UNSUPPORTED;
+            softmax_long_lines_kernel<T><<<(unsigned)blocks, kBlock, 0, s>>>(x, y, lines, g.R, g.inner);
+        } else {
+            const LineGrid lg(lines, g.R, own, CE && loss);
+            if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
+            with_own<32>(own, [&](auto o) {
+                softmax_lines_kernel<T, CE, decltype(o)::value><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
+                    x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
+                return 0;
+            });
+        }
     } else {
-        if (!grid_ok(lines)) return ZENU_ERR_UNSUPPORTED;
-        const bool vec = g.R % VEC == 0 && aligned16(x) && aligned16(y) && (!CE || aligned16(target));
-        const bool reg = g.R <= (int64_t)kRegPacks * kBlock * (vec ? VEC : 1);
-        const unsigned grid = (unsigned)lines;
-        const bool nt = vec && reg && lines * g.R * (int64_t)sizeof(T) * 2 >= kStreamBytes;
-        // (one wavefront or 128 threads per row with more vectors per lane measured 4-9 % slower)
-        if (nt)               softmax_rows_kernel<T, VEC, CE, true, true><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
-        else if (vec && reg)  softmax_rows_kernel<T, VEC, CE, true, false><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
-        else if (vec)         softmax_rows_kernel<T, VEC, CE, false, false><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
-        else if (reg)         softmax_rows_kernel<T, 1, CE, true, false><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
-        else                  softmax_rows_kernel<T, 1, CE, false, false><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
+        const bool nt = lines * g.R * (int64_t)sizeof(T) * 2 >= kStreamBytes;
+        const int rc = with_row_shape<kMost<T>>(g.R, nt, [&](auto lanes, auto ept, auto is_long) -> int {
+            constexpr bool LONG = decltype(is_long)::value;
+            // f32: two workgroups of 512 threads on a CU instead of one of 1024, see softmax_rows_kernel
+            constexpr bool two = decltype(lanes)::value == 1024 && decltype(ept)::value == 32 && !LONG && !CE;
+            constexpr int L = two ? 512 : decltype(lanes)::value, E = two ? 64 : decltype(ept)::value;
+            constexpr int B = L < 256 ? 256 : L;
+            const int64_t grid = (lines + B / L - 1) / (B / L);
+            if (!grid_ok(grid)) return ZENU_ERR_UNSUPPORTED;
+            if (nt) softmax_rows_kernel<T, CE, true, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(x, y, lines, g.R, target, rowloss, zmath::ExpLog<T>());
+            else    softmax_rows_kernel<T, CE, false, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(x, y, lines, g.R, target, rowloss, zmath::ExpLog<T>());
+            return ZENU_OK;
+        });
+        if (rc) return rc;
     }
     ZENU_LAUNCH_CHECK();
     return ZENU_OK;
@@ -787,7 +963,7 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
                             hipStream_t s, T *colsum = nullptr)
 {
     const int64_t lines = g.outer * g.inner;
-    if (colsum && !(g.inner == 1 && g.R <= kLineRegs && lines <= kBlock)) return ZENU_ERR_UNSUPPORTED;
+    if (colsum && !(g.inner == 1 && g.R <= kLineRegs && lines <= kHeadLines)) return ZENU_ERR_UNSUPPORTED;
     if constexpr (CE) {
         if (g.inner == 1 && g.R <= kLineRegs && lines <= kHeadLines) {           // a classifier head: four lanes per line
             ce_head_backward_kernel<T><<<1, kHeadBlock, 0, s>>>(y, gy_or_target, gx, lines, g.R, gout, neg_n, colsum);
@@ -796,22 +972,33 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
         }
     }
     if (g.inner != 1 || g.R <= kLineMaxR) {
-        const int64_t blocks = (lines + kBlock - 1) / kBlock;
-        if (!grid_ok(blocks)) return ZENU_ERR_UNSUPPORTED;
-        softmax_bwd_lines_kernel<T, CE><<<(unsigned)blocks, kBlock, 0, s>>>(y, gy_or_target, gx, lines, g.R, g.inner,
-                                                                             gout, neg_n, colsum);
+        const int own = line_own(lines, g.R, kMost<T>);
+        if (own == 0) {
+            const int64_t blocks = (lines + kBlock - 1) / kBlock;
+            if (!grid_ok(blocks)) return ZENU_ERR_UNSUPPORTED;
+            softmax_bwd_long_lines_kernel<T><<<(unsigned)blocks, kBlock, 0, s>>>(y, gy_or_target, gx, lines, g.R, g.inner);
+        } else {
+            const LineGrid lg(lines, g.R, own, false);
+            if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
+            with_own<kMost<T>>(own, [&](auto o) {
+                softmax_bwd_lines_kernel<T, CE, decltype(o)::value><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
+                    y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
+                return 0;
+            });
+        }
     } else {
-        if (!grid_ok(lines)) return ZENU_ERR_UNSUPPORTED;
-        constexpr int VEC = VecOf<T>::N;
-        const bool vec = g.R % VEC == 0 && aligned16(y) && aligned16(gy_or_target) && aligned16(gx);
-        const bool reg = g.R <= (int64_t)kRegPacks * kBlock * (vec ? VEC : 1);
-        const bool nt = vec && reg && lines * g.R * (int64_t)sizeof(T) * 3 >= kStreamBytes;
-        const unsigned grid = (unsigned)lines;
-        if (nt)              softmax_bwd_rows_kernel<T, VEC, CE, true, true><<<grid, kBlock, 0, s>>>(y, gy_or_target, gx, g.R, gout, neg_n);
-        else if (vec && reg) softmax_bwd_rows_kernel<T, VEC, CE, true, false><<<grid, kBlock, 0, s>>>(y, gy_or_target, gx, g.R, gout, neg_n);
-        else if (vec)        softmax_bwd_rows_kernel<T, VEC, CE, false, false><<<grid, kBlock, 0, s>>>(y, gy_or_target, gx, g.R, gout, neg_n);
-        else if (reg)        softmax_bwd_rows_kernel<T, 1, CE, true, false><<<grid, kBlock, 0, s>>>(y, gy_or_target, gx, g.R, gout, neg_n);
-        else                 softmax_bwd_rows_kernel<T, 1, CE, false, false><<<grid, kBlock, 0, s>>>(y, gy_or_target, gx, g.R, gout, neg_n);
+        const bool nt = lines * g.R * (int64_t)sizeof(T) * 3 >= kStreamBytes;
+        const int rc = with_row_shape<kMost<T>>(g.R, nt, [&](auto lanes, auto ept, auto is_long) -> int {
+            constexpr int L = decltype(lanes)::value, E = decltype(ept)::value;
+            constexpr bool LONG = decltype(is_long)::value;
+            constexpr int B = L < 256 ? 256 : L;
+            const int64_t grid = (lines + B / L - 1) / (B / L);
+            if (!grid_ok(grid)) return ZENU_ERR_UNSUPPORTED;
+            if (nt) softmax_bwd_rows_kernel<T, CE, true, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(y, gy_or_target, gx, lines, g.R, gout, neg_n);
+            else    softmax_bwd_rows_kernel<T, CE, false, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(y, gy_or_target, gx, lines, g.R, gout, neg_n);
+            return ZENU_OK;
+        });
+        if (rc) return rc;
     }
     ZENU_LAUNCH_CHECK();
     return ZENU_OK;

@@ -55,14 +55,25 @@ template <typename T, int N, bool NT> __device__ __forceinline__ void store_pack
 // or more load streams beside the store (add: 31.8 us with `nt`, 32.1 - 32.2 us with `sc1 nt`;
 // the seven streams of Adam: 114.5 against 115.8 us) plain `nt` stays ahead.  The compiler has no
 // spelling for this combination, so the instruction is written out; the s_nop keeps the data
-// registers untouched for the one wait state a 128-bit store needs after issue.
+// registers untouched for the two wait states that a store of more than 64 bits needs after issue on gfx940 and
+// later, before a vector instruction writes to them (the compiler inserts them for stores of its own only).
 template <typename T, int N> __device__ __forceinline__ void store_pack_wt(T *p, const Pack<T, N> &r)
 {
     static_assert(sizeof(T) * N == 16, "128-bit packs only");
     typedef typename NativeVec<T, N>::type V;
     V x;
     __builtin_memcpy(&x, &r, sizeof(V));
-    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0" ::"v"(reinterpret_cast<V *>(p)), "v"(x) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(reinterpret_cast<V *>(p)), "v"(x) : "memory");
+}
+
+// the same at row + at, `row` being the same in the whole wavefront and 0 <= at < 2^29: one address register
+template <typename T, int N> __device__ __forceinline__ void store_pack_wt_at(T *row, int at, const Pack<T, N> &r)
+{
+    static_assert(sizeof(T) * N == 16, "128-bit packs only");
+    typedef typename NativeVec<T, N>::type V;
+    V x;
+    __builtin_memcpy(&x, &r, sizeof(V));
+    asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" ::"v"(at * (int)sizeof(T)), "v"(x), "s"(row) : "memory");
 }
 
 template <typename T, int N> __device__ __forceinline__ Pack<T, N> splat(T s)
