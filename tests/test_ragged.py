@@ -86,3 +86,43 @@ def test_streaming_sizes(hip):
     same(out.to_numpy(), b.T, "transposed copy")
     out.relu(A, 0.0)
     same(out.to_numpy(), np.maximum(a, 0), "relu")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("largest", [4099, 1 << 20], ids=["cached", "streamed"])
+def test_optimizer_tensors_of_any_size_and_alignment(hip, dtype, largest):
+    """More tensors than one launch holds, around a vector and a tile long, each at another alignment: the
+    operations of the update are single IEEE operations, so the CPU gives the same bits; nothing else is written"""
+    import zenu_oracle as zo
+    r = np.random.default_rng(3)
+    sizes = [1, 2, 3, 4, 5, 511, 512, 513, 1021, 1023, 1024, 1025, 1027, 2049, largest] * 5
+    params, state, expect = {}, {"m": {}, "v": {}}, {}
+    keep = []
+    for i, n in enumerate(sizes):
+        host = [r.standard_normal(n).astype(dtype) * s for s in (1, 0.1, 0.01)] + [np.square(r.standard_normal(n)).astype(dtype)]
+        host = [np.ascontiguousarray(h, dtype) for h in host]
+        dev = []
+        for j, h in enumerate(host):
+            m = hip.Matrix.from_numpy(np.concatenate([np.full(i % 4 if j else (i + 1) % 4, 7, dtype), h, np.full(3, 7, dtype)]))
+            dev.append(hip.Matrix(m.buf, m.shape[0] - n - 3, (n,), (1,), dtype))
+            keep.append((m, dev[-1]))
+        name = f"t{i}.weight" if i % 2 else f"t{i}.bias"
+        params[name] = (dev[0], dev[1])
+        state["m"][name], state["v"][name] = dev[2], dev[3]
+        p, g, m, v = (h.copy() for h in host)
+        zo.adamw_update(p, g, m, v, 1e-2, 0.9, 0.999, 1e-8, 0.01, i % 2, 4)
+        expect[name] = (p, m, v)
+    opt = hip.AdamW(1e-2, 0.9, 0.999, 1e-8, 0.01, {}, [k for k in params if k.endswith("weight")])
+    opt.m, opt.v, opt.step = state["m"], state["v"], 3
+    opt.update(params)
+    for name, (p, m, v) in expect.items():
+        same(params[name][0].to_numpy(), p, (name, p.size, "parameter"))
+        same(state["m"][name].to_numpy(), m, (name, p.size, "first moment"))
+        same(state["v"][name].to_numpy(), v, (name, p.size, "second moment"))
+    for whole, part in keep:
+        around = np.delete(whole.to_numpy(), np.arange(part.offset, part.offset + part.shape[0]))
+        assert np.all(around == 7)
+    before = {k: p.to_numpy() for k, (p, _) in params.items()}
+    hip.SGD(0.3).update(params)
+    for name, (p, g) in params.items():
+        same(p.to_numpy(), before[name] - g.to_numpy() * dtype(0.3), (name, "sgd"))
