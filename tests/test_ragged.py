@@ -1,6 +1,8 @@
 """Sizes and alignments that are nobody's choice: rows of odd length, views that start in the middle of a
 vector, edge tiles one element wide.  The elementwise results are IEEE operations on the same operands, so
 numpy gives the same bits."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -126,3 +128,53 @@ def test_optimizer_tensors_of_any_size_and_alignment(hip, dtype, largest):
     hip.SGD(0.3).update(params)
     for name, (p, g) in params.items():
         same(p.to_numpy(), before[name] - g.to_numpy() * dtype(0.3), (name, "sgd"))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", [(5, 1), (9, 3), (3, 16), (70, 17), (33, 31), (600, 129), (40, 1003), (2049, 127), (3, 8195),
+                                   (1, 300001), (9000, 1021)], ids=str)
+def test_reductions_at_any_alignment(hip, dtype, shape):
+    """Sums, magnitudes, maxima and their first positions along both axes, rows starting anywhere in a vector, the
+    source a whole tensor and a column slice of a wider one.  n terms added in any order are off by less than
+    (n - 1) eps of the sum of their magnitudes."""
+    rows, cols = shape
+    r = np.random.default_rng(cols)
+    eps = np.finfo(dtype).eps
+    wide = r.standard_normal((rows, cols + 3)).astype(dtype)
+    for a in (wide[:, :cols], wide[:, 2:cols + 2]):
+        a = np.ascontiguousarray(a)
+        if cols > 2:
+            a[::3, cols - 1] = a[::3].max(axis=1)          # the maximum twice, the second time at the end
+            a[1::4, 1] = np.nan                            # not in position 0: the scan passes over it
+        clean = np.nan_to_num(a, nan=0.0)
+        whole = offset_matrix(hip, a, 1)
+        big = hip.Matrix.from_numpy(np.concatenate([np.full((rows, 3), 9, dtype), a, np.full((rows, 2), 9, dtype)], axis=1))
+        part = big.slice(slice(None), slice(3, 3 + cols))
+        for name, m in (("whole", whole), ("slice", part)):
+            what = (shape, name)
+            for axis, n in ((0, rows), (1, cols)):
+                at = hip.Matrix.alloc((a.size // n,), np.float64)
+                top = offset_matrix(hip, np.zeros(a.size // n, dtype), 1)
+                code = hip._lib.F32 if dtype == np.float32 else hip._lib.F64
+                hip._lib.check(hip.lib().zenu_hip_max_axis_idx(code, at.as_ptr(), C.byref(m.desc()), axis, None), "max_axis_idx")
+                hip._lib.check(hip.lib().zenu_hip_max_axis(code, C.byref(top.desc()), C.byref(m.desc()), axis, None), "max_axis")
+                # a NaN in position 0 stays; elsewhere it never replaces
+                scan = np.where(np.isnan(a), -np.inf, a)
+                first = np.isnan(np.take(a, 0, axis=axis))
+                want = np.where(first, 0, np.argmax(scan, axis=axis))
+                assert np.array_equal(at.to_numpy().view(np.int64), want), what
+                picked = np.take_along_axis(a, np.expand_dims(want, axis), axis).reshape(-1)
+                assert np.array_equal(top.to_numpy(), picked, equal_nan=True), what
+        for name, m in (("whole", offset_matrix(hip, clean, 3)),):
+            for axis, n in ((0, rows), (1, cols)):
+                kept = (1, cols) if axis == 0 else (rows, 1)
+                out = offset_matrix(hip, np.zeros(kept, dtype), 1)
+                hip.sum_to(m, out)
+                exact = clean.sum(axis=axis, keepdims=True, dtype=np.longdouble)
+                bound = n * eps * np.abs(clean).sum(axis=axis, keepdims=True, dtype=np.longdouble)
+                assert np.all(np.abs(out.to_numpy() - exact) <= bound), (shape, axis)
+            total = hip.Matrix.alloc((1,), dtype)
+            hip._lib.check(hip.lib().zenu_hip_asum(hip._lib.F32 if dtype == np.float32 else hip._lib.F64, total.as_ptr(),
+                                                   C.byref(m.desc()), None), "asum")
+            exact = np.abs(clean).sum(dtype=np.longdouble)
+            assert abs(total.to_numpy()[0] - exact) <= clean.size * eps * exact, shape

@@ -152,6 +152,7 @@ template <typename T> struct SumTr {
     typedef T Acc;
     static constexpr bool kHasIdx = false;
     __device__ __forceinline__ static Acc identity() { return (T)0; }
+    __device__ __forceinline__ static T pad() { return (T)0; }      // an element that update() takes without effect
     __device__ __forceinline__ static Acc update(Acc a, T x, int64_t) { return a + x; }
     __device__ __forceinline__ static Acc first(Acc a, T) { return a; }
     __device__ __forceinline__ static Acc from_partial(T x, int64_t) { return x; }
@@ -195,6 +196,7 @@ template <typename T> struct ArgmaxTr {
         a.idx = gt ? (int32_t)pos : a.idx;
         return a;
     }
+    __device__ __forceinline__ static T pad() { return -(T)INFINITY; }
     // `x` is the element at position 0 of the reduced axis, already folded in by update()
     __device__ __forceinline__ static Acc first(Acc a, T x)
     {
@@ -493,14 +495,24 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(RedParams<T> p)
 #pragma unroll
                             for (int j = 0; j < VEC; j++) acc[u] = Tr::update(acc[u], x[u].v[j], r + u * step + j);
                         }
-                    } else {                   // the last, partial chunk of the row
-                        for (; r + VEC <= R; r += step) {
-                            Pack<T, VEC> x = load_pack<T, VEC, false>(row + r);
+                    } else {
+                        // the last, partial chunk of the row: a vector that would run past the end is moved back to
+                        // end with the row and the elements that others own are masked, so that the loads stay
+                        // vectors in flight together (R >= VEC)
+                        Pack<T, VEC> x[U];
 #pragma unroll
-                            for (int j = 0; j < VEC; j++) acc[0] = Tr::update(acc[0], x.v[j], r + j);
+                        for (int u = 0; u < U; u++) {
+                            const int64_t ru = r + u * step;
+                            x[u] = load_pack<T, VEC, false>(row + (ru + VEC <= R ? ru : R - VEC));
                         }
-                        if (r < R)             // ragged end (R % VEC != 0): one lane
-                            for (int j = 0; r + j < R; j++) acc[0] = Tr::update(acc[0], row[r + j], r + j);
+#pragma unroll
+                        for (int u = 0; u < U; u++) {
+                            const int64_t ru = r + u * step;
+                            const int64_t at = ru + VEC <= R ? ru : R - VEC;
+                            if (b + u * step >= R) break;         // uniform
+#pragma unroll
+                            for (int j = 0; j < VEC; j++) acc[u] = Tr::update(acc[u], at + j >= ru ? x[u].v[j] : Tr::pad(), at + j);
+                        }
                     }
                 }
                 if (split == 0 && lane == 0) acc[0] = Tr::first(acc[0], row[0]);
@@ -651,9 +663,12 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
     const int split = (int)split_u;
     const int64_t q = q_u;
     const int64_t group = q * col_tiles + ct;   // the workgroups that share these outputs
-    const int64_t c = ((int64_t)ct * tx_n + tx) * VEC;
-
-    const int ncol = (c + VEC <= p.inner) ? VEC : (c < p.inner ? (int)(p.inner - c) : 0);
+    // A thread whose vector would run past the end of the row takes the row's last VEC columns instead; those that
+    // its neighbour has as well come to the same bits and are written twice.  (With PRE inner % VEC == 0: no element
+    // of pre_out has two writers.)
+    const int64_t c0 = ((int64_t)ct * tx_n + tx) * VEC;
+    const int64_t c = c0 + VEC <= p.inner ? c0 : p.inner - VEC;
+    const int ncol = c0 < p.inner ? VEC : 0;
     const T *src = p.in + q * p.outer_stride + c;
     constexpr int U = 4;
     const int64_t R = p.R;
@@ -701,7 +716,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
         // the source top to bottom together
         const int64_t chunk = U * ty_n;
         const int64_t row_step = (int64_t)ty_n * p.elem_stride;
-        if (ncol == VEC && VEC > 1) {
+        if (ncol == VEC) {
             const T *ptr = src + ((int64_t)split * chunk + ty) * p.elem_stride;
             const int64_t ptr_step = (int64_t)p.splits * chunk * p.elem_stride;
             for (int64_t b = split * chunk; b < R; b += p.splits * chunk, ptr += ptr_step) {
@@ -724,10 +739,6 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
                     }
                 }
             }
-        } else if (ncol > 0) {
-            for (int64_t b = split * chunk; b < R; b += p.splits * chunk)
-                for (int64_t r = b + ty; r < R && r < b + chunk; r += ty_n)
-                    ZENU_FOR_COLS(j) acc[j] = Tr::update(acc[j], src[r * p.elem_stride + j], r);
         }
         if (split == 0 && ty == 0)
             ZENU_FOR_COLS(j) acc[j] = Tr::first(acc[j], src[j]);
@@ -894,7 +905,8 @@ template <typename T, typename Tr>
 int launch_rows(const RedParams<T> &p, hipStream_t s)
 {
     constexpr int VEC = VecOf<T>::N;
-    const bool vec = p.elem_stride == 1 && p.inner == 1 && aligned16(p.in) && p.outer_stride % VEC == 0;
+    // vectors whatever the alignment of the rows; [10007,1003] f64 row sums take 13.6 us (80 MB) as with scalar loads
+    const bool vec = p.elem_stride == 1 && p.inner == 1 && p.R >= VEC;
     const bool nt = vec && stream_source(p);
     const bool wave_row = p.splits == 1 && p.R <= 1024;
     if (wave_row) {
@@ -933,21 +945,14 @@ inline int cols_tx_shift(int64_t inner, int v)
     return shift;
 }
 
-template <typename T> inline bool cols_vec_ok(const RedParams<T> &p)
-{
-    constexpr int VEC = VecOf<T>::N;
-    return aligned16(p.in) && p.inner % VEC == 0 && p.outer_stride % VEC == 0 && p.elem_stride % VEC == 0;
-}
-
 template <typename T, typename Tr>
 int launch_cols(const RedParams<T> &p, hipStream_t s)
 {
     constexpr int VEC = VecOf<T>::N;
-    const bool vec = cols_vec_ok(p);
-    const bool nt = vec && stream_source(p);
-    const int v = vec ? VEC : 1;
+    // (vectors whatever the alignment: column sums of [10007,1003] f64 19.6 us (80 MB), 32.3 with scalar loads)
+    const bool nt = stream_source(p);
     const int shift = p.cols_shift;
-    const int64_t per_tile = ((int64_t)1 << shift) * v;
+    const int64_t per_tile = ((int64_t)1 << shift) * VEC;
     const int64_t col_tiles = (p.inner + per_tile - 1) / per_tile;
     const int64_t outer = p.nout / p.inner;
     int64_t grid = outer * col_tiles * p.splits;
@@ -956,11 +961,9 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
     const dim3 g = g3 ? dim3((unsigned)col_tiles, (unsigned)p.splits, (unsigned)outer) : dim3((unsigned)grid);
     const uint32_t ctl = (uint32_t)col_tiles;
     // the regular geometry: full vector tiles of 32 x 8 threads, a split axis with a flat counter
-    const bool regular = vec && g3 && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits &&
-                         p.cstride == 1 && (Tr::kHasIdx || aligned16(p.out_val));
+    const bool regular = g3 && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
     if constexpr (!Tr::kHasIdx && std::is_same<Tr, SumTr<T>>::value) {
-        if (p.pre_x) {   // the transform rides on the vector paths only (the caller has checked the layout)
-            if (!vec) return ZENU_ERR_UNSUPPORTED;
+        if (p.pre_x) {   // (the caller has checked that a row is a whole number of vectors)
             if (regular) {
                 if (nt) reduce_cols_regular_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p);
                 else    reduce_cols_regular_kernel<T, Tr, VEC, false, true><<<g, kBlock, 0, s>>>(p);
@@ -978,9 +981,8 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
         ZENU_LAUNCH_CHECK();
         return ZENU_OK;
     }
-    if (nt)       reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-    else if (vec) reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-    else          reduce_cols_kernel<T, Tr, 1, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    if (nt) reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    else    reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
     ZENU_LAUNCH_CHECK();
     return ZENU_OK;
 }
@@ -1033,19 +1035,18 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
     p.g_elem_stride = elem_stride;
 
     const bool use_cols = inner >= 16;
-    if (pre_x && (!use_cols || !cols_vec_ok(p))) return ZENU_ERR_UNSUPPORTED;   // the caller falls back to two launches
+    if (pre_x && (!use_cols || inner % VEC)) return ZENU_ERR_UNSUPPORTED;   // the caller falls back to two launches
     int64_t splits = 1, groups = nout;
     p.cols_shift = 0;
     if (use_cols) {
-        const int v = cols_vec_ok(p) ? VEC : 1;
-        int shift = cols_tx_shift(inner, v);
-        auto tiles_at = [&](int sh) { return (inner + (((int64_t)1 << sh) * v) - 1) / (((int64_t)1 << sh) * v); };
+        int shift = cols_tx_shift(inner, VEC);
+        auto tiles_at = [&](int sh) { return (inner + (((int64_t)1 << sh) * VEC) - 1) / (((int64_t)1 << sh) * VEC); };
         // A small source with a short reduced axis is bound by latencies, and the hand-off of a split
         // (about 3 us) is the longest of them: narrower column tiles (down to 64-byte row pieces, which
         // stream at less than half the rate, but there is little to stream) give more workgroups
         // without one.  Column sums of [256,512] f32 with the ReLU-gradient transform: 7.7 us as
         // 4 tiles x 4 splits, 5.8 us as 16 tiles of 32 columns, 5.0 us as 32 tiles of 16 columns.
-        if (v > 1 && R <= kSmallColsRows && outer * R * inner * (int64_t)sizeof(T) <= kSmallColsBytes)
+        if (R <= kSmallColsRows && outer * R * inner * (int64_t)sizeof(T) <= kSmallColsBytes)
             while (shift > 2 && outer * tiles_at(shift) < target_blocks) shift--;
         p.cols_shift = shift;
         const int64_t col_tiles = tiles_at(shift);
