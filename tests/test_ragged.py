@@ -178,3 +178,39 @@ def test_reductions_at_any_alignment(hip, dtype, shape):
                                                    C.byref(m.desc()), None), "asum")
             exact = np.abs(clean).sum(dtype=np.longdouble)
             assert abs(total.to_numpy()[0] - exact) <= clean.size * eps * exact, shape
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", [(3, 1), (5, 3), (4, 256), (7, 1500), (33, 1027), (9000, 999), (8200, 1024)], ids=str)
+@pytest.mark.parametrize("with_pre", [True, False])
+def test_bias_relu_at_any_alignment(hip, dtype, shape, with_pre):
+    r = np.random.default_rng(shape[1])
+    z, bias = r.standard_normal(shape).astype(dtype), r.standard_normal(shape[1]).astype(dtype)
+    act, pre = offset_matrix(hip, np.zeros(shape, dtype), 3), offset_matrix(hip, np.zeros(shape, dtype), 2)
+    act.bias_add_relu(offset_matrix(hip, z, 1), offset_matrix(hip, bias, 1), 0.25, pre=pre if with_pre else None)
+    a = z + bias
+    if with_pre:
+        same(pre.to_numpy(), a, ("pre", shape))
+    same(act.to_numpy(), np.where(a > 0, a, dtype(0.25) * a), ("act", shape))
+
+
+# the kept run in front, in the middle and at the end; pieces shorter than a vector, of one vector, longer than a
+# workgroup; more channels than workgroups wanted, fewer, and so few that the axes go one after the other
+SUMS = [((2, 3, 5, 7), (1, 3, 1, 1)), ((64, 5, 2, 1), (1, 5, 1, 1)), ((6, 4, 3, 1), (1, 4, 1, 1)), ((9, 16, 2, 2), (1, 16, 1, 1)),
+        ((64, 33, 14, 14), (1, 33, 1, 1)), ((130, 3, 65, 67), (1, 3, 1, 1)), ((2, 2, 80, 81), (1, 2, 1, 1)), ((1, 40, 9, 11), (1, 40, 1, 1)),
+        ((3, 600, 7, 7), (1, 600, 1, 1)), ((20, 70, 90, 91), (1, 70, 1, 1)), ((4, 5, 6, 37), (37,)), ((4, 5, 6, 37), (6, 37)), ((7, 3, 5), ()),
+        ((3, 4, 5, 6), (1, 4, 1, 6)), ((3, 4, 5, 6), (3, 1, 1, 6))]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape,kept", SUMS, ids=str)
+def test_sums_over_several_axes(hip, dtype, shape, kept):
+    """n terms added in any order are off by less than (n - 1) eps of the sum of their magnitudes"""
+    x = np.random.default_rng(len(kept)).standard_normal(shape).astype(dtype)
+    out = offset_matrix(hip, np.full(kept, 5, dtype), 1)
+    hip.sum_to(offset_matrix(hip, x, 1), out)
+    axes = tuple(i for i in range(len(shape)) if i < len(shape) - len(kept) or (len(kept) == len(shape) and kept[i] != shape[i]))
+    wide = x.astype(np.longdouble)
+    exact, scale = wide.sum(axis=axes).reshape(kept), np.abs(wide).sum(axis=axes).reshape(kept)
+    n = x.size // max(exact.size, 1)
+    assert np.all(np.abs(out.to_numpy() - exact) <= n * np.finfo(dtype).eps * scale)

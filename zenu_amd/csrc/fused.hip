@@ -741,32 +741,51 @@ __global__ __launch_bounds__(kHeadBlock) void ce_head_backward_kernel(const T *y
 // ---- bias add + ReLU ----------------------------------------------------------------------------------------
 // pre = z + bias (broadcast over rows), act = pre > 0 ? pre : alpha * pre  (relu.rs:44-48)
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(kBlock) void bias_relu_kernel(const T *z, const T *bias, T *pre, T *act,
-                                                            int64_t rows, int64_t packs_per_row, T alpha)
+// Any row length, any alignment: the tensor as one run of vectors, one per lane of a 64-thread workgroup; a vector
+// that spans two rows gathers its bias.  [1000,1500] f32 4.85 us (18 MB), 5.2 with a 64-bit division per vector
+// in a grid-stride loop.
+constexpr int kTileLanes = 64;
+template <typename T, int VEC, bool NT, typename Index>
+__global__ __launch_bounds__(kTileLanes) void bias_relu_kernel(const T *z, const T *bias, T *pre, T *act, Index n,
+                                                               Index F, T alpha)
 {
-    const int64_t total = rows * packs_per_row;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total; i += (int64_t)gridDim.x * kBlock) {
-        const int64_t row = i / packs_per_row;
-        const int64_t col = (i - row * packs_per_row) * VEC;
-        const int64_t off = i * VEC;
-        const Pack<T, VEC> v = load_pack<T, VEC, false>(z + off);
-        const Pack<T, VEC> b = load_pack<T, VEC, false>(bias + col);
+    const Index off = ((Index)blockIdx.x * kTileLanes + threadIdx.x) * VEC;
+    const Index col = off % F;
+    if (off + VEC <= n) {
+        const Pack<T, VEC> v = load_pack<T, VEC, NT>(z + off);
+        Pack<T, VEC> b;
+        if (col + VEC <= F) {
+            b = load_pack<T, VEC, false>(bias + col);
+        } else {
+            Index c = col;
+#pragma unroll
+            for (int j = 0; j < VEC; j++) {
+                b.v[j] = bias[c];
+                c = c + 1 == F ? 0 : c + 1;
+            }
+        }
         Pack<T, VEC> a, h;
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
             a.v[j] = v.v[j] + b.v[j];
             h.v[j] = a.v[j] > (T)0 ? a.v[j] : alpha * a.v[j];
         }
-        if (pre) store_pack<T, VEC, false>(pre + off, a);
-        store_pack<T, VEC, false>(act + off, h);
+        if (pre) store_pack<T, VEC, NT>(pre + off, a);
+        store_pack<T, VEC, NT>(act + off, h);
+    } else {
+        Index c = col;
+        for (Index i = off; i < n; i++) {
+            const T a = z[i] + bias[c];
+            if (pre) pre[i] = a;
+            act[i] = a > (T)0 ? a : alpha * a;
+            c = c + 1 == F ? 0 : c + 1;
+        }
     }
 }
 
 // Rows that are a whole number of 64-lane vectors: a 64-thread workgroup per contiguous piece of a
 // row, one vector per lane (the shape that streams best when most of the traffic is stores); the
 // row / column split is one 32-bit division per workgroup on the scalar unit.
-constexpr int kTileLanes = 64;
 template <typename T, int VEC, bool NT>
 __global__ __launch_bounds__(kTileLanes) void bias_relu_tile_kernel(const T *z, const T *bias, T *pre, T *act,
                                                                      uint32_t tiles_per_row, T alpha)
@@ -1108,26 +1127,23 @@ int bias_relu_t(int dtype, const zenu_tensor_t *pre, const zenu_tensor_t &act, c
     ContigOut<T> pout(pre ? *pre : act, dtype, s);
     if (pre && pout.status) return pout.status;
     T *pp = pre ? pout.ptr : nullptr;
-    const int64_t rows = n / F;
-    const bool vec = F % VEC == 0 && aligned16(zin.ptr) && aligned16(bin.ptr) && aligned16(aout.ptr) &&
-                     (!pp || aligned16(pp));
-    const int64_t packs = vec ? F / VEC : F;
-    if (vec && packs % kTileLanes == 0 && rows * (packs / kTileLanes) <= 0x7fffffffLL) {
+    const bool nt = n * (int64_t)sizeof(T) * (pp ? 3 : 2) >= kStreamBytes;
+    const int64_t packs = F / VEC;
+    const T al = (T)alpha;
+    const int64_t grid = (n + kTileLanes * VEC - 1) / (kTileLanes * VEC);
+    if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
+    const unsigned g = (unsigned)grid;
+    if (F % (VEC * kTileLanes) == 0) {
         const uint32_t tiles = (uint32_t)(packs / kTileLanes);
-        const unsigned grid = (unsigned)(rows * tiles);
-        const bool nt = n * (int64_t)sizeof(T) * (pp ? 3 : 2) >= kStreamBytes;
-        if (nt) bias_relu_tile_kernel<T, VEC, true><<<grid, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, tiles, (T)alpha);
-        else    bias_relu_tile_kernel<T, VEC, false><<<grid, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, tiles, (T)alpha);
-        ZENU_LAUNCH_CHECK();
-        int rc2 = aout.finish();
-        if (!rc2 && pre) rc2 = pout.finish();
-        return rc2;
+        if (nt) bias_relu_tile_kernel<T, VEC, true><<<g, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, tiles, al);
+        else    bias_relu_tile_kernel<T, VEC, false><<<g, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, tiles, al);
+    } else if (n < ((int64_t)1 << 32) - 65536) {
+        const uint32_t n32 = (uint32_t)n, f32 = (uint32_t)F;
+        if (nt) bias_relu_kernel<T, VEC, true, uint32_t><<<g, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, n32, f32, al);
+        else    bias_relu_kernel<T, VEC, false, uint32_t><<<g, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, n32, f32, al);
+    } else {
+        bias_relu_kernel<T, VEC, true, uint64_t><<<g, kTileLanes, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, (uint64_t)n, (uint64_t)F, al);
     }
-    int64_t blocks = (rows * packs + kBlock - 1) / kBlock;
-    const int64_t cap = (int64_t)device_info().num_cus * 16;
-    if (blocks > cap) blocks = cap;
-    if (vec) bias_relu_kernel<T, VEC><<<(unsigned)blocks, kBlock, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, rows, packs, (T)alpha);
-    else     bias_relu_kernel<T, 1><<<(unsigned)blocks, kBlock, 0, s>>>(zin.ptr, bin.ptr, pp, aout.ptr, rows, packs, (T)alpha);
     ZENU_LAUNCH_CHECK();
     int rc = aout.finish();
     if (!rc && pre) rc = pout.finish();

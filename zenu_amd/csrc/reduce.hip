@@ -893,6 +893,55 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
     if (threadIdx.x == 0) store_agent(p.counters + group, 0);
 }
 
+// ---- kernel C: pieces -----------------------------------------------------------------------------------------
+// Source [N, C, I], contiguous, reduced over N and I: the sum of channel c, split s, is that of the pieces
+// src[n, c, :] for n = s, s + splits, ...  The pieces of a workgroup are walked as one run of vectors, four in flight
+// per thread, so that short pieces (a 7 x 7 image plane) keep every lane busy; the last vector of a piece is moved
+// back to end with it and masked.  Read once, in one launch when the channels fill the chip: the bias gradient of a
+// convolution's [64,512,14,14] f32 output (26 MB) 7.0 us; summed over one axis after the other, through two
+// workspaces, 12.4 us and three launches.
+template <typename T, int VEC, bool NT>
+__global__ __launch_bounds__(kBlock) void reduce_pieces_kernel(const T *src, T *out, uint32_t N, uint32_t C, int64_t I,
+                                                               uint32_t splits, uint32_t vecs)
+{
+    typedef SumTr<T> Tr;
+    constexpr int U = 4;
+    const uint32_t c = blockIdx.x / splits, split = blockIdx.x - c * splits;
+    const uint32_t pieces = (N - split + splits - 1) / splits;
+    const int64_t piece_step = (int64_t)splits * C * I;
+    const T *const base = src + ((int64_t)split * C + c) * I;
+    T acc[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) acc[u] = (T)0;
+    // position (piece, vector) of this thread; moving on by kBlock vectors needs no further division
+    const uint32_t jump = kBlock / vecs, rest = kBlock - jump * vecs;
+    uint32_t n = threadIdx.x / vecs, v = threadIdx.x - n * vecs;
+    while (n < pieces) {
+        Pack<T, VEC> x[U];
+        int skip[U];             // leading elements of the vector that belong to the one before; VEC: none of it counts
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t i = (int64_t)v * VEC;
+            const int64_t at = i + VEC <= I ? i : I - VEC;
+            skip[u] = n < pieces ? (int)(i - at) : VEC;
+            x[u] = load_pack<T, VEC, NT>(n < pieces ? base + n * piece_step + at : base);
+            n += jump;
+            v += rest;
+            if (v >= vecs) {
+                v -= vecs;
+                n++;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) acc[u] = acc[u] + (j >= skip[u] ? x[u].v[j] : (T)0);
+        }
+    }
+    const T total = block_allreduce<Tr>((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if (threadIdx.x == 0) out[blockIdx.x] = total;
+}
+
 // ---- host side ---------------------------------------------------------------------------------------------
 
 // the source is read once; when it is larger than the caches the loads carry the streaming hint
@@ -1170,6 +1219,34 @@ bool reduced_shape_ok(const zenu_tensor_t &out, const zenu_tensor_t &src, int ax
         return true;
     }
     return false;
+}
+
+// sum over N and I of a contiguous [N, C, I] source; ZENU_ERR_UNSUPPORTED where the geometry does not fit the kernel
+template <typename T>
+int sum_pieces(const T *src, int64_t N, int64_t C, int64_t I, T *out, hipStream_t s)
+{
+    constexpr int VEC = VecOf<T>::N;
+    if (N == 1) return reduce_contiguous<T, SumTr<T>>(src, C, I, 1, out, nullptr, s);
+    if (I == 1) return reduce_contiguous<T, SumTr<T>>(src, 1, N, C, out, nullptr, s);
+    const int64_t vecs = (I + VEC - 1) / VEC;
+    if (I < VEC || N >= (1 << 30) || C >= (1 << 30) || vecs >= (1 << 30)) return ZENU_ERR_UNSUPPORTED;
+    // two workgroups per CU, none with less than four vectors per thread; at most one per piece, and where those
+    // leave CUs idle over long pieces the axes are summed one after the other
+    const int64_t want = (2 * (int64_t)device_info().num_cus + C - 1) / C;
+    const int64_t most = (N * vecs + 4 * kBlock - 1) / (4 * kBlock);
+    int64_t splits = want < most ? want : most;
+    if (splits > N) splits = N;
+    if (C * splits < device_info().num_cus && splits == N && vecs > 4 * kBlock) return ZENU_ERR_UNSUPPORTED;
+    if (C * splits > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
+    Workspace ws(splits > 1 ? (size_t)(C * splits) * sizeof(T) : 0, s);
+    if (ws.status) return ws.status;
+    T *const part = splits > 1 ? static_cast<T *>(ws.ptr) : out;
+    const bool nt = N * C * I * (int64_t)sizeof(T) >= kStreamBytes;
+    const unsigned grid = (unsigned)(C * splits);
+    if (nt) reduce_pieces_kernel<T, VEC, true><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs);
+    else    reduce_pieces_kernel<T, VEC, false><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs);
+    ZENU_LAUNCH_CHECK();
+    return splits > 1 ? reduce_contiguous<T, SumTr<T>>(part, C, splits, 1, out, nullptr, s) : ZENU_OK;
 }
 
 enum RedKind { kSum, kAsum, kMax };
@@ -1535,6 +1612,30 @@ int zenu_hip_sum_to(int dtype, const zenu_tensor_t *target, const zenu_tensor_t 
         for (int i = 0; i < target->ndim; i++)
             if (src->shape[diff + i] != target->shape[i]) return ZENU_ERR_SHAPE;
         for (int i = 0; i < diff; i++) { axes[na] = 0; keep[na] = 0; na++; }
+    }
+
+    // Two or more axes of a contiguous source that leave one run of kept dims in the middle, [N, C, I]: in one go.
+    // (A target inside the source is written by the last of several launches only, as below.)
+    if (na >= 2 && num_elm(*src) > 0 && is_default_stride_strict(*src) && is_default_stride_strict(*target) &&
+        !view_overlaps(*src, esz, target->ptr, (size_t)num_elm(*target) * esz)) {
+        bool reduced[kMaxDim] = {};
+        for (int a = 0; a < na; a++) reduced[diff ? a : axes[a]] = true;
+        int64_t part[3] = {1, 1, 1};      // N, C, I
+        int at = 0;
+        for (int i = 0; i < src->ndim && at < 3; i++) {
+            if (src->shape[i] == 1) continue;
+            if (at == 0 && !reduced[i]) at = 1;
+            else if (at == 1 && reduced[i]) at = 2;
+            else if (at == 2 && !reduced[i]) at = 3;       // a second kept run
+            if (at < 3) part[at] *= src->shape[i];
+        }
+        if (at < 3) {
+            rc = dtype == ZENU_F32 ? sum_pieces<float>(static_cast<const float *>(src->ptr), part[0], part[1], part[2],
+                                                       static_cast<float *>(target->ptr), s)
+                                   : sum_pieces<double>(static_cast<const double *>(src->ptr), part[0], part[1], part[2],
+                                                        static_cast<double *>(target->ptr), s);
+            if (rc != ZENU_ERR_UNSUPPORTED) return rc;
+        }
     }
 
     zenu_tensor_t cur = *src;
