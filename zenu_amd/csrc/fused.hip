@@ -57,6 +57,35 @@ template <typename T, bool MAX, int BLOCK = kBlock> __device__ __forceinline__ T
 constexpr int kLineRegs = 16;   // classes of the one-workgroup classifier head kernels below
 constexpr int kLineWaves = 16;  // wavefronts that can share the lines of a workgroup
 
+// Every quotient of a softmax line has the same divisor.  With r = RN(1 / sum): q0 = RN(a r), the
+// exact remainder a - sum q0 (one fma) and q = fma(remainder, r, q0) is the correctly rounded
+// a / sum (Markstein) unless the divisor's mantissa is all ones, as long as nothing underflows:
+// three instructions per element instead of the division's eleven.  A thread takes that road
+// when its terms are zero (the quotient is, too) or at least 2^-64 and the sum lies in [1, 2^23) (quotient
+// and remainder stay normal); otherwise it divides.  On 9.6e9 random pairs from those ranges (terms down to
+// 2^-80) the host finds no quotient that differs from the division's.  f32 only.
+// least: the smallest of the thread's terms above zero, as its bits less one (all ones before the first)
+template <typename T> __device__ __forceinline__ uint32_t least_term(uint32_t least, T a)
+{
+    if constexpr (sizeof(T) == 4) return min(least, __float_as_uint(a) - 1u);
+    return least;
+}
+template <typename T> __device__ __forceinline__ bool divides_by_reciprocal(uint32_t least, T sum)
+{
+    if constexpr (sizeof(T) == 4)
+        return least >= __float_as_uint(0x1p-64f) - 1u && sum >= (T)1 && sum < (T)0x1p23f &&
+               (__float_as_uint(sum) & 0x7fffffu) != 0x7fffffu;
+    return false;
+}
+template <typename T> __device__ __forceinline__ T quotient(T a, T sum, T rcp)
+{
+    if constexpr (sizeof(T) == 4) {
+        const float q0 = a * rcp;
+        return __builtin_fmaf(__builtin_fmaf(-sum, q0, a), rcp, q0);
+    }
+    return a / sum;
+}
+
 // Where a wavefront of the two lines kernels stands: a workgroup has `waves` wavefronts along R for every 64
 // lines, wavefront w of them holds elements [w OWN, (w + 1) OWN) of each of its lines in registers.
 struct LineSpot {
@@ -104,8 +133,8 @@ __device__ __forceinline__ T sum_in_order(const T (&x)[OWN], int valid, const Li
 // The softmax axis is not the last one, or is short: a lane per line, and as many wavefronts along the line as it
 // takes to hold it in registers, so that it is read and written once with all its loads in flight together.  The
 // sums run over the line in index order exactly as sum.rs:20-25 adds (they are handed from wavefront to wavefront).
-// Bound by the passes over memory: [16,21,16384] f32 (22 MB each way, cached) 17.0 us, 26.1 when one thread
-// walked a line three times, one load in flight; its backward pass 11.9 us, 20.5.
+// Bound by the passes over memory: [16,21,16384] f32 (22 MB each way, cached) 14.9 us, 26.1 when one thread
+// walked a line three times, one load in flight; its backward pass 11.1 us, 20.5.
 // With `loss` set (cross-entropy, every line in this one workgroup) the kernel also folds the row
 // terms and divides by -N, in the order of ce_finalize_kernel: the whole loss in one launch.
 template <typename T, bool CE, int OWN>
@@ -143,18 +172,28 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T 
         __syncthreads();
     }
     m = combine<T, true>(x0, m);
-#pragma unroll
-    for (int i = 0; i < OWN; i++)
-        if (i < valid) v[i] = ml.exp(v[i] - m);
-    const T sum = sum_in_order<T, OWN>(v, valid, at, waves, shared);
+    uint32_t least = ~0u;
 #pragma unroll
     for (int i = 0; i < OWN; i++) {
         if (i < valid) {
-            const T s = v[i] / sum;
-            if (at.active) yl[i * inner] = s;
-            if constexpr (CE) v[i] = target[at.base + r0 + i] * ml.log(s);
+            v[i] = ml.exp_flat(v[i] - m);
+            least = least_term<T>(least, v[i]);
         }
     }
+    const T sum = sum_in_order<T, OWN>(v, valid, at, waves, shared);
+    auto finish = [&](auto by_reciprocal) {
+        const T rcp = decltype(by_reciprocal)::value ? (T)1 / sum : (T)0;
+#pragma unroll
+        for (int i = 0; i < OWN; i++) {
+            if (i < valid) {
+                const T s = decltype(by_reciprocal)::value ? quotient<T>(v[i], sum, rcp) : v[i] / sum;
+                if (at.active) yl[i * inner] = s;
+                if constexpr (CE) v[i] = target[at.base + r0 + i] * ml.log(s);
+            }
+        }
+    };
+    if (divides_by_reciprocal<T>(least, sum)) finish(std::true_type());
+    else finish(std::false_type());
     if constexpr (CE) {
         if (waves > 1) __syncthreads();        // the sum of the exponentials has been read
         const T term = sum_in_order<T, OWN>(v, valid, at, waves, shared);
@@ -344,7 +383,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
             for (int j = 0; j < VEC; j++) {      // an element that is not the slot's own is exp(-inf), zero
                 v[k].v[j] = ml.exp_flat(v[k].v[j] - m);
                 sum = sum + v[k].v[j];
-                if constexpr (sizeof(T) == 4) least = min(least, __float_as_uint(v[k].v[j]) - 1u);
+                least = least_term<T>(least, v[k].v[j]);
             }
         }
     }
@@ -361,17 +400,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
         });
     }
     sum = block_red<T, false, LANES>(sum, lds);
-    // Every quotient of the row has the same divisor.  With r = RN(1 / sum): q0 = RN(a r), the
-    // exact remainder a - sum q0 (one fma) and q = fma(remainder, r, q0) is the correctly rounded
-    // a / sum (Markstein) unless the divisor's mantissa is all ones, as long as nothing underflows:
-    // three instructions per element instead of the division's eleven.  The thread takes that road
-    // when its terms are zero (the quotient is, too) or at least 2^-64 and the sum lies in [1, 2^23) (quotient
-    // and remainder stay normal); otherwise it divides.  On 9.6e9 random pairs from those ranges (terms down to
-    // 2^-80) the host finds no quotient that differs from the division's.
-    bool shared_divisor = false;
-    if constexpr (sizeof(T) == 4)
-        shared_divisor = least >= __float_as_uint(0x1p-64f) - 1u && sum >= (T)1 && sum < (T)0x1p23f &&
-                         (__float_as_uint(sum) & 0x7fffffu) != 0x7fffffu;
+    const bool shared_divisor = divides_by_reciprocal<T>(least, sum);
     asm volatile("" : "+v"(first));
     auto finish = [&](auto by_reciprocal) {
         const T rcp = decltype(by_reciprocal)::value ? (T)1 / sum : (T)0;
@@ -382,14 +411,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
                 const Pack<T, VEC> t = tg[k];
 #pragma unroll
                 for (int j = 0; j < VEC; j++) {
-                    T s;
-                    if constexpr (decltype(by_reciprocal)::value && sizeof(T) == 4) {
-                        const float a = v[k].v[j];
-                        const float q0 = a * rcp;
-                        s = __builtin_fmaf(__builtin_fmaf(-sum, q0, a), rcp, q0);
-                    } else {
-                        s = v[k].v[j] / sum;
-                    }
+                    const T s = decltype(by_reciprocal)::value ? quotient<T>(v[k].v[j], sum, rcp) : v[k].v[j] / sum;
                     v[k].v[j] = s;
                     if (CE) acc = (LONG || slot.own(j)) ? acc + t.v[j] * ml.log(s) : acc;
                 }
