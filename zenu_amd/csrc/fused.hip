@@ -334,29 +334,40 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
     const int head = (NT && !LONG && R + kMaxHead <= LANES * EPT) ? line_head(yr) : 0;
     int first = tid * VEC - head;
     const int Rr = LONG ? LANES * EPT : (int)R;        // the part in registers
+    // slots that every thread has whole, or no thread has: uniform, so that a row shorter than the registers costs
+    // neither loads nor masks for what it lacks
+    auto inner = [&](int k) { return LONG || (k * step >= head && (k + 1) * step - head <= Rr); };
+    auto beyond = [&](int k) { return !LONG && k * step - head >= Rr; };
     const T x0 = xr[0];
     T acc = (T)0;
 
     Pack<T, VEC> v[kPacks];
 #pragma unroll
-    for (int k = 0; k < kPacks; k++) v[k] = load_pack<T, VEC, NT>(xr + RowSlot<VEC>(first + k * step, Rr).at);
+    for (int k = 0; k < kPacks; k++) {
+        v[k] = splat<T, VEC>(-(T)INFINITY);
+        if (!beyond(k)) v[k] = load_pack<T, VEC, NT>(xr + RowSlot<VEC>(first + k * step, Rr).at);
+    }
     // the targets of the cross-entropy terms travel with the row: loaded where they are used, each
     // pack cost the end of the kernel a round trip of its own
     Pack<T, VEC> tg[kPacks];
     if (CE) {
 #pragma unroll
-        for (int k = 0; k < kPacks; k++) tg[k] = load_pack<T, VEC, NT>(tr + RowSlot<VEC>(first + k * step, Rr).at);
+        for (int k = 0; k < kPacks; k++)
+            if (!beyond(k)) tg[k] = load_pack<T, VEC, NT>(tr + RowSlot<VEC>(first + k * step, Rr).at);
     }
     ml.init(true, CE);      // after the row's loads are issued: the table fetch overlaps them
     asm volatile("" : "+v"(first));   // the slots are computed anew in every phase: kept, they take more registers than the row
     T m = -INFINITY;
 #pragma unroll
     for (int k = 0; k < kPacks; k++) {
-        const RowSlot<VEC> s(first + k * step, Rr);
+        if (!inner(k) && !beyond(k)) {
+            const RowSlot<VEC> s(first + k * step, Rr);
 #pragma unroll
-        for (int j = 0; j < VEC; j++) {
-            if (!LONG) v[k].v[j] = s.own(j) ? v[k].v[j] : -(T)INFINITY;
-            m = combine<T, true>(m, v[k].v[j]);
+            for (int j = 0; j < VEC; j++) v[k].v[j] = s.own(j) ? v[k].v[j] : -(T)INFINITY;
+        }
+        if (!beyond(k)) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) m = combine<T, true>(m, v[k].v[j]);
         }
     }
     if constexpr (LONG) {
@@ -378,7 +389,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
     uint32_t least = ~0u;   // f32: the smallest of this thread's terms above zero, as its bits less one
 #pragma unroll
     for (int k = 0; k < kPacks; k++) {
-        if (LONG || RowSlot<VEC>(first + k * step, Rr).any()) {
+        if (inner(k) || (!beyond(k) && RowSlot<VEC>(first + k * step, Rr).any())) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) {      // an element that is not the slot's own is exp(-inf), zero
                 v[k].v[j] = ml.exp_flat(v[k].v[j] - m);
@@ -407,7 +418,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
 #pragma unroll
         for (int k = 0; k < kPacks; k++) {
             const RowSlot<VEC> slot(first + k * step, Rr);
-            if (LONG || slot.any()) {
+            if (inner(k) || (!beyond(k) && slot.any())) {
                 const Pack<T, VEC> t = tg[k];
 #pragma unroll
                 for (int j = 0; j < VEC; j++) {
@@ -554,24 +565,34 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void softmax_bwd_rows_ke
     const int first = tid * VEC - head;
     const int Rr = LONG ? LANES * EPT : (int)R;
     auto product = [&](T yv, T g) { return yv * (CE ? (g * g_total) / yv : g); };
+    auto inner = [&](int k) { return LONG || (k * step >= head && (k + 1) * step - head <= Rr); };   // as in the forward pass
+    auto beyond = [&](int k) { return !LONG && k * step - head >= Rr; };
     T sum = (T)0;
     Pack<T, VEC> yv[kPacks], t[kPacks];
     // all loads of the thread first: with the loads inside a bounds check the compiler waits for each pair
     // before it issues the next, because the running sum orders the blocks
 #pragma unroll
     for (int k = 0; k < kPacks; k++) {
-        const RowSlot<VEC> s(first + k * step, Rr);
-        yv[k] = load_pack<T, VEC, NT && !CE>(yr + s.at);
-        t[k] = load_pack<T, VEC, NT>(sr + s.at);
+        if (!beyond(k)) {
+            const RowSlot<VEC> s(first + k * step, Rr);
+            yv[k] = load_pack<T, VEC, NT && !CE>(yr + s.at);
+            t[k] = load_pack<T, VEC, NT>(sr + s.at);
+        }
     }
 #pragma unroll
     for (int k = 0; k < kPacks; k++) {
         const RowSlot<VEC> s(first + k * step, Rr);
-        if (LONG || s.any()) {
+        if (inner(k)) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) {
                 t[k].v[j] = product(yv[k].v[j], t[k].v[j]);
-                sum = (LONG || s.own(j)) ? sum + t[k].v[j] : sum;
+                sum = sum + t[k].v[j];
+            }
+        } else if (!beyond(k) && s.any()) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) {
+                t[k].v[j] = product(yv[k].v[j], t[k].v[j]);
+                sum = s.own(j) ? sum + t[k].v[j] : sum;
             }
         }
     }
@@ -594,7 +615,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void softmax_bwd_rows_ke
 #pragma unroll
     for (int k = 0; k < kPacks; k++) {
         const RowSlot<VEC> s(first + k * step, Rr);
-        if (LONG || s.any()) {
+        if (inner(k) || (!beyond(k) && s.any())) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) t[k].v[j] = t[k].v[j] - yv[k].v[j] * sum;
             store_slot<T, VEC>(gr, s, t[k], [](T *row, int at, const Pack<T, VEC> &z) { store_pack<T, VEC, NT>(row + at, z); });
@@ -932,20 +953,19 @@ struct LineGrid {
 // the terms of the forward pass with the constants of exp, in 64 of them (f64 with 32 elements spills)
 template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
 
-// Threads per row and elements per thread of the rows kernels by row length; `spare` leaves
-// room for the alignment of a streaming row.  go(lanes, elements, long) gets constants.
-template <int EPT_LONG, typename Go> int with_row_shape(int64_t R, bool spare, Go go)
+// Threads per row and elements per thread of the rows kernels by row length (a streaming row
+// is cut at cache lines where the registers leave room for it).  go(lanes, elements, long) gets constants.
+template <int EPT_LONG, typename Go> int with_row_shape(int64_t R, Go go)
 {
-    const int64_t need = R + (spare ? kMaxHead : 0);
     typedef std::integral_constant<int, 64> L64;
     typedef std::integral_constant<int, 256> L256;
     typedef std::integral_constant<int, 512> L512;
     typedef std::integral_constant<int, 1024> L1024;
     typedef std::integral_constant<int, EPT_LONG> Long;
-    if (need <= 512) return go(L64(), std::integral_constant<int, 8>(), std::false_type());
-    if (need <= 1024) return go(L256(), std::integral_constant<int, 4>(), std::false_type());
-    if (need <= 4096) return go(L256(), std::integral_constant<int, 16>(), std::false_type());
-    if (need <= 512 * EPT_LONG) return go(L512(), Long(), std::false_type());
+    if (R <= 512) return go(L64(), std::integral_constant<int, 8>(), std::false_type());
+    if (R <= 1024) return go(L256(), std::integral_constant<int, 4>(), std::false_type());
+    if (R <= 4096) return go(L256(), std::integral_constant<int, 16>(), std::false_type());
+    if (R <= 512 * EPT_LONG) return go(L512(), Long(), std::false_type());
     if (R <= 1024 * EPT_LONG) return go(L1024(), Long(), std::false_type());
     return go(L1024(), Long(), std::true_type());
 }
@@ -981,7 +1001,7 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
         }
     } else {
         const bool nt = lines * g.R * (int64_t)sizeof(T) * 2 >= kStreamBytes;
-        const int rc = with_row_shape<kMost<T>>(g.R, nt, [&](auto lanes, auto ept, auto is_long) -> int {
+        const int rc = with_row_shape<kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
             constexpr bool LONG = decltype(is_long)::value;
             // f32: two workgroups of 512 threads on a CU instead of one of 1024, see softmax_rows_kernel
             constexpr bool two = decltype(lanes)::value == 1024 && decltype(ept)::value == 32 && !LONG && !CE;
@@ -1029,7 +1049,7 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
         }
     } else {
         const bool nt = lines * g.R * (int64_t)sizeof(T) * 3 >= kStreamBytes;
-        const int rc = with_row_shape<kMost<T>>(g.R, nt, [&](auto lanes, auto ept, auto is_long) -> int {
+        const int rc = with_row_shape<kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
             constexpr int L = decltype(lanes)::value, E = decltype(ept)::value;
             constexpr bool LONG = decltype(is_long)::value;
             constexpr int B = L < 256 ? 256 : L;
