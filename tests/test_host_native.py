@@ -73,6 +73,48 @@ def test_zmath_matches_host_libm(tmp_path):
                                   "tanhf_ulp2_beyond_2ulp", "0", "tanf_glibc", "0", "sin_glibc", "0", "cos_glibc", "0", "log_glibc", "0", "pow_glibc", "0"]
 
 
+def wait_states_before_stores(asm):
+    """for every store with a scalar base address: the wait states since a vector instruction wrote a register of it"""
+    import re
+    found, since = [], {}                   # register -> wait states since then
+    for line in asm.splitlines():
+        op = re.match(r"\t([a-z]\w+)\s*(.*)", line)
+        if not op:
+            if line.endswith(":"):
+                since = {}
+            continue
+        name, args = op.groups()
+        store = re.match(r"global_store_dwordx4 v\d+, v\[\d+:\d+\], s\[(\d+):(\d+)\]", f"{name} {args}")
+        if store:
+            found.append(min(since.get(r, 99) for r in range(int(store[1]), int(store[2]) + 1)))
+        states = int(args) + 1 if name == "s_nop" else 1
+        since = {r: n + states for r, n in since.items()}
+        written = re.match(r"s(\d+)\b", args)
+        if name.startswith(("v_readfirstlane", "v_readlane")) and written:
+            since[int(written[1])] = 0
+    return found
+
+
+def test_scalar_base_stores_wait_for_their_address(tmp_path):
+    """store_pack_wt_at right behind the vector instruction that produces its scalar address: gfx950 needs five wait
+    states between the two, and the compiler puts none in front of a written-out instruction"""
+    hipcc = "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    out = str(tmp_path / "store.s")
+    subprocess.check_call([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                           "-packed-fp32-ops", "--cuda-device-only", "-S", "-I", os.path.join(ROOT, "zenu_amd", "csrc"),
+                           os.path.join(NATIVE, "store_wait_states.hip"), "-o", out], stderr=subprocess.DEVNULL)
+    with open(out) as f:
+        states = wait_states_before_stores(f.read())
+    assert len(states) == 2 and min(states) >= 5, states
+    # the count itself: nothing in between, a wait count, s_nop
+    assert wait_states_before_stores("k:\n\tv_readfirstlane_b32 s3, v0\n\ts_waitcnt vmcnt(0)\n"
+                                     "\tglobal_store_dwordx4 v1, v[4:7], s[2:3] sc1 nt\n") == [1]
+    assert wait_states_before_stores("k:\n\tv_readlane_b32 s2, v0, 1\n\ts_nop 4\n"
+                                     "\tglobal_store_dwordx4 v1, v[4:7], s[2:3] sc1 nt\n") == [5]
+
+
 def _macro_numbers(text, name, following, pattern):
     import re
     start = text.index("#define " + name)
