@@ -91,6 +91,39 @@ def test_streaming_sizes(hip):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("fn", ["sigmoid", "exp", "sin", "tanh_backward", "add"])
+def test_small_tensors_give_the_bits_of_large_ones(hip, dtype, fn):
+    """Transcendental functions over small tensors go one element per lane, over larger ones by vectors: both sides of
+    either limit (2^17 and 2^20 elements on 256 CUs), single elements and every remainder of a vector, at two
+    alignments, against the same elements inside a tensor beyond both limits; nothing else is written"""
+    lim, r = 4096 * 256, np.random.default_rng(5)
+    n_all = lim + 4099
+    x, gy = (r.standard_normal(n_all) * 3).astype(dtype), r.standard_normal(n_all).astype(dtype)
+
+    def run(n, off):
+        whole = hip.Matrix.from_numpy(np.full(off + n + 4, 7, dtype))
+        out = hip.Matrix(whole.buf, off, (n,), (1,), dtype)
+        X, G = offset_matrix(hip, x[:n], off), offset_matrix(hip, gy[:n], 3)
+        if fn == "sigmoid":
+            code = hip._lib.F32 if dtype == np.float32 else hip._lib.F64
+            hip._lib.check(hip.lib().zenu_hip_unary(hip._lib.SIGMOID, code, C.byref(out.desc()), C.byref(X.desc()), None), fn)
+        elif fn == "tanh_backward":
+            out.tanh_backward(G, X)
+        elif fn == "add":
+            out.add_array(X, G)
+        else:
+            getattr(out, fn + "_array")(X)
+        got = whole.to_numpy()
+        assert np.all(got[:off] == 7) and np.all(got[off + n:] == 7), (n, off)
+        return got[off:off + n]
+
+    expect = run(n_all, 0)
+    for n in (1, 2, 3, 63, 65, 257, 511, 512, 514, 2047, 10007, 512 * 256, 512 * 256 + 1, lim - 1, lim, lim + 1, lim + 2, lim + 3):
+        for off in (0, 1):
+            assert np.array_equal(run(n, off), expect[:n]), (n, off)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("largest", [4099, 1 << 20], ids=["cached", "streamed"])
 def test_optimizer_tensors_of_any_size_and_alignment(hip, dtype, largest):
     """More tensors than one launch holds, around a vector and a tile long, each at another alignment: the

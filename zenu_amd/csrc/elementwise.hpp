@@ -285,6 +285,17 @@ template <> struct IsValuBound<PowF<double>> { static constexpr bool value = tru
 template <typename T> struct IsValuBound<TanhBwdF<T>> { static constexpr bool value = true; };
 template <typename T> struct IsValuBound<SigmoidBwdF<T>> { static constexpr bool value = true; };
 
+// Largest tensor, in elements per CU, that goes one element per lane instead of as vectors.  A transcendental functor
+// makes a lane's VEC * kUnroll elements a long chain; while the vectors leave SIMDs without work, four times the
+// wavefronts with a quarter of the chain are faster.  us as vectors / one per lane, by number of elements: f32 sigmoid
+// 10007: 4.1 / 2.4, 100003: 3.4 / 2.4, 600000: 3.9 / 3.3, 2^20: 4.2 / 4.1, 2^21: 6.2 / 6.1; f64 sigmoid 100003:
+// 3.3 / 2.7, 600000: 5.3 / 4.8, 2^20: 6.8 / 6.6; f32 exp 10007: 3.0 / 2.3, 100003: 3.0 / 2.4, 200000: 2.8 / 2.8,
+// 300001: 2.7 / 3.1.  Light functors (add, relu, copy) gain nothing.
+template <typename F> struct IsTranscendental { static constexpr bool value = IsValuBound<F>::value; };
+template <typename T, int FN> struct IsTranscendental<UnaryF<T, FN>> { static constexpr bool value = FN != ZENU_SQRT && FN != ZENU_ABS; };
+template <typename T> struct IsTranscendental<PowF<T>> { static constexpr bool value = true; };
+template <typename F> constexpr int64_t kSinglesPerCu = IsValuBound<F>::value ? 4096 : IsTranscendental<F>::value ? 512 : 0;
+
 template <typename F> struct ContigShape {
     static constexpr bool kSmall = F::NIN == 1 && !IsValuBound<F>::value;
     static constexpr int kBlock = kSmall ? ZENU_EW1_BLOCK : 256;
@@ -975,6 +986,14 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
     if (all_unit) {
         const int64_t n = p.numel;
         constexpr int cb = ContigShape<F>::kBlock, cu = ContigShape<F>::kUnroll;
+        if constexpr (kSinglesPerCu<F> > 0) {
+            if (n <= kSinglesPerCu<F> * device_info().num_cus) {
+                constexpr int64_t singles = (int64_t)cb * cu;
+                ew_contig_kernel<T, 1, false, F><<<(unsigned)((n + singles - 1) / singles), cb, 0, stream>>>(out, a, b, n, f);
+                ZENU_LAUNCH_CHECK();
+                return ZENU_OK;
+            }
+        }
         int64_t tile = (int64_t)cb * VEC * cu;
         int64_t grid = (n + tile - 1) / tile;
         if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
