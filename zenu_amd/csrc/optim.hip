@@ -303,11 +303,21 @@ int adam_t(void *p, const void *g, void *m, void *v, int64_t n, const AdamConsts
     constexpr int VEC = VecOf<T>::N;
     if (n == 0) return ZENU_OK;
     if (adam_arrays_overlap(p, g, m, v, (size_t)n * sizeof(T))) return ZENU_ERR_ARG;
-    const bool nt = n * (int64_t)sizeof(T) * 7 >= kStreamBytes;  // 7 passes exceed the caches: stream
-    const int64_t tile = (int64_t)kBlock * VEC * kUnroll;
+    const bool aligned = aligned16(p) && aligned16(g) && aligned16(m) && aligned16(v);
+    const bool stream = n * (int64_t)sizeof(T) * 7 >= kStreamBytes;  // 7 passes exceed the caches: stream
+    // Seven streams of unaligned vectors, each split over two cache lines at its ends, are slower than single elements
+    // (us, vectors / elements, one element past a vector: f32 10007: 3.9 / 2.9, 300001: 4.8 / 3.6, 2^24: 90 / 76; f64
+    // 10007: 3.4 / 2.8, 2^24: 197 / 166), but for arrays that pass through caches full of other kernels' results, where
+    // the hint counts for more: 2^21 f32 12.8 / 15.8, 2^20 f64 12.7 / 16.0.
+    const bool vec = aligned || (stream && n * (int64_t)sizeof(T) < kStreamBytes);
+    const bool nt = vec && stream;
+    const int64_t tile = (int64_t)kBlock * (vec ? VEC : 1) * kUnroll;
     const int64_t grid = (n + tile - 1) / tile;
     if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
-    if (nt)
+    if (!vec)
+        adam_kernel<T, 1, false><<<(unsigned)grid, kBlock, 0, s>>>(
+            static_cast<T *>(p), static_cast<const T *>(g), static_cast<T *>(m), static_cast<T *>(v), n, k, decay);
+    else if (nt)
         adam_kernel<T, VEC, true><<<(unsigned)grid, kBlock, 0, s>>>(
             static_cast<T *>(p), static_cast<const T *>(g), static_cast<T *>(m), static_cast<T *>(v), n, k, decay);
     else
