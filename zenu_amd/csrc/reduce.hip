@@ -954,8 +954,11 @@ template <typename T, typename Tr>
 int launch_rows(const RedParams<T> &p, hipStream_t s)
 {
     constexpr int VEC = VecOf<T>::N;
-    // vectors whatever the alignment of the rows; [10007,1003] f64 row sums take 13.6 us (80 MB) as with scalar loads
-    const bool vec = p.elem_stride == 1 && p.inner == 1 && p.R >= VEC;
+    // Vectors whatever the alignment of the rows, but for rows that a wavefront takes in one load per lane either way:
+    // the masked vectors are more instructions than single elements (us, vectors / elements: row sums of [65536,33] f32
+    // 10.4 / 8.4, f64 11.5 / 10.1, arg-max 16.3 / 14.0; of [16384,64] 4.2 / 3.9).  Longer rows, f32: [65536,101] 11.7 /
+    // 12.9, [16384,255] 9.3 / 11.3, [1000,999] 2.7 / 3.3; f64: [10007,1003] 13.5 / 13.6, [1000,999] 3.3 / 4.3.
+    const bool vec = p.elem_stride == 1 && p.inner == 1 && p.R >= VEC && p.R > kWave;
     const bool nt = vec && stream_source(p);
     const bool wave_row = p.splits == 1 && p.R <= 1024;
     if (wave_row) {
