@@ -213,6 +213,39 @@ def test_reductions_at_any_alignment(hip, dtype, shape):
             assert abs(total.to_numpy()[0] - exact) <= clean.size * eps * exact, shape
 
 
+# rows of a wavefront's lanes and one around them; columns: one per lane, narrow and wide vector tiles, each with and
+# without splits, around the limits of rows (512, 1024, 4096) and columns (64, 128, 256, 512)
+EXACT = [(70, 63), (70, 64), (70, 65), (64, 17), (513, 65), (600, 127), (1024, 129), (1025, 127), (1025, 131), (2048, 255), (3000, 257),
+         (4097, 33), (5000, 67), (10007, 127), (30001, 65), (3000, 513), (1000, 1001)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", EXACT, ids=str)
+def test_reductions_of_small_integers_are_exact(hip, dtype, shape):
+    """Integers of -15 .. 15 without 0: every partial sum stays below 2^24, so any order of the additions gives the exact
+    result in f32, and an element that is lost, added twice or taken from beside the source changes it.  The same source
+    gives the first positions of the maxima, of which every row and column holds several."""
+    rows, cols = shape
+    r = np.random.default_rng(rows + cols)
+    a = (r.integers(1, 16, shape) * r.choice([-1, 1], shape)).astype(dtype)
+    whole = offset_matrix(hip, a, 1)
+    big = hip.Matrix.from_numpy(np.concatenate([np.full((rows, 3), 1e6, dtype), a, np.full((rows, 2), 1e6, dtype)], axis=1))
+    code = hip._lib.F32 if dtype == np.float32 else hip._lib.F64
+    for m in (hip.Matrix.from_numpy(a), whole, big.slice(slice(None), slice(3, 3 + cols))):
+        for axis in (0, 1):
+            kept = (1, cols) if axis == 0 else (rows, 1)
+            out = offset_matrix(hip, np.full(kept, 7, dtype), 1)
+            hip.sum_to(m, out)
+            same(out.to_numpy(), a.sum(axis=axis, keepdims=True), ("sum", shape, axis))
+            at = hip.Matrix.alloc((a.size // a.shape[axis],), np.float64)
+            hip._lib.check(hip.lib().zenu_hip_max_axis_idx(code, at.as_ptr(), C.byref(m.desc()), axis, None), "max_axis_idx")
+            same(at.to_numpy().view(np.int64), np.argmax(a, axis=axis), ("arg-max", shape, axis))
+    total = hip.Matrix.alloc((1,), dtype)
+    few = offset_matrix(hip, np.clip(a, -1, 1), 3)
+    hip._lib.check(hip.lib().zenu_hip_asum(code, total.as_ptr(), C.byref(few.desc()), None), "asum")
+    assert total.to_numpy()[0] == a.size
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("shape", [(3, 1), (5, 3), (4, 256), (7, 1500), (33, 1027), (9000, 999), (8200, 1024)], ids=str)
 @pytest.mark.parametrize("with_pre", [True, False])

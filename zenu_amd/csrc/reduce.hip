@@ -261,6 +261,7 @@ template <typename T> struct RedParams {
     // value gather for max: value = gsrc[q * g_outer_stride + c + idx * g_elem_stride]
     const T *gsrc;
     int64_t g_outer_stride, g_elem_stride;
+    int cols_vec;            // columns of a lane in the column kernels, VEC or 1 (for the host; last, so that it moves no other field)
 };
 
 template <typename T, typename Tr>
@@ -1001,10 +1002,9 @@ template <typename T, typename Tr>
 int launch_cols(const RedParams<T> &p, hipStream_t s)
 {
     constexpr int VEC = VecOf<T>::N;
-    // (vectors whatever the alignment: column sums of [10007,1003] f64 19.6 us (80 MB), 32.3 with scalar loads)
     const bool nt = stream_source(p);
     const int shift = p.cols_shift;
-    const int64_t per_tile = ((int64_t)1 << shift) * VEC;
+    const int64_t per_tile = ((int64_t)1 << shift) * p.cols_vec;
     const int64_t col_tiles = (p.inner + per_tile - 1) / per_tile;
     const int64_t outer = p.nout / p.inner;
     int64_t grid = outer * col_tiles * p.splits;
@@ -1013,7 +1013,7 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
     const dim3 g = g3 ? dim3((unsigned)col_tiles, (unsigned)p.splits, (unsigned)outer) : dim3((unsigned)grid);
     const uint32_t ctl = (uint32_t)col_tiles;
     // the regular geometry: full vector tiles of 32 x 8 threads, a split axis with a flat counter
-    const bool regular = g3 && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
+    const bool regular = g3 && p.cols_vec == VEC && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
     if constexpr (!Tr::kHasIdx && std::is_same<Tr, SumTr<T>>::value) {
         if (p.pre_x) {   // (the caller has checked that a row is a whole number of vectors)
             if (regular) {
@@ -1033,8 +1033,9 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
         ZENU_LAUNCH_CHECK();
         return ZENU_OK;
     }
-    if (nt) reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-    else    reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    if (p.cols_vec == 1) reduce_cols_kernel<T, Tr, 1, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    else if (nt)         reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    else                 reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
     ZENU_LAUNCH_CHECK();
     return ZENU_OK;
 }
@@ -1090,9 +1091,27 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
     if (pre_x && (!use_cols || inner % VEC)) return ZENU_ERR_UNSUPPORTED;   // the caller falls back to two launches
     int64_t splits = 1, groups = nout;
     p.cols_shift = 0;
+    p.cols_vec = VEC;
     if (use_cols) {
-        int shift = cols_tx_shift(inner, VEC);
-        auto tiles_at = [&](int sh) { return (inner + (((int64_t)1 << sh) * VEC) - 1) / (((int64_t)1 << sh) * VEC); };
+        // Vectors of columns whatever the alignment (column sums of [10007,1003] f64 19.6 us, 32.3 with single ones), but
+        // for two kinds of source where a lane takes one column, so that four (f64: two) times as many column tiles
+        // share the fold and its hand-over.  Arg-max below the streaming sizes: its partial results are pairs and its
+        // updates three instructions ([3000,127] f32 10.4 -> 7.7 us, [10007,255] 18.7 -> 9.7, [30000,65] 27.7 -> 13.2).
+        // Not with many rows of under 64 columns ([30000,17] 10 against 18) nor over 512 columns of f64 ([1000,1003] 7.2
+        // against 8.0); beyond those sizes vectors ([10007,5001] f32 28 against 43).  And sums over few rows of a narrow
+        // source that is no whole number of aligned vectors ([600,65] f32 5.7 -> 5.3, [64,65] 3.4 -> 3.0).
+        const bool whole = aligned16(src) && inner % VEC == 0 && outer_stride % VEC == 0 && elem_stride % VEC == 0;
+        const int64_t bytes = nout * R * (int64_t)sizeof(T);
+        const bool narrow = inner < kColsTx * VEC;
+        if (!pre_x && (Tr::kHasIdx ? bytes < kStreamBytes && (inner >= 2 * kColsTx || R <= 4096) && (VEC == 4 || inner <= 512) : !whole && narrow && R <= 1024)) p.cols_vec = 1;
+        const int v = p.cols_vec;
+        int shift = cols_tx_shift(inner, v);
+        auto tiles_at = [&](int sh) { return (inner + (((int64_t)1 << sh) * v) - 1) / (((int64_t)1 << sh) * v); };
+        // One or two column tiles over many rows: hundreds of workgroups hand over to one or two that fold them.  Tiles of a
+        // quarter of the width have fewer splits each (column sums of [30000,65] f32 16.4 -> 8.2 us, [10007,127]
+        // 11.6 -> 7.4, [65536,128] 22 -> 11; f64 [30000,33] 13.2 -> 7.9).  Larger sources stream better in wide rows
+        // ([65537,101] f64, 53 MB, 18.3 against 23; [65537,127] f32, 33 MB, 28 -> 18).
+        if (v == VEC && !pre_x && shift > 3 && outer * tiles_at(shift) <= 2 && R > 1024 && bytes < (sizeof(T) == 4 ? 2 * kStreamBytes : kStreamBytes / 2)) shift = 3;
         // A small source with a short reduced axis is bound by latencies, and the hand-off of a split
         // (about 3 us) is the longest of them: narrower column tiles (down to 64-byte row pieces, which
         // stream at less than half the rate, but there is little to stream) give more workgroups
