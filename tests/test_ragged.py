@@ -280,3 +280,23 @@ def test_sums_over_several_axes(hip, dtype, shape, kept):
     exact, scale = wide.sum(axis=axes).reshape(kept), np.abs(wide).sum(axis=axes).reshape(kept)
     n = x.size // max(exact.size, 1)
     assert np.all(np.abs(out.to_numpy() - exact) <= n * np.finfo(dtype).eps * scale)
+
+
+# channels fewer and more than compute units (one and several workgroups per channel), pieces of part of a cache line, of
+# whole ones and of one and a part, and a million pieces, whose axes go one after the other
+PIECES = [(5, 3, 7), (2, 256, 4), (37, 257, 9), (130, 300, 25), (600, 31, 32), (9, 520, 64), (70, 513, 16), (2100, 500, 4), (3, 40, 3001)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", PIECES, ids=str)
+def test_sums_over_images_and_pixels_are_exact(hip, dtype, shape):
+    """integers whose sums are exact in any order, the source starting at three alignments; one element counted twice or
+    left out changes a channel's sum"""
+    n, c, i = shape
+    r = np.random.default_rng(sum(shape))
+    x = (r.integers(1, 16, shape) * r.choice([-1, 1], shape)).astype(dtype)
+    exp = x.sum(axis=(0, 2), keepdims=True)
+    for off in (0, 1, 32):
+        out = offset_matrix(hip, np.full((1, c, 1), 7, dtype), 1)
+        hip.sum_to(offset_matrix(hip, x, off), out)
+        same(out.to_numpy(), exp, (shape, off))

@@ -903,11 +903,18 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
 // workspaces, 12.4 us and three launches.
 template <typename T, int VEC, bool NT>
 __global__ __launch_bounds__(kBlock) void reduce_pieces_kernel(const T *src, T *out, uint32_t N, uint32_t C, int64_t I,
-                                                               uint32_t splits, uint32_t vecs)
+                                                               uint32_t splits, uint32_t vecs, bool banded)
 {
     typedef SumTr<T> Tr;
     constexpr int U = 4;
-    const uint32_t c = blockIdx.x / splits, split = blockIdx.x - c * splits;
+    // Workgroup i runs on XCD i mod 8.  With neighbouring channels on neighbouring workgroups every XCD reads every cache
+    // line that two short pieces share; `banded` gives each XCD a run of consecutive ones, and its L2 serves the second.
+    uint32_t wg = blockIdx.x;
+    if (banded) {
+        const uint32_t share = gridDim.x >> 3, rest = gridDim.x & 7, xcd = wg & 7;
+        wg = xcd * share + (xcd < rest ? xcd : rest) + (wg >> 3);
+    }
+    const uint32_t c = wg / splits, split = wg - c * splits;
     const uint32_t pieces = (N - split + splits - 1) / splits;
     const int64_t piece_step = (int64_t)splits * C * I;
     const T *const base = src + ((int64_t)split * C + c) * I;
@@ -940,7 +947,7 @@ __global__ __launch_bounds__(kBlock) void reduce_pieces_kernel(const T *src, T *
         }
     }
     const T total = block_allreduce<Tr>((acc[0] + acc[1]) + (acc[2] + acc[3]));
-    if (threadIdx.x == 0) out[blockIdx.x] = total;
+    if (threadIdx.x == 0) out[wg] = total;
 }
 
 // ---- host side ---------------------------------------------------------------------------------------------
@@ -1260,13 +1267,20 @@ int sum_pieces(const T *src, int64_t N, int64_t C, int64_t I, T *out, hipStream_
     if (splits > N) splits = N;
     if (C * splits < device_info().num_cus && splits == N && vecs > 4 * kBlock) return ZENU_ERR_UNSUPPORTED;
     if (C * splits > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
+    // Pieces that share cache lines with their neighbours.  From a million on the axes go one after the other, whole rows at
+    // a time ([1024,2048,4] f32 12 us against 48 and, banded, 21; [4096,256,25] 25 / 40 / 34).  Banded with many channels
+    // ([256,2048,9] 14.4 -> 6.0 us, [128,2048,25] 10.0 -> 5.0, [256,2048,49] 28.6 -> 24.0), not with few, whose pieces are
+    // spread over workgroups ([30000,8,9] 5.8 against 12.3), nor where pieces are whole lines ([256,2048,16] f64 12.4 / 14.3).
+    const bool share_lines = I * (int64_t)sizeof(T) % 128 != 0 || reinterpret_cast<uintptr_t>(src) % 128 != 0;
+    if (share_lines && N * C >= (1 << 20)) return ZENU_ERR_UNSUPPORTED;
+    const bool banded = share_lines && C >= device_info().num_cus;
     Workspace ws(splits > 1 ? (size_t)(C * splits) * sizeof(T) : 0, s);
     if (ws.status) return ws.status;
     T *const part = splits > 1 ? static_cast<T *>(ws.ptr) : out;
     const bool nt = N * C * I * (int64_t)sizeof(T) >= kStreamBytes;
     const unsigned grid = (unsigned)(C * splits);
-    if (nt) reduce_pieces_kernel<T, VEC, true><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs);
-    else    reduce_pieces_kernel<T, VEC, false><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs);
+    if (nt) reduce_pieces_kernel<T, VEC, true><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs, banded);
+    else    reduce_pieces_kernel<T, VEC, false><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs, banded);
     ZENU_LAUNCH_CHECK();
     return splits > 1 ? reduce_contiguous<T, SumTr<T>>(part, C, splits, 1, out, nullptr, s) : ZENU_OK;
 }
