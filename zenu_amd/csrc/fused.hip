@@ -985,6 +985,15 @@ inline int line_own(int64_t lines, int64_t R, int most)
     }
     return 8;
 }
+// The most elements a thread of the forward pass holds.  Rows of the last axis (R <= 64) need no more than eight
+// wavefronts of 8, and the loss takes those: with a logarithm per element its constants spill at 16 and 32 elements (f32
+// [65536,64] 93.8 us at 32, 51.8 at 8; f64 110 / 77.5); plain f64 takes 16 (96 -> 38 us).  Plain f32 and other axes
+// hold up to 32.
+template <typename T, bool CE> inline int line_most(const Geometry &g)
+{
+    if (g.inner > 1 || g.R <= 16) return 32;
+    return CE ? 8 : sizeof(T) == 8 ? 16 : 32;
+}
 // calls go(own) with `own` as a constant
 template <int MOST, typename Go> int with_own(int own, Go go)
 {
@@ -1043,7 +1052,7 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
     }
     if (g.inner != 1 || g.R <= kLineMaxR) {
         // (16 elements at most where the whole loss is one workgroup: 16 wavefronts hold 256 lines of 64)
-        int own = line_own(lines, g.R, 32);
+        int own = line_own(lines, g.R, line_most<T, CE>(g));
         if (CE && loss && own < 16 && (lines + 63) / 64 * ((g.R + own - 1) / own) > kLineWaves) own = 16;
         if (own == 0) {
             const int64_t blocks = (lines + kBlock - 1) / kBlock;
