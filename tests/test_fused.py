@@ -225,6 +225,51 @@ def test_softmax_kernel_edges(hip, dtype, shape):
     assert np.all(ends[:2] == 0) and np.all(ends[-5:] == 7)
 
 
+# Rows for the exact test below: few and many, around each limit of a wavefront, of 256 threads (single elements and
+# vectors) and of larger workgroups, totals below and above the streaming size.  Powers of two of them, see below.
+EXACT_ROWS = [(4, 65), (512, 127), (1024, 128), (2048, 255), (512, 256), (1024, 300), (512, 511), (2048, 512), (2048, 513), (4, 600),
+              (2048, 769), (2048, 1001), (4, 1023), (2048, 1024), (8, 1025), (8, 1100), (16, 2047), (16, 2048), (8, 2052), (16, 4095),
+              (16, 4096), (4, 4097), (4, 16383), (4, 16385), (2, 32769), (2, 40003), (65536, 33), (131072, 64), (16384, 255), (8192, 1001)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("n,c", EXACT_ROWS)
+def test_rows_count_every_element_once(hip, dtype, n, c, off):
+    """Operands for which every sum is exact in any order, so that one element left out, or taken twice, shows at any
+    length: constant rows, whose divisor is the row's length; backward over small whole numbers, n a power of two.
+    The loss, targets all one, sums c logarithms: a thread adds at most 64, 16 levels follow and 16 for
+    the rows, a logarithm and a quotient are off by a few eps; one term of 40003 is 400 eps."""
+    print(f"[case] exact rows {n}x{c}+{off} {np.dtype(dtype).name}", flush=True)
+    eps = np.finfo(dtype).eps
+
+    def put(a):
+        m = hip.Matrix.from_numpy(np.concatenate([np.zeros(off, dtype), a.reshape(-1)]))
+        return hip.Matrix(m.buf, off, (n, c), hip.default_stride((n, c)), dtype)
+
+    x = put(np.full((n, c), 1.25, dtype))
+    y = put(np.zeros((n, c), dtype))
+    y.softmax_assign(x, 1)
+    got = y.to_numpy()
+    assert np.all(np.abs(got.astype(np.float64) * c - 1) <= 2 * eps)
+    loss, prob = hip.cross_entropy(x, put(np.ones((n, c), dtype)))
+    assert np.all(np.abs(prob.to_numpy().astype(np.float64) * c - 1) <= 2 * eps)
+    if n <= 2048:
+        assert abs(float(loss.to_numpy()) / (c * np.log(float(c))) - 1) <= 112 * eps
+
+    r = np.random.default_rng(n + c)
+    yv = r.integers(1, 3, (n, c)).astype(dtype)
+    gy = r.integers(-1, 3, (n, c)).astype(dtype)
+    gx, yd, gd = put(np.zeros((n, c), dtype)), put(yv), put(gy)
+    code = hip._lib.F32 if dtype == np.float32 else hip._lib.F64
+    hip._lib.check(hip.lib().zenu_hip_softmax_backward(code, C.byref(gx.desc()), C.byref(yd.desc()), C.byref(gd.desc()), 1, None),
+                   "softmax_backward")
+    t = yv * gy
+    assert np.array_equal(gx.to_numpy(), t - yv * t.sum(axis=1, keepdims=True))
+    g = hip.cross_entropy_backward(yd, gd).to_numpy()
+    assert np.array_equal(g * n, yv * gy.sum(axis=1, keepdims=True) - gy)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("n,c", [(193, 40), (130, 64), (257, 63), (31, 513), (1000, 999), (700, 4099), (2, 32769)])
 def test_cross_entropy_kernel_edges(hip, dtype, n, c):

@@ -306,13 +306,13 @@ template <typename T, int VEC> __device__ __forceinline__ void store_some(T *p, 
         if (j < n) p[j] = v.v[j];
 }
 
-// Plain softmax over rows of whole, aligned vectors that 256 threads hold in four vectors each: without the slots of
-// the general kernel below, whose bookkeeping costs 4 - 8 % here (f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
-// 44.7 / 48.7, [32768,1024] 61.0 / 63.0; from 512 elements down a wavefront per row is faster: [65536,512] 92 / 47).
-template <typename T, bool NT>
-__global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, T *y, int64_t R, zmath::ExpLog<T> ml)
+// Rows that 256 threads hold in four vectors each, single elements with VEC == 1: without the slots of the general
+// kernel below, whose bookkeeping costs 3 - 9 % on long rows (f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
+// 44.7 / 48.7) and more where a launch is a few microseconds; whole_row_vector says which rows come here.
+template <typename T, bool CE, bool NT, int VEC>
+__global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, T *y, int64_t R, const T *target, T *rowloss,
+                                                                     zmath::ExpLog<T> ml)
 {
-    constexpr int VEC = VecOf<T>::N;
     __shared__ T lds[kWaves];
     const int64_t row = blockIdx.x;
     const T *xr = x + row * R;
@@ -329,7 +329,15 @@ __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, 
 #pragma unroll
         for (int j = 0; j < VEC; j++) m = combine<T, true>(m, v[k].v[j]);
     }
-    ml.init(true, false);   // after the row's loads are issued: the table fetch overlaps them
+    Pack<T, VEC> tg[kWholePacks];
+    if (CE) {
+#pragma unroll
+        for (int k = 0; k < kWholePacks; k++) {
+            const int64_t r = first + k * step;
+            if (r < R) tg[k] = load_pack<T, VEC, NT>(target + row * R + r);
+        }
+    }
+    ml.init(true, CE);   // after the row's loads are issued: the table fetch overlaps them
     m = block_red<T, true, kBlock>(m, lds);
     if (x0 != x0) m = x0;   // a NaN in position 0 is never replaced
     T sum = (T)0;
@@ -346,6 +354,7 @@ __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, 
         }
     }
     sum = block_red<T, false, kBlock>(sum, lds);
+    T acc = (T)0;
     auto finish = [&](auto by_reciprocal) {
         const T rcp = decltype(by_reciprocal)::value ? (T)1 / sum : (T)0;
 #pragma unroll
@@ -353,15 +362,21 @@ __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, 
             const int64_t r = first + k * step;
             if (r < R) {
 #pragma unroll
-                for (int j = 0; j < VEC; j++)
+                for (int j = 0; j < VEC; j++) {
                     v[k].v[j] = decltype(by_reciprocal)::value ? quotient<T>(v[k].v[j], sum, rcp) : v[k].v[j] / sum;
-                if constexpr (NT) store_pack_wt<T, VEC>(yr + r, v[k]);
+                    if (CE) acc = acc + tg[k].v[j] * ml.log(v[k].v[j]);
+                }
+                if constexpr (NT && !CE) store_pack_wt<T, VEC>(yr + r, v[k]);
                 else store_pack<T, VEC, false>(yr + r, v[k]);
             }
         }
     };
     if (divides_by_reciprocal<T>(least, sum)) finish(std::true_type());
     else finish(std::false_type());
+    if (CE) {
+        acc = block_red<T, false, kBlock>(acc, lds);
+        if (threadIdx.x == 0) rowloss[row] = acc;
+    }
 }
 
 // The softmax axis is the last one: LANES threads hold a row in registers, EPT elements each, and read and write
@@ -1023,7 +1038,7 @@ template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
 
 // Threads per row and elements per thread of the rows kernels by row length (a streaming row
 // is cut at cache lines where the registers leave room for it).  go(lanes, elements, long) gets constants.
-template <int EPT_LONG, typename Go> int with_row_shape(int64_t R, Go go)
+template <int VEC, int EPT_LONG, typename Go> int with_row_shape(int64_t R, Go go)
 {
     typedef std::integral_constant<int, 64> L64;
     typedef std::integral_constant<int, 256> L256;
@@ -1032,10 +1047,34 @@ template <int EPT_LONG, typename Go> int with_row_shape(int64_t R, Go go)
     typedef std::integral_constant<int, EPT_LONG> Long;
     if (R <= 512) return go(L64(), std::integral_constant<int, 8>(), std::false_type());
     if (R <= 1024) return go(L256(), std::integral_constant<int, 4>(), std::false_type());
+    if (R <= 1024 * VEC) return go(L256(), std::integral_constant<int, 4 * VEC>(), std::false_type());
     if (R <= 4096) return go(L256(), std::integral_constant<int, 16>(), std::false_type());
     if (R <= 512 * EPT_LONG) return go(L512(), Long(), std::false_type());
     if (R <= 1024 * EPT_LONG) return go(L1024(), Long(), std::false_type());
     return go(L1024(), Long(), std::true_type());
+}
+
+template <typename T> inline bool whole_rows(int64_t R, const T *in, const T *out)
+{
+    return R % VecOf<T>::N == 0 && aligned16(in) && aligned16(out);
+}
+// Vector width with which softmax_whole_rows_kernel takes rows of R > kLineMaxR elements; 0: the general kernel does.
+// Single elements: few rows (four per CU, in f64 up to 256 elements two), as long as a wavefront would hold a long row
+// or one with ragged ends: the shorter chain counts (f32 [100,301] 3.3 us against 4.2 in the general kernel, f64 [100,512]
+// 3.8 / 5.2, its loss [100,256] 5.9 / 7.0; but f64 loss [1000,127] 8.2 / 7.2); and ragged rows beyond a wavefront's 512,
+// [32768,513] f32 39.6 / 47 us, f64 62 / 65 (the loss to 768: [32768,641] 67 / 80 us, [32768,1001] 95 / 90 after writes).
+// Vectors: plain rows beyond 512 (those of a wavefront are faster: [65536,512] 92 / 47 us), the loss beyond one
+// vector per thread ([32768,1100] f32 108 / 123 us, [4096,1100] f64 30 / 41; [4096,1024] f32 18.8 / 17.9).
+template <typename T, bool CE> inline int whole_row_vector(int64_t lines, int64_t R, bool whole)
+{
+    constexpr int VEC = VecOf<T>::N;
+    const int64_t cus = device_info().num_cus;
+    const bool few = lines <= (sizeof(T) == 8 && R <= 256 ? 2 : 4) * cus;
+    if (R <= kWholePacks * kBlock) {
+        if (few && (!whole || R > 256 || sizeof(T) == 8)) return 1;
+        if (!whole && R > 512 && (!CE || R <= 768)) return 1;
+    }
+    return whole && R > (CE ? kBlock * VEC : 512) && R <= kWholePacks * kBlock * VEC ? VEC : 0;
 }
 
 template <typename T, bool CE>
@@ -1068,18 +1107,22 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
             });
         }
     } else {
-        const bool nt = lines * g.R * (int64_t)sizeof(T) * 2 >= kStreamBytes;
-        if constexpr (!CE) {
-            constexpr int VEC = VecOf<T>::N;
-            if (g.R > 512 && g.R <= kWholePacks * kBlock * VEC && g.R % VEC == 0 && aligned16(x) && aligned16(y)) {
-                if (!grid_ok(lines)) return ZENU_ERR_UNSUPPORTED;
-                if (nt) softmax_whole_rows_kernel<T, true><<<(unsigned)lines, kBlock, 0, s>>>(x, y, g.R, zmath::ExpLog<T>());
-                else    softmax_whole_rows_kernel<T, false><<<(unsigned)lines, kBlock, 0, s>>>(x, y, g.R, zmath::ExpLog<T>());
-                ZENU_LAUNCH_CHECK();
-                return ZENU_OK;
-            }
+        const bool whole = whole_rows<T>(g.R, x, y);
+        // ragged rows of a wavefront share their first and last lines with other rows: written past the cache, softmax of
+        // [32768,255] f32 takes 53 us, 19 without the hint.  The loss keeps its probabilities cached in any case.
+        const bool nt = lines * g.R * (int64_t)sizeof(T) * 2 >= kStreamBytes && (CE || whole || g.R > 1024);
+        constexpr int VEC = VecOf<T>::N;
+        const int vec = whole_row_vector<T, CE>(lines, g.R, whole);
+        if (vec) {
+            if (!grid_ok(lines)) return ZENU_ERR_UNSUPPORTED;
+            const unsigned grid = (unsigned)lines;
+            if (vec == 1) softmax_whole_rows_kernel<T, CE, false, 1><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
+            else if (nt)  softmax_whole_rows_kernel<T, CE, true, VEC><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
+            else          softmax_whole_rows_kernel<T, CE, false, VEC><<<grid, kBlock, 0, s>>>(x, y, g.R, target, rowloss, zmath::ExpLog<T>());
+            ZENU_LAUNCH_CHECK();
+            return ZENU_OK;
         }
-        const int rc = with_row_shape<kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
+        const int rc = with_row_shape<VecOf<T>::N, kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
             constexpr bool LONG = decltype(is_long)::value;
             // f32: two workgroups of 512 threads on a CU instead of one of 1024, see softmax_rows_kernel
             constexpr bool two = decltype(lanes)::value == 1024 && decltype(ept)::value == 32 && !LONG && !CE;
@@ -1127,7 +1170,7 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
         }
     } else {
         const bool nt = lines * g.R * (int64_t)sizeof(T) * 3 >= kStreamBytes;
-        const int rc = with_row_shape<kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
+        const int rc = with_row_shape<VecOf<T>::N, kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
             constexpr int L = decltype(lanes)::value, E = decltype(ept)::value;
             constexpr bool LONG = decltype(is_long)::value;
             constexpr int B = L < 256 ? 256 : L;
