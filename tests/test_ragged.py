@@ -72,6 +72,17 @@ def test_rows_of_a_wider_matrix(hip, dtype, cols):
     same(D.to_numpy(), exp, "slice copy")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 5, 7])
+def test_short_rows_repeated(hip, dtype, cols):
+    """a row shorter than a vector, as long, and longer, over many rows"""
+    row = np.arange(1, cols + 1).astype(dtype)
+    for rows in (1, 37, 3001):
+        out = offset_matrix(hip, np.zeros((rows, cols), dtype), 1)
+        out.broadcast(offset_matrix(hip, row, 3))
+        same(out.to_numpy(), np.broadcast_to(row, (rows, cols)), rows)
+
+
 def test_streaming_sizes(hip):
     """beyond the caches (streaming accesses), every operand starting in the middle of a vector"""
     r = np.random.default_rng(3)
