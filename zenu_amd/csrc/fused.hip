@@ -28,7 +28,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kWholePacks = 4;  // vectors per thread of softmax_whole_rows_kernel
-constexpr int kLineMaxR = 64;   // rows up to this length: one thread per row
+constexpr int kLineMaxR = 64;   // rows up to this length: a lane per row, on one or several wavefronts
 
 // ---- workgroup reductions in a fixed order ------------------------------------------------------------
 
@@ -307,8 +307,8 @@ template <typename T, int VEC> __device__ __forceinline__ void store_some(T *p, 
 }
 
 // Rows that 256 threads hold in four vectors each, single elements with VEC == 1: without the slots of the general
-// kernel below, whose bookkeeping costs 3 - 9 % on long rows (f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
-// 44.7 / 48.7) and more where a launch is a few microseconds; whole_row_vector says which rows come here.
+// kernel below, whose bookkeeping costs 5 - 9 % on long rows (f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
+// 44.7 / 48.7; even at [32768,1024], 61 - 63) and more where a launch is a few microseconds; whole_row_vector says which rows come here.
 template <typename T, bool CE, bool NT, int VEC>
 __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, T *y, int64_t R, const T *target, T *rowloss,
                                                                      zmath::ExpLog<T> ml)

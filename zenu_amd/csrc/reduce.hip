@@ -435,7 +435,7 @@ __device__ __forceinline__ bool arrive_last(int *c, int split, int splits, int f
 }
 
 // ---- kernel A: rows --------------------------------------------------------------------------------------
-// VEC > 1 requires elem_stride == 1, 16-byte aligned rows (checked on the host).
+// VEC > 1 requires elem_stride == 1 and rows of VEC elements or more, at any alignment.
 // WAVE_ROW: one wavefront per output (4 outputs per workgroup, never split), otherwise one
 // workgroup per (output, split); with splits > 1 the last workgroup of an output to finish folds
 // that output's partials in a fixed order.
