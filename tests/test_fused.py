@@ -554,6 +554,19 @@ def test_relu_backward_bias_grad(hip, dtype, shape, alpha):
     assert bits_equal(GY.to_numpy(), gx.to_numpy()) and bits_equal(gb3.to_numpy(), gb.to_numpy())
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("n,c", [(1025, 64), (1100, 128), (4096, 32), (10007, 256), (30000, 16), (2000, 192)])
+def test_bias_gradient_has_the_bits_of_sum_to(hip, dtype, n, c):
+    """many rows of one or a few column tiles: the sums of the one-launch form and of the plain reduction share their geometry"""
+    r = np.random.default_rng(n)
+    M = hip.Matrix
+    x, gy = M.from_numpy(r.standard_normal((n, c)).astype(dtype)), M.from_numpy(r.standard_normal((n, c)).astype(dtype))
+    gx, gb, plain = M.alloc((n, c), dtype), M.alloc((c,), dtype), M.alloc((c,), dtype)
+    gx.relu_backward_bias_grad(gb, gy, x, 0.1)
+    hip.sum_to(gx, plain)
+    assert bits_equal(gb.to_numpy(), plain.to_numpy())
+
+
 def test_relu_backward_bias_grad_views_and_errors(hip):
     """strided operands take the two-call road with the same results; shape errors and a bias gradient
     inside the gradient are refused"""

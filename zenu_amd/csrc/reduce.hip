@@ -1117,8 +1117,9 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
         // One or two column tiles over many rows: hundreds of workgroups hand over to one or two that fold them.  Tiles of a
         // quarter of the width have fewer splits each (column sums of [30000,65] f32 16.4 -> 8.2 us, [10007,127]
         // 11.6 -> 7.4, [65536,128] 22 -> 11; f64 [30000,33] 13.2 -> 7.9).  Larger sources stream better in wide rows
-        // ([65537,101] f64, 53 MB, 18.3 against 23; [65537,127] f32, 33 MB, 28 -> 18).
-        if (v == VEC && !pre_x && shift > 3 && outer * tiles_at(shift) <= 2 && R > 1024 && bytes < (sizeof(T) == 4 ? 2 * kStreamBytes : kStreamBytes / 2)) shift = 3;
+        // ([65537,101] f64, 53 MB, 18.3 against 23; [65537,127] f32, 33 MB, 28 -> 18).  With the ReLU gradient on the loads too,
+        // whose sums are the plain ones' bits ([10007,128] f32 12.8 -> 8.9 us, [65536,128] 34 -> 22).
+        if (v == VEC && shift > 3 && outer * tiles_at(shift) <= 2 && R > 1024 && bytes < (sizeof(T) == 4 ? 2 * kStreamBytes : kStreamBytes / 2)) shift = 3;
         // A small source with a short reduced axis is bound by latencies, and the hand-off of a split
         // (about 3 us) is the longest of them: narrower column tiles (down to 64-byte row pieces, which
         // stream at less than half the rate, but there is little to stream) give more workgroups
