@@ -307,8 +307,10 @@ template <typename T, int VEC> __device__ __forceinline__ void store_some(T *p, 
 }
 
 // Rows that 256 threads hold in four vectors each, single elements with VEC == 1: without the slots of the general
-// kernel below, whose bookkeeping costs 5 - 9 % on long rows (f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
+// kernel below, whose bookkeeping costs 5 - 9 % on long rows (both with streaming stores: f32 [8192,4096] 46.5 against 48.7 us, [16384,2048]
 // 44.7 / 48.7; even at [32768,1024], 61 - 63) and more where a launch is a few microseconds; whole_row_vector says which rows come here.
+// NT: streamed loads; the result is written through and not past the caches ([8192,4096] 43.8 us against 45.8, the
+// backward pass that reads it 58.9 against 65.2).
 template <typename T, bool CE, bool NT, int VEC>
 __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, T *y, int64_t R, const T *target, T *rowloss,
                                                                      zmath::ExpLog<T> ml)
@@ -366,7 +368,7 @@ __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, 
                     v[k].v[j] = decltype(by_reciprocal)::value ? quotient<T>(v[k].v[j], sum, rcp) : v[k].v[j] / sum;
                     if (CE) acc = acc + tg[k].v[j] * ml.log(v[k].v[j]);
                 }
-                if constexpr (NT && !CE) store_pack_wt<T, VEC>(yr + r, v[k]);
+                if constexpr (NT && !CE) store_pack_through<T, VEC>(yr + r, v[k]);
                 else store_pack<T, VEC, false>(yr + r, v[k]);
             }
         }
@@ -382,14 +384,15 @@ __global__ __launch_bounds__(kBlock) void softmax_whole_rows_kernel(const T *x, 
 // The softmax axis is the last one: LANES threads hold a row in registers, EPT elements each, and read and write
 // it once (a wavefront takes a row of its own when LANES == 64).  LONG: the row is longer than that; what is
 // beyond the registers is read three times and its exponentials are computed twice, from and into the same place.
-// Bound by memory and, f32, by the 11 f64 operations of an exp: [2048,32003] f32 108 us (524 MB, 4.8 TB/s), 329 when
+// Bound by memory and, f32, by the 11 f64 operations of an exp: [2048,32003] f32 106 us (524 MB, 4.9 TB/s), 329 when
 // the row was walked three times with scalar accesses.  One workgroup of 1024 threads per CU takes 146 us: loading,
 // exp and storing follow each other; two of 512 threads with 64 elements each overlap theirs.
-template <typename T, bool CE, bool NT, bool LONG, int LANES, int EPT>
+template <typename T, bool CE, bool NT, int STORE, bool LONG, int LANES, int EPT>
 __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void softmax_rows_kernel(const T *x, T *y, int64_t rows, int64_t R,
                                                                                   const T *target, T *rowloss,
                                                                                   zmath::ExpLog<T> ml)
 {
+    // STORE: how the rows are written, see softmax_forward_launch
     // (ml arrives as an argument so that the f64 constants of exp / log sit in scalar registers; written
     // as literals each is copied into a register pair per use, and this kernel is bound by its scalar
     // instructions: the branch-free exp for the same reason)
@@ -503,8 +506,8 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES, EPT == 64 ? 4 : 1) void 
                 // the CE output is read again by the backward pass; plain softmax is one stream in, one out
                 if (active)
                     store_slot<T, VEC>(yr, slot, v[k], [](T *row, int at, const Pack<T, VEC> &z) {
-                        if constexpr (NT && !CE) store_pack_wt_at<T, VEC>(row, at, z);
-                        else store_pack<T, VEC, false>(row + at, z);
+                        if constexpr (STORE == kStorePlain) store_pack<T, VEC, false>(row + at, z);
+                        else store_pack_wt_at<T, VEC, STORE == kStoreStream>(row, at, z);
                     });
             }
         }
@@ -615,7 +618,8 @@ __global__ __launch_bounds__(kBlock) void softmax_bwd_long_lines_kernel(const T 
 }
 
 // Rows in registers, as in softmax_rows_kernel: y and y * gy are held, two reads and one write.  LONG: what is
-// beyond the registers is read twice.  [2048,32003] f32 134 us (787 MB, 5.9 TB/s), 311 with scalar accesses
+// beyond the registers is read twice.  [2048,32003] f32 126 us (787 MB, 6.2 TB/s; 137 when y had been written past the
+// caches), 311 with scalar accesses
 // and t written out and read back.
 template <typename T, bool CE, bool NT, bool LONG, int LANES, int EPT>
 __global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void softmax_bwd_rows_kernel(const T *y, const T *gy_or_target, T *gx,
@@ -1130,8 +1134,27 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
             constexpr int B = L < 256 ? 256 : L;
             const int64_t grid = (lines + B / L - 1) / (B / L);
             if (!grid_ok(grid)) return ZENU_ERR_UNSUPPORTED;
-            if (nt) softmax_rows_kernel<T, CE, true, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(x, y, lines, g.R, target, rowloss, zmath::ExpLog<T>());
-            else    softmax_rows_kernel<T, CE, false, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(x, y, lines, g.R, target, rowloss, zmath::ExpLog<T>());
+            auto go = [&](auto nt_c, auto store_c) {
+                softmax_rows_kernel<T, CE, decltype(nt_c)::value, decltype(store_c)::value, LONG, L, E><<<(unsigned)grid, B, 0, s>>>(
+                    x, y, lines, g.R, target, rowloss, zmath::ExpLog<T>());
+            };
+            if (!nt) {
+                go(std::false_type(), std::integral_constant<int, kStorePlain>());
+            } else if constexpr (CE || LONG) {   // (the loss's probabilities are read again by its backward pass; a long row's by itself)
+                go(std::true_type(), std::integral_constant<int, kStorePlain>());
+            } else {
+                // How a streamed row is stored (us, softmax / the backward pass that reads it again): past the caches (`sc1
+                // nt`) the ragged ends of rows, lines that two rows share, are written in part, and a burst of whole rows
+                // meets a busy memory.  Plainly [4096,4003] f32 takes 28 / 32 (35 / 34 past the caches, 35 / 31 written
+                // through), [2048,32003] 106 / 126 (112 / 137), [2048,4003] f64 27 / 32 (32 / 34).  Whole rows are written
+                // through: [4096,16384] 91 / 119 (99 / 134; 89 / 126 plainly), [1024,16000] 25 / 32 (24 / 35; 26 / 32).  A
+                // small result, or one batch of workgroups, still waits at its end for what is dirty in the L2 then:
+                // [300,32003] 27 us plainly, 25 past the caches, [16384,300] 15.8 and 14.2.
+                if (L >= 512 && whole) go(std::true_type(), std::integral_constant<int, L >= 512 ? kStoreThrough : kStorePlain>());
+                else if (lines >= 4 * (int64_t)device_info().num_cus && lines * g.R * (int64_t)sizeof(T) >= kStreamBytes)
+                    go(std::true_type(), std::integral_constant<int, kStorePlain>());
+                else go(std::true_type(), std::integral_constant<int, kStoreStream>());
+            }
             return ZENU_OK;
         });
         if (rc) return rc;
@@ -1169,7 +1192,9 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
             });
         }
     } else {
-        const bool nt = lines * g.R * (int64_t)sizeof(T) * 3 >= kStreamBytes;
+        // y was written just before: loads without the hint find what the caches still hold of it ([4096,1000] f32 10.3 us
+        // with the hint, 8.9 without; [16384,300] 11.9 / 9.7; level at 33 MB a tensor)
+        const bool nt = lines * g.R * (int64_t)sizeof(T) >= kStreamBytes;
         const int rc = with_row_shape<VecOf<T>::N, kMost<T>>(g.R, [&](auto lanes, auto ept, auto is_long) -> int {
             constexpr int L = decltype(lanes)::value, E = decltype(ept)::value;
             constexpr bool LONG = decltype(is_long)::value;

@@ -66,18 +66,33 @@ template <typename T, int N> __device__ __forceinline__ void store_pack_wt(T *p,
     asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(reinterpret_cast<V *>(p)), "v"(x) : "memory");
 }
 
-// the same at row + at, `row` being the same in the whole wavefront and 0 <= at * sizeof(T) < 2^31: one address
-// register.  The five wait states in front are what a memory instruction needs after a vector instruction has written
-// one of its scalar registers (v_readfirstlane, or v_readlane where a spilled one is taken back); the compiler counts
-// them for instructions of its own only, so without them a store right behind would go to the register's old address.
-template <typename T, int N> __device__ __forceinline__ void store_pack_wt_at(T *row, int at, const Pack<T, N> &r)
+// Written through without the streaming hint (`sc1`): the line goes to memory at once, nothing is left to be written back
+// at the end of the kernel, and the next kernel finds it in the memory-side cache (256 MB).
+template <typename T, int N> __device__ __forceinline__ void store_pack_through(T *p, const Pack<T, N> &r)
 {
     static_assert(sizeof(T) * N == 16, "128-bit packs only");
     typedef typename NativeVec<T, N>::type V;
     V x;
     __builtin_memcpy(&x, &r, sizeof(V));
-    asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" ::"v"(at * (int)sizeof(T)), "v"(x), "s"(row) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(reinterpret_cast<V *>(p)), "v"(x) : "memory");
 }
+
+// the same at row + at, `row` being the same in the whole wavefront and 0 <= at * sizeof(T) < 2^31: one address
+// register.  The five wait states in front are what a memory instruction needs after a vector instruction has written
+// one of its scalar registers (v_readfirstlane, or v_readlane where a spilled one is taken back); the compiler counts
+// them for instructions of its own only, so without them a store right behind would go to the register's old address.
+template <typename T, int N, bool NT = true> __device__ __forceinline__ void store_pack_wt_at(T *row, int at, const Pack<T, N> &r)
+{
+    static_assert(sizeof(T) * N == 16, "128-bit packs only");
+    typedef typename NativeVec<T, N>::type V;
+    V x;
+    __builtin_memcpy(&x, &r, sizeof(V));
+    if constexpr (NT) asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" ::"v"(at * (int)sizeof(T)), "v"(x), "s"(row) : "memory");
+    else asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" ::"v"(at * (int)sizeof(T)), "v"(x), "s"(row) : "memory");
+}
+
+// how a kernel with a choice stores: write-back, written through (`sc1`), written through and streaming (`sc1 nt`)
+enum { kStorePlain, kStoreThrough, kStoreStream };
 
 template <typename T, int N> __device__ __forceinline__ Pack<T, N> splat(T s)
 {
