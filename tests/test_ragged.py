@@ -311,3 +311,31 @@ def test_sums_over_images_and_pixels_are_exact(hip, dtype, shape):
         out = offset_matrix(hip, np.full((1, c, 1), 7, dtype), 1)
         hip.sum_to(offset_matrix(hip, x, off), out)
         same(out.to_numpy(), exp, (shape, off))
+
+
+# rows that don't start at cache lines, in column tiles that are dealt to the XCDs in bands: one tile, fewer tiles than
+# XCDs, a number of them that 8 does not divide; one workgroup per tile and several; the gradient on the loads
+BANDS = [(1, 40, 36), (1, 300, 1404), (1, 1000, 1500), (1, 2100, 1004), (5, 33, 1004), (3, 1100, 716), (1, 9, 4100)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", BANDS, ids=str)
+def test_column_tiles_that_share_cache_lines_are_exact(hip, dtype, shape):
+    """small integers: every order of the sums gives the same value"""
+    outer, rows, cols = shape
+    r = np.random.default_rng(cols)
+    a = r.integers(-8, 9, shape).astype(dtype)
+    for off in (0, 1, 4):
+        m = offset_matrix(hip, a, off)
+        same(m.sum(1).to_numpy().reshape(outer, cols), a.sum(axis=1), (shape, off, "sum"))
+        same(np.array(m.max_axis_idx_ravel(1)).reshape(outer, cols), a.argmax(axis=1), (shape, off, "position"))
+    if outer == 1:
+        x = r.integers(-3, 4, (rows, cols)).astype(dtype)
+        gy, gx, gb = (hip.Matrix.from_numpy(t) for t in (a[0], np.zeros((rows, cols), dtype), np.zeros(cols, dtype)))
+        gx.relu_backward_bias_grad(gb, gy, hip.Matrix.from_numpy(x), 0.0)
+        grad = a[0] * np.where(x > 0, dtype(1), dtype(0) * dtype(-1))
+        same(gx.to_numpy(), grad, (shape, "gradient"))
+        same(gb.to_numpy(), grad.sum(axis=0), (shape, "bias gradient"))
+        gy.relu_backward_bias_grad(gb, gy, hip.Matrix.from_numpy(x), 0.0)      # in place
+        same(gy.to_numpy(), grad, (shape, "gradient in place"))
+        same(gb.to_numpy(), grad.sum(axis=0), (shape, "bias gradient in place"))

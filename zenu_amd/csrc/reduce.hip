@@ -330,20 +330,26 @@ __device__ __forceinline__ typename Tr::Acc load_partial(const RedParams<T> &p, 
     return Tr::from_partial(k, i);
 }
 
-// a vector of the source; with PRE the ReLU-gradient transform described at RedParams::pre_x
-template <typename T, int VEC, bool NT, bool PRE>
-__device__ __forceinline__ Pack<T, VEC> load_src(const RedParams<T> &p, const T *ptr)
-{
-    Pack<T, VEC> g = load_pack<T, VEC, NT>(ptr);
-    if constexpr (PRE) {
-        const int64_t off = ptr - p.in;
-        const Pack<T, VEC> x = load_pack<T, VEC, NT>(p.pre_x + off);
-#pragma unroll
-        for (int j = 0; j < VEC; j++) g.v[j] = g.v[j] * ((x.v[j] > (T)0) ? (T)1 : p.pre_alpha * (T)-1);
-        store_pack<T, VEC, NT>(p.pre_out + off, g);
+// A vector of the source; with PRE and its vector of pre_x, turned into the ReLU gradient (RedParams::pre_x) by apply().
+// The loads of a batch come before the first apply(): that stores, and no load moves ahead of a store that might write
+// what it reads, so with the two together every vector of a column kernel's thread waited for the one before
+// ([1000,1500] f32 with the gradient 9.6 us, 8.5 with the loads first; [4096,4096] 44 and 36.5, 201 MB).
+template <typename T, int VEC, bool PRE> struct SrcVec {
+    Pack<T, VEC> g, x;
+    template <bool NT> __device__ __forceinline__ void load(const RedParams<T> &p, const T *ptr)
+    {
+        g = load_pack<T, VEC, NT>(ptr);
+        if constexpr (PRE) x = load_pack<T, VEC, NT>(p.pre_x + (ptr - p.in));
     }
-    return g;
-}
+    template <bool NT> __device__ __forceinline__ void apply(const RedParams<T> &p, const T *ptr)
+    {
+        if constexpr (PRE) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) g.v[j] = g.v[j] * ((x.v[j] > (T)0) ? (T)1 : p.pre_alpha * (T)-1);
+            store_pack<T, VEC, NT>(p.pre_out + (ptr - p.in), g);
+        }
+    }
+};
 
 // ---- hand-off through tagged words ---------------------------------------------------------------------
 // The faster of the two cross-workgroup stages (whole-tensor f32 sum of 128 MiB: 21.5 us against
@@ -637,7 +643,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(RedParams<T> p)
 #define ZENU_FOR_COLS(j) _Pragma("unroll") for (int j = 0; j < VEC; j++) if (j < ncol)
 
 template <typename T, typename Tr, int VEC, bool NT, bool PRE = false>
-__global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uint32_t col_tiles, int tx_shift, int grid3d)
+__global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uint32_t col_tiles, int tx_shift, int grid3d, int banded)
 {
     typedef typename Tr::Acc A;
     __shared__ A lds[kBlock * VEC];
@@ -660,6 +666,19 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
         ct = blk - b1 * col_tiles;
         q_u = b1 / (uint32_t)p.splits;
         split_u = b1 - q_u * (uint32_t)p.splits;
+    }
+    if (banded) {
+        // Workgroup i runs on XCD i mod 8: neighbouring column tiles of rows that do not start at cache lines each read
+        // the line between them, on another XCD.  In bands every XCD takes a run of consecutive tiles and its L2 serves
+        // the second reader (and, with PRE, puts the two halves of the line together).
+        const uint32_t ns = (uint32_t)p.splits, total = col_tiles * ns * gridDim.z;
+        const uint32_t wg = (q_u * ns + split_u) * col_tiles + ct;
+        const uint32_t share = total >> 3, rest = total & 7, xcd = wg & 7;
+        const uint32_t t = xcd * share + (xcd < rest ? xcd : rest) + (wg >> 3);
+        const uint32_t b1 = t / col_tiles;
+        ct = t - b1 * col_tiles;
+        q_u = b1 / ns;
+        split_u = b1 - q_u * ns;
     }
     const int split = (int)split_u;
     const int64_t q = q_u;
@@ -723,20 +742,23 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
             for (int64_t b = split * chunk; b < R; b += p.splits * chunk, ptr += ptr_step) {
                 const int64_t r = b + ty;
                 if (b + chunk <= R) {
-                    Pack<T, VEC> x[U];
+                    SrcVec<T, VEC, PRE> x[U];
 #pragma unroll
-                    for (int u = 0; u < U; u++) x[u] = load_src<T, VEC, NT, PRE>(p, ptr + u * row_step);
+                    for (int u = 0; u < U; u++) x[u].template load<NT>(p, ptr + u * row_step);
 #pragma unroll
                     for (int u = 0; u < U; u++) {
+                        x[u].template apply<NT>(p, ptr + u * row_step);
 #pragma unroll
-                        for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x[u].v[j], r + u * ty_n);
+                        for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x[u].g.v[j], r + u * ty_n);
                     }
                 } else {
                     const T *pt = ptr;
                     for (int64_t rr = r; rr < R; rr += ty_n, pt += row_step) {
-                        Pack<T, VEC> x = load_src<T, VEC, false, PRE>(p, pt);
+                        SrcVec<T, VEC, PRE> x;
+                        x.template load<false>(p, pt);
+                        x.template apply<false>(p, pt);
 #pragma unroll
-                        for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x.v[j], rr);
+                        for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x.g.v[j], rr);
                     }
                 }
             }
@@ -828,19 +850,22 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
     for (int64_t b = (int64_t)split * chunk; b < R; b += (int64_t)splits * chunk) {
         const int64_t r = b + ty;
         if (b + chunk <= R) {
-            Pack<T, VEC> x[U];
+            SrcVec<T, VEC, PRE> x[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) x[u] = load_src<T, VEC, NT, PRE>(p, src + (r + u * TY) * es);
+            for (int u = 0; u < U; u++) x[u].template load<NT>(p, src + (r + u * TY) * es);
 #pragma unroll
             for (int u = 0; u < U; u++) {
+                x[u].template apply<NT>(p, src + (r + u * TY) * es);
 #pragma unroll
-                for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x[u].v[j], r + u * TY);
+                for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x[u].g.v[j], r + u * TY);
             }
         } else {
             for (int64_t rr = r; rr < R; rr += TY) {
-                const Pack<T, VEC> x = load_src<T, VEC, false, PRE>(p, src + rr * es);
+                SrcVec<T, VEC, PRE> x;
+                x.template load<false>(p, src + rr * es);
+                x.template apply<false>(p, src + rr * es);
 #pragma unroll
-                for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x.v[j], rr);
+                for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x.g.v[j], rr);
             }
         }
     }
@@ -1019,6 +1044,12 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
     const int g3 = (p.splits <= 65535 && outer <= 65535) ? 1 : 0;
     const dim3 g = g3 ? dim3((unsigned)col_tiles, (unsigned)p.splits, (unsigned)outer) : dim3((unsigned)grid);
     const uint32_t ctl = (uint32_t)col_tiles;
+    // Column tiles that share cache lines, one XCD per band of them (us, without / with): column sums f64 [10007,1003]
+    // 19.3 / 16.9 (80 MB, 4.8 TB/s), [4001,4001] 30.4 / 26.5, f32 [16384,1003] 18.6 / 16.5, arg-max [4096,4095] 19.1 / 17.6,
+    // [10007,255] 11.3 / 9.7, with the ReLU gradient [1000,1500] 8.46 / 8.21, [300,1404] 5.1 / 4.4.  The index arithmetic
+    // in front of the first load is felt where a small source is split: [1000,999] 6.1 / 6.4.
+    const bool share_lines = reinterpret_cast<uintptr_t>(p.in) % 128 || p.elem_stride * (int64_t)sizeof(T) % 128 || p.outer_stride * (int64_t)sizeof(T) % 128;
+    const int banded = g3 && col_tiles > 1 && share_lines && (p.pre_x || p.splits == 1 || p.nout * p.R * (int64_t)sizeof(T) >= kStreamBytes / 4);
     // the regular geometry: full vector tiles of 32 x 8 threads, a split axis with a flat counter
     const bool regular = g3 && p.cols_vec == VEC && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
     if constexpr (!Tr::kHasIdx && std::is_same<Tr, SumTr<T>>::value) {
@@ -1027,8 +1058,8 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
                 if (nt) reduce_cols_regular_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p);
                 else    reduce_cols_regular_kernel<T, Tr, VEC, false, true><<<g, kBlock, 0, s>>>(p);
             } else {
-                if (nt) reduce_cols_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-                else    reduce_cols_kernel<T, Tr, VEC, false, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+                if (nt) reduce_cols_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
+                else    reduce_cols_kernel<T, Tr, VEC, false, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
             }
             ZENU_LAUNCH_CHECK();
             return ZENU_OK;
@@ -1040,9 +1071,9 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
         ZENU_LAUNCH_CHECK();
         return ZENU_OK;
     }
-    if (p.cols_vec == 1) reduce_cols_kernel<T, Tr, 1, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-    else if (nt)         reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
-    else                 reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3);
+    if (p.cols_vec == 1) reduce_cols_kernel<T, Tr, 1, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
+    else if (nt)         reduce_cols_kernel<T, Tr, VEC, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
+    else                 reduce_cols_kernel<T, Tr, VEC, false><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
     ZENU_LAUNCH_CHECK();
     return ZENU_OK;
 }
