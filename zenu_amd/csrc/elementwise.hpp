@@ -250,6 +250,38 @@ template <typename T> struct CopyF {
     __device__ __forceinline__ T operator()(T a, T) const { return a; }
 };
 
+// ---- how a kernel's operands pass the caches --------------------------------------------------------
+// Below kStreamBytes: no hints.  Above, stores stream (a store that allocates pushes out what the next call reads), and
+//   kMemKeep    inputs are loaded plainly while the call's operands fit the 256 MB memory-side cache: they are often read
+//               again, a data matrix by the next statistic, a forward input by the backward pass.
+//   kMemFeed    a layer's own step, whose result is what the next call reads: ReLU, its backward pass, a bias per channel
+//               or row.  Written through without the hint, it waits in the memory-side cache; the inputs stream.
+//   kMemStream  beyond that everything streams.
+// us with everything streaming / by these rules, three sets of operands in turn: bias, ReLU, NCHW -> NHWC, ReLU backward,
+// bias gradient of [64,512,14,14] f32 53.5 / 47.7 (257 MB moved), [64,256,28,28] 95.8 / 88.2, f64 [16,64,56,56] 54.8 /
+// 49.5; a + row, a * column, a + b^T, 0.5 a of [3001,2047] f32 43.2 / 38.6, [2000,4000] 55.0 / 46.3, [4096,4096] 102.1 /
+// 92.6; ReLU and its backward pass of 8 million 27.9 / 25.7; sigmoid's of 2^24 62.6 / 59.5.
+// Where the lines lie: keeping the inputs of 537 MB calls, ReLU of 2^26 80 / 86 us, backward 128 / 140; feeding from the
+// 201 MB of a ReLU backward of 2^24 31.7 / 33.6, from 154 MB 24.9 / 24.1.
+enum { kMemCached, kMemKeep, kMemFeed, kMemStream };
+constexpr int64_t kKeepBytes = 8 * kStreamBytes, kFeedBytes = 6 * kStreamBytes;
+constexpr bool streams_loads(int mem) { return mem == kMemStream || mem == kMemFeed; }
+
+// ONE_IN: one input streams beside the output (the written-through streaming store, vecmem.hpp)
+template <typename T, int VEC, int MEM, bool ONE_IN> __device__ __forceinline__ void store_mem(T *p, const Pack<T, VEC> &r)
+{
+    if constexpr (VEC == 1 || MEM == kMemCached) store_pack<T, VEC, false>(p, r);
+    else if constexpr (MEM == kMemFeed) store_pack_through<T, VEC>(p, r);
+    else if constexpr (ONE_IN) store_pack_wt<T, VEC>(p, r);
+    else store_pack<T, VEC, true>(p, r);
+}
+
+template <typename F> struct IsLayerStep { static constexpr bool value = false; };
+template <typename T> struct IsLayerStep<ReluF<T>> { static constexpr bool value = true; };
+template <typename T> struct IsLayerStep<ReluBwdF<T>> { static constexpr bool value = true; };
+template <typename F> struct IsAdd { static constexpr bool value = false; };
+template <typename T> struct IsAdd<BinF<T, ZENU_ADD>> { static constexpr bool value = true; };
+
 template <typename T, int N, typename F>
 __device__ __forceinline__ Pack<T, N> apply_pack(const F &f, const Pack<T, N> &a, const Pack<T, N> &b)
 {
@@ -302,7 +334,7 @@ template <typename F> struct ContigShape {
     static constexpr int kUnroll = kSmall ? ZENU_EW1_UNROLL : zenu::kUnroll;
 };
 
-template <typename T, int VEC, bool NT, typename F>
+template <typename T, int VEC, int MEM, typename F>
 __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *out, const T *a, const T *b,
                                                                          int64_t n, F f)
 {
@@ -316,8 +348,8 @@ __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *ou
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
             int64_t i = base + ((int64_t)u * kBlock + tid) * VEC;
-            va[u] = load_pack<T, VEC, NT>(a + i);
-            if constexpr (F::NIN == 2) vb[u] = load_pack<T, VEC, NT>(b + i);
+            va[u] = load_pack<T, VEC, streams_loads(MEM)>(a + i);
+            if constexpr (F::NIN == 2) vb[u] = load_pack<T, VEC, streams_loads(MEM)>(b + i);
             else vb[u] = va[u];
         }
         f.init();   // after the loads are issued: what it fetches (a device scalar, a table) overlaps them
@@ -325,9 +357,7 @@ __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *ou
         for (int u = 0; u < kUnroll; u++) {
             int64_t i = base + ((int64_t)u * kBlock + tid) * VEC;
             const Pack<T, VEC> r = apply_pack<T, VEC, F>(f, va[u], vb[u]);
-            // one streamed input, one streamed output: the written-through streaming store (vecmem.hpp)
-            if constexpr (NT && ContigShape<F>::kSmall && VEC > 1) store_pack_wt<T, VEC>(out + i, r);
-            else store_pack<T, VEC, NT>(out + i, r);
+            store_mem<T, VEC, MEM, ContigShape<F>::kSmall>(out + i, r);
         }
     } else {   // the last tile: whole vectors while they last, then the remaining elements one by one
         f.init();
@@ -362,7 +392,7 @@ __global__ __launch_bounds__(ContigShape<F>::kBlock) void ew_contig_kernel(T *ou
 // flat and aligned however long the row is: [3001,2047] + [2047] f32 takes 9.9 us (5.0 TB/s), 24.4 us when rows of
 // odd length were walked one by one with scalar accesses.)
 
-template <typename T, int VEC, bool NT, typename F, bool Y_FIRST, int MODE, int kBlock, int kUnroll>
+template <typename T, int VEC, int MEM, typename F, bool Y_FIRST, int MODE, int kBlock, int kUnroll>
 __global__ __launch_bounds__(kBlock) void ew_periodic_kernel(T *out, const T *x, const T *y, uint32_t n,
                                                              uint32_t inner, uint32_t mid, F f)
 {
@@ -401,15 +431,14 @@ __global__ __launch_bounds__(kBlock) void ew_periodic_kernel(T *out, const T *x,
         for (int u = 0; u < kUnroll; u++) {
             const uint32_t i0 = base + (uint32_t)(u * kBlock + threadIdx.x) * VEC;
             yv[u] = y_of(i0);
-            if constexpr (F::NIN == 2) xv[u] = load_pack<T, VEC, NT>(x + i0);
+            if constexpr (F::NIN == 2) xv[u] = load_pack<T, VEC, streams_loads(MEM)>(x + i0);
             else xv[u] = yv[u];
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
             const uint32_t i0 = base + (uint32_t)(u * kBlock + threadIdx.x) * VEC;
             const Pack<T, VEC> r = Y_FIRST ? apply_pack<T, VEC, F>(f, yv[u], xv[u]) : apply_pack<T, VEC, F>(f, xv[u], yv[u]);
-            if constexpr (NT && VEC > 1) store_pack_wt<T, VEC>(out + i0, r);   // at most one streamed input beside the output
-            else store_pack<T, VEC, NT>(out + i0, r);
+            store_mem<T, VEC, MEM, true>(out + i0, r);   // at most one streamed input beside the output
         }
     } else {
         for (int u = 0; u < kUnroll; u++) {
@@ -616,7 +645,7 @@ struct TileParams {
     uint32_t tiles_r_magic;     // min(floor(2^32 / tiles_r), 2^32 - 1): x mod tiles_r from one high multiply and a fix-up
 };
 
-template <typename T, bool NT, typename F, bool SMALL = false>
+template <typename T, int MEM, typename F, bool SMALL = false>
 __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_kernel(T *out, const T *a, const T *b,
                                                                                   TileParams p, F f)
 {
@@ -744,8 +773,8 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         for (int k = 0; k < K; k++) {
             const int o = other_of(k);
             const int lane_v = vec_of(k);
-            xa[k] = load_pack<T, VEC, NT>(abase + clip_vec(lane_v, ta) + (int64_t)clip_other(o, ta) * pitch_a);
-            if constexpr (F::NIN == 2) xb[k] = load_pack<T, VEC, NT>(bbase + clip_vec(lane_v, tb) + (int64_t)clip_other(o, tb) * pitch_b);
+            xa[k] = load_pack<T, VEC, streams_loads(MEM)>(abase + clip_vec(lane_v, ta) + (int64_t)clip_other(o, ta) * pitch_a);
+            if constexpr (F::NIN == 2) xb[k] = load_pack<T, VEC, streams_loads(MEM)>(bbase + clip_vec(lane_v, tb) + (int64_t)clip_other(o, tb) * pitch_b);
         }
         if (ta) {
 #pragma unroll
@@ -799,7 +828,7 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
                 if ((r < nr) & (lane_v < nc)) {
                     T *const orow = obase + (int64_t)r * ldr0;
                     if (lane_v + VEC <= nc) {
-                        store_pack<T, VEC, NT>(orow + lane_v, z);
+                        store_mem<T, VEC, MEM, false>(orow + lane_v, z);
                     } else {
                         const int c = clip_vec(lane_v, false);
 #pragma unroll
@@ -808,7 +837,7 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
                     }
                 }
             } else {
-                store_pack<T, VEC, NT>(obase + (int64_t)r * ldr0 + lane_v, z);
+                store_mem<T, VEC, MEM, false>(obase + (int64_t)r * ldr0 + lane_v, z);
             }
         }
     };
@@ -970,8 +999,15 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
     const T *a = static_cast<const T *>(p.ptr[1]);
     const T *b = (F::NIN == 2) ? static_cast<const T *>(p.ptr[2]) : a;
     const int nin = F::NIN;
-    // operands are streamed once: hint the caches when the op is larger than they are
-    const bool nt = p.numel * (int64_t)sizeof(T) * (nin + 1) >= kStreamBytes;
+    const int64_t moved = p.numel * (int64_t)sizeof(T) * (nin + 1);
+    const bool nt = moved >= kStreamBytes;
+    // calls go(mem) with the way past the caches as a constant; feed: see kMemFeed
+    auto with_mem = [&](auto feed, auto go) {
+        constexpr bool FEED = decltype(feed)::value;
+        if (!nt) go(std::integral_constant<int, kMemCached>());
+        else if (moved < (FEED ? kFeedBytes : kKeepBytes)) go(std::integral_constant<int, FEED ? kMemFeed : kMemKeep>());
+        else go(std::integral_constant<int, kMemStream>());
+    };
     if (p.ndim == 0) {  // a single element
         p.ndim = 1;
         p.shape[0] = 1;
@@ -989,7 +1025,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
         if constexpr (kSinglesPerCu<F> > 0) {
             if (n <= kSinglesPerCu<F> * device_info().num_cus) {
                 constexpr int64_t singles = (int64_t)cb * cu;
-                ew_contig_kernel<T, 1, false, F><<<(unsigned)((n + singles - 1) / singles), cb, 0, stream>>>(out, a, b, n, f);
+                ew_contig_kernel<T, 1, kMemCached, F><<<(unsigned)((n + singles - 1) / singles), cb, 0, stream>>>(out, a, b, n, f);
                 ZENU_LAUNCH_CHECK();
                 return ZENU_OK;
             }
@@ -997,8 +1033,9 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
         int64_t tile = (int64_t)cb * VEC * cu;
         int64_t grid = (n + tile - 1) / tile;
         if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
-        if (nt) ew_contig_kernel<T, VEC, true, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
-        else    ew_contig_kernel<T, VEC, false, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
+        with_mem(std::integral_constant<bool, IsLayerStep<F>::value>(), [&](auto mem) {
+            ew_contig_kernel<T, VEC, decltype(mem)::value, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
+        });
         ZENU_LAUNCH_CHECK();
         return ZENU_OK;
     }
@@ -1050,8 +1087,9 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                         constexpr int B = small ? ZENU_EW1_BLOCK : 256, U = small ? ZENU_EW1_UNROLL : 2;
                         const int64_t tile = (int64_t)B * VEC * U;
                         const unsigned grid = (unsigned)((p.numel + tile - 1) / tile);
-                        if (nt) ew_periodic_kernel<T, VEC, true, F, YF, MODE, B, U><<<grid, B, 0, stream>>>(out, x, y, n32, in32, mid32, f);
-                        else    ew_periodic_kernel<T, VEC, false, F, YF, MODE, B, U><<<grid, B, 0, stream>>>(out, x, y, n32, in32, mid32, f);
+                        with_mem(std::integral_constant<bool, IsAdd<F>::value && (MODE == 1 || MODE == 2)>(), [&](auto mem) {
+                            ew_periodic_kernel<T, VEC, decltype(mem)::value, F, YF, MODE, B, U><<<grid, B, 0, stream>>>(out, x, y, n32, in32, mid32, f);
+                        });
                     };
                     auto by_mode = [&](auto yfirst_c) {
                         if (mode == 0) go(yfirst_c, std::integral_constant<int, 0>());
@@ -1229,7 +1267,9 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                                          : dim3((unsigned)tp.tiles_c, (unsigned)tp.tiles_r, (unsigned)tp.nbatch);
                 const size_t lds = (size_t)(tp.trans_a + tp.trans_b) * kTile * (kTile + 1) * sizeof(T);
                 constexpr int kThreads = TileThreads<T, F, SMALL>::value;
-                ew_tile_kernel<T, NT, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
+                if constexpr (!NT) ew_tile_kernel<T, kMemCached, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
+                else if (moved < kKeepBytes) ew_tile_kernel<T, kMemKeep, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
+                else ew_tile_kernel<T, kMemStream, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
                 return ZENU_OK;
             };
             const int rc_tiles = large          ? launch_tiles(std::false_type(), std::true_type())
