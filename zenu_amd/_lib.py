@@ -6,6 +6,11 @@ shared object is missing, loading fails loudly.
 import ctypes as C
 import os
 
+try:
+    from . import _pyhost
+except ImportError as e:
+    raise ImportError("zenu_amd/_pyhost.so is missing: build it with `make -C zenu_amd/csrc` (or __graft_entry__.build())") from e
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libzenu_hip.so")
 
@@ -159,6 +164,7 @@ def lib():
     l.zenu_hip_validated_libm.restype = C.c_char_p
     l.zenu_hip_last_hip_error_string.argtypes = []
     l.zenu_hip_last_hip_error_string.restype = C.c_char_p
+    _pyhost.bind(l._handle)
     _lib = l
     return l
 

@@ -15,7 +15,9 @@ tests read like the reference's own tests:
   copies        copy_from, to_default_stride        copy_from.rs:211-267, to_default_stride.rs:7-15
 
 Where the reference panics, a ZenuHipError is raised (status RANK / SHAPE / AXIS).  Every
-operation is one call into libzenu_hip.so; nothing here computes on the host.
+operation is one call into libzenu_hip.so; nothing here computes on the host.  The calls that programs
+make all the time go through _pyhost (csrc/pyhost.cpp), which says True once it has made the call and
+False for operands that it leaves to ctypes.
 """
 import ctypes as C
 import math
@@ -23,7 +25,7 @@ import struct
 
 import numpy as np
 
-from . import _lib
+from . import _lib, _pyhost
 from ._lib import ZenuHipError, Tensor, check
 
 _stream = None  # hipStream_t as int / None = null stream
@@ -69,6 +71,8 @@ def default_stride(shape):
 
 # zenu_tensor_t by number of dimensions: pointer, ndim, reserved, shape and stride padded to MAX_DIM
 _DESC = [struct.Struct(f"Pi4x{n}q{8 * (_lib.MAX_DIM - n)}x{n}q{8 * (_lib.MAX_DIM - n)}x").pack for n in range(_lib.MAX_DIM + 1)]
+
+_tensor_of = Tensor.from_buffer_copy
 
 
 class DeviceBuffer:
@@ -148,9 +152,12 @@ class Matrix:
 
     def desc(self):
         # packed in one go: a small call is bound by its host side, and a field by field descriptor of two
-        # dimensions takes twice as long (0.74 against 0.39 us, two to four of them per call)
-        shape = self.shape
-        return Tensor.from_buffer_copy(_DESC[len(shape)](self.as_ptr(), len(shape), *shape, *self.stride))
+        # dimensions takes twice as long (0.74 us; 0.39 packed here)
+        data = _pyhost.pack(self)
+        if data is None:
+            shape = self.shape
+            data = _DESC[len(shape)](self.as_ptr(), len(shape), *shape, *self.stride)
+        return _tensor_of(data)
 
     def _view(self, offset, shape, stride):
         """a view of this matrix's memory; offset, shape and stride are integers of Python's own already"""
@@ -202,6 +209,9 @@ class Matrix:
         """swap the last two axes (shape_stride.rs:94-114)"""
         if self.ndim < 2:
             raise ValueError("transpose needs at least 2 dims")
+        view = _pyhost.transpose(self)
+        if view is not None:
+            return view
         shape, stride = list(self.shape), list(self.stride)
         shape[-1], shape[-2] = shape[-2], shape[-1]
         stride[-1], stride[-2] = stride[-2], stride[-1]
@@ -240,13 +250,15 @@ class Matrix:
 
     # ---- copies -------------------------------------------------------------------------
     def copy_from(self, src):
-        check(_lib.lib().zenu_hip_copy(_dt(self.dtype), C.byref(self.desc()), C.byref(src.desc()), _stream),
-              "copy_from")
+        if not _pyhost.copy(self, src, _stream):
+            check(_lib.lib().zenu_hip_copy(_dt(self.dtype), C.byref(self.desc()), C.byref(src.desc()), _stream),
+                  "copy_from")
 
     def broadcast(self, source):
         """broadcast.rs:11-43"""
-        check(_lib.lib().zenu_hip_broadcast(_dt(self.dtype), C.byref(self.desc()), C.byref(source.desc()), _stream),
-              "broadcast")
+        if not _pyhost.broadcast(self, source, _stream):
+            check(_lib.lib().zenu_hip_broadcast(_dt(self.dtype), C.byref(self.desc()), C.byref(source.desc()), _stream),
+                  "broadcast")
 
     def to_default_stride(self):
         out = self.alloc_like()
@@ -258,21 +270,25 @@ class Matrix:
 
     # ---- binary -------------------------------------------------------------------------
     def _binary_array(self, op, lhs, rhs):
-        check(_lib.lib().zenu_hip_binary(op, _dt(self.dtype), C.byref(self.desc()), C.byref(lhs.desc()),
-                                         C.byref(rhs.desc()), _stream), "binary")
+        if not _pyhost.binary(op, self, lhs, rhs, _stream):
+            check(_lib.lib().zenu_hip_binary(op, _dt(self.dtype), C.byref(self.desc()), C.byref(lhs.desc()),
+                                             C.byref(rhs.desc()), _stream), "binary")
 
     def _binary_assign(self, op, rhs):
-        check(_lib.lib().zenu_hip_binary_assign(op, _dt(self.dtype), C.byref(self.desc()),
-                                                C.byref(rhs.desc()), _stream), "binary_assign")
+        if not _pyhost.binary_assign(op, self, rhs, _stream):
+            check(_lib.lib().zenu_hip_binary_assign(op, _dt(self.dtype), C.byref(self.desc()),
+                                                    C.byref(rhs.desc()), _stream), "binary_assign")
 
     def _binary_scalar(self, op, other, scalar):
-        check(_lib.lib().zenu_hip_binary_scalar(op, _dt(self.dtype), C.byref(self.desc()),
-                                                C.byref(other.desc()), float(scalar), _stream),
-              "binary_scalar")
+        if not _pyhost.binary_scalar(op, self, other, scalar, _stream):
+            check(_lib.lib().zenu_hip_binary_scalar(op, _dt(self.dtype), C.byref(self.desc()),
+                                                    C.byref(other.desc()), float(scalar), _stream),
+                  "binary_scalar")
 
     def _binary_scalar_assign(self, op, scalar):
-        check(_lib.lib().zenu_hip_binary_scalar_assign(op, _dt(self.dtype), C.byref(self.desc()),
-                                                       float(scalar), _stream), "binary_scalar_assign")
+        if not _pyhost.binary_scalar_assign(op, self, scalar, _stream):
+            check(_lib.lib().zenu_hip_binary_scalar_assign(op, _dt(self.dtype), C.byref(self.desc()),
+                                                           float(scalar), _stream), "binary_scalar_assign")
 
     def _operator(self, op, rhs):
         if isinstance(rhs, Matrix):
@@ -313,8 +329,9 @@ class Matrix:
 
     # ---- unary --------------------------------------------------------------------------
     def _unary_array(self, fn, other):
-        check(_lib.lib().zenu_hip_unary(fn, _dt(self.dtype), C.byref(self.desc()), C.byref(other.desc()),
-                                        _stream), "unary")
+        if not _pyhost.unary(fn, self, other, _stream):
+            check(_lib.lib().zenu_hip_unary(fn, _dt(self.dtype), C.byref(self.desc()), C.byref(other.desc()),
+                                            _stream), "unary")
 
     def _unary_assign(self, fn):
         check(_lib.lib().zenu_hip_unary_assign(fn, _dt(self.dtype), C.byref(self.desc()), _stream),
@@ -338,8 +355,9 @@ class Matrix:
         return self._unary(_lib.SIGMOID)
 
     def relu(self, other, alpha):
-        check(_lib.lib().zenu_hip_relu(_dt(self.dtype), C.byref(self.desc()), C.byref(other.desc()),
-                                       float(alpha), _stream), "relu")
+        if not _pyhost.relu(self, other, alpha, _stream):
+            check(_lib.lib().zenu_hip_relu(_dt(self.dtype), C.byref(self.desc()), C.byref(other.desc()),
+                                           float(alpha), _stream), "relu")
 
     def relu_backward_mask(self, other, alpha):
         check(_lib.lib().zenu_hip_relu_backward_mask(_dt(self.dtype), C.byref(self.desc()),
@@ -348,25 +366,29 @@ class Matrix:
 
     def tanh_backward(self, gy, x):
         """self = gy / cosh(x)^2: zenu-autograd/src/functions/tanh.rs:30-37 in one pass"""
-        check(_lib.lib().zenu_hip_tanh_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
-                                                C.byref(x.desc()), _stream), "tanh_backward")
+        if not _pyhost.tanh_backward(self, gy, x, _stream):
+            check(_lib.lib().zenu_hip_tanh_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
+                                                    C.byref(x.desc()), _stream), "tanh_backward")
 
     def sigmoid_backward(self, gy, x):
         """self = d sigmoid(x) * gy with the roundings of the autograd chain (activation/sigmoid.rs:7-15)"""
-        check(_lib.lib().zenu_hip_sigmoid_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
-                                                   C.byref(x.desc()), _stream), "sigmoid_backward")
+        if not _pyhost.sigmoid_backward(self, gy, x, _stream):
+            check(_lib.lib().zenu_hip_sigmoid_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
+                                                       C.byref(x.desc()), _stream), "sigmoid_backward")
 
     def relu_backward(self, gy, x, alpha):
         """self = gy * relu_backward_mask(x): zenu-autograd/src/activation/relu.rs:35-44 in one pass"""
-        check(_lib.lib().zenu_hip_relu_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
-                                                C.byref(x.desc()), float(alpha), _stream), "relu_backward")
+        if not _pyhost.relu_backward(self, gy, x, alpha, _stream):
+            check(_lib.lib().zenu_hip_relu_backward(_dt(self.dtype), C.byref(self.desc()), C.byref(gy.desc()),
+                                                    C.byref(x.desc()), float(alpha), _stream), "relu_backward")
 
     def relu_backward_bias_grad(self, gbias, gy, x, alpha):
         """self = gy * relu'(x) and gbias = the column sums of self (the bias gradient of the layer
         before), in one pass over gy"""
-        check(_lib.lib().zenu_hip_relu_backward_bias_grad(_dt(self.dtype), C.byref(self.desc()), C.byref(gbias.desc()),
-                                                          C.byref(gy.desc()), C.byref(x.desc()), float(alpha), _stream),
-              "relu_backward_bias_grad")
+        if not _pyhost.relu_backward_bias_grad(self, gbias, gy, x, alpha, _stream):
+            check(_lib.lib().zenu_hip_relu_backward_bias_grad(_dt(self.dtype), C.byref(self.desc()), C.byref(gbias.desc()),
+                                                              C.byref(gy.desc()), C.byref(x.desc()), float(alpha), _stream),
+                  "relu_backward_bias_grad")
 
     # ---- clip (zenu-matrix/src/operation/clip.rs:289-318) -----------------------------------
     def clip(self, lo, hi):
@@ -394,14 +416,16 @@ class Matrix:
         """softmax.rs:10-25, one launch"""
         if not (0 <= axis < self.ndim):
             raise ZenuHipError(_lib.ERR_AXIS, "softmax_assign", "axis must be less than the number of dimensions")
-        check(_lib.lib().zenu_hip_softmax(_dt(self.dtype), C.byref(self.desc()), C.byref(source.desc()),
-                                          axis, _stream), "softmax_assign")
+        if not _pyhost.softmax(self, source, axis, _stream):
+            check(_lib.lib().zenu_hip_softmax(_dt(self.dtype), C.byref(self.desc()), C.byref(source.desc()),
+                                              axis, _stream), "softmax_assign")
 
     def bias_add_relu(self, z, bias, alpha, pre=None):
         """self = relu(z + bias, alpha); pre (optional) receives z + bias"""
-        check(_lib.lib().zenu_hip_bias_add_relu(_dt(self.dtype), C.byref(pre.desc()) if pre is not None else None,
-                                                C.byref(self.desc()), C.byref(z.desc()), C.byref(bias.desc()),
-                                                float(alpha), _stream), "bias_add_relu")
+        if not _pyhost.bias_add_relu(self, z, bias, alpha, pre, _stream):
+            check(_lib.lib().zenu_hip_bias_add_relu(_dt(self.dtype), C.byref(pre.desc()) if pre is not None else None,
+                                                    C.byref(self.desc()), C.byref(z.desc()), C.byref(bias.desc()),
+                                                    float(alpha), _stream), "bias_add_relu")
 
     # ---- reductions ---------------------------------------------------------------------
     def sum(self, axis, keep_dim=False):
@@ -636,5 +660,9 @@ def split(matrix, axis, num_splits):
 
 def sum_to(source, target):
     """sum.rs:35-94: reduce `source` into the (smaller) `target` in place"""
-    check(_lib.lib().zenu_hip_sum_to(_dt(source.dtype), C.byref(target.desc()), C.byref(source.desc()),
-                                     _stream), "sum_to")
+    if not _pyhost.sum_to(source, target, _stream):
+        check(_lib.lib().zenu_hip_sum_to(_dt(source.dtype), C.byref(target.desc()), C.byref(source.desc()),
+                                         _stream), "sum_to")
+
+
+_pyhost.setup(Matrix, C.c_void_p, np.dtype(np.float32), np.dtype(np.float64), check)
