@@ -339,3 +339,30 @@ def test_column_tiles_that_share_cache_lines_are_exact(hip, dtype, shape):
         gy.relu_backward_bias_grad(gb, gy, hip.Matrix.from_numpy(x), 0.0)      # in place
         same(gy.to_numpy(), grad, (shape, "gradient in place"))
         same(gb.to_numpy(), grad.sum(axis=0), (shape, "bias gradient in place"))
+
+
+# runs of one element less than a vector to one more than the kernel for a short side takes, last workgroups of 1 .. 64 positions,
+# sizes on both sides of the line below which square tiles take the copy
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", [(130, 1, 64), (129, 2, 65), (17, 3, 1023), (3, 3, 4097), (9, 4, 1024), (33, 5, 259), (1, 7, 9001), (140, 16, 67),
+                                   (86, 23, 96), (2, 24, 4161), (2, 24, 4096), (40, 25, 300), (300, 3, 49)], ids=str)
+def test_copies_with_one_short_side(hip, dtype, shape):
+    r = np.random.default_rng(shape[2])
+    n, short, long = shape
+    for off in (0, 1):
+        a = r.standard_normal(shape).astype(dtype)
+        A = offset_matrix(hip, a, off)
+        out = offset_matrix(hip, np.full((n, long, short), 7, dtype), 3 - off)
+        out.copy_from(A.transpose())
+        same(out.to_numpy(), a.transpose(0, 2, 1), ("into the short side", shape, off))
+        back = offset_matrix(hip, np.full(shape, 7, dtype), off)
+        back.copy_from(out.transpose())
+        same(back.to_numpy(), a, ("out of it", shape, off))
+        # runs that are part of longer ones, on either side; nothing else is written
+        wide = hip.Matrix.from_numpy(np.full((n, short, long + 5), 7, dtype))
+        wide.slice(slice(0, n), slice(0, short), slice(2, long + 2)).copy_from(out.transpose())
+        exp = np.full((n, short, long + 5), 7, dtype)
+        exp[:, :, 2:long + 2] = a
+        same(wide.to_numpy(), exp, ("into part of longer runs", shape, off))
+        out.copy_from(wide.slice(slice(0, n), slice(0, short), slice(1, long + 1)).transpose())
+        same(out.to_numpy(), exp[:, :, 1:long + 1].transpose(0, 2, 1), ("from part of longer runs", shape, off))

@@ -279,6 +279,8 @@ template <typename T, int VEC, int MEM, bool ONE_IN> __device__ __forceinline__ 
 template <typename F> struct IsLayerStep { static constexpr bool value = false; };
 template <typename T> struct IsLayerStep<ReluF<T>> { static constexpr bool value = true; };
 template <typename T> struct IsLayerStep<ReluBwdF<T>> { static constexpr bool value = true; };
+template <typename F> struct IsCopy { static constexpr bool value = false; };
+template <typename T> struct IsCopy<CopyF<T>> { static constexpr bool value = true; };
 template <typename F> struct IsAdd { static constexpr bool value = false; };
 template <typename T> struct IsAdd<BinF<T, ZENU_ADD>> { static constexpr bool value = true; };
 
@@ -910,6 +912,124 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
     }
 }
 
+// ---- kernel 3b: transposed copies with one short side ------------------------------------------------
+// Images with few channels between NCHW and NHWC, the weights of a small head: a [long][short] matrix without gaps on
+// one side, `nshort` runs of it `pitch` apart on the other.  Square tiles are mostly padding there (3 of 32 columns) and
+// their accesses single elements.  Here a workgroup takes 2^log_run positions of all runs, 16 KB: vectors on both sides,
+// turned in LDS, where run s starts at s * lds_pitch: 64 / nshort banks (rounded to whole vectors) from the one before,
+// so that the elements of a wavefront's vectors, nshort runs by 64 / nshort positions, lie in different banks.
+// THIN_OUT: the side without gaps is the output.
+struct ThinParams {
+    OuterDesc outer;
+    int64_t nlong, pitch;
+    int nshort, log_run, lds_pitch;
+    uint32_t magic;             // ceil(2^20 / nshort): e / nshort = e * magic >> 20 where e * nshort <= 2^20
+};
+constexpr int kThinBytes = 16384, kThinVecs = kThinBytes / 16 / kBlock;   // per workgroup; vectors per thread
+// us of square tiles / this kernel, into [long][short] and out of it, f32: [128,3,12544] 59 / 7.2 and 53 / 7.4 (39 MB,
+// 5.3 TB/s), [64,8,3136] 8.5 / 4.2 and 8.4 / 4.8, [32,16,3136] 5.9 / 4.2 and 5.7 / 4.7, [8,24,12544] 6.1 / 5.1 and 6.1 /
+// 5.7; f64: [128,3,12544] 50 / 12.4 (77 MB, 6.2 TB/s), [8,24,12544] 11.4 / 7.2.  From runs of 28 on they are level, whole
+// tiles of 32 are faster (f64 [64,32,784] 6.0 / 6.8), and so are tiles of a few thousand positions, where the divisions
+// show: [10,4096] 2.2 / 2.6, [14,1497] 2.3 / 2.6.
+constexpr int64_t kThinMax = 24, kThinPositions = 8192;
+
+template <typename T, int MEM, bool THIN_OUT>
+__global__ __launch_bounds__(kBlock) void ew_thin_kernel(T *out, const T *in, ThinParams p)
+{
+    constexpr int VEC = VecOf<T>::N, LV = VEC == 4 ? 2 : 1;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    T *const lds = reinterpret_cast<T *>(lds_raw);
+    const int tid = threadIdx.x, S = p.nshort, run = 1 << p.log_run, K = p.lds_pitch;
+    int64_t oo, oi, unused;
+    decompose32(p.outer, blockIdx.y, oo, oi, unused);
+    const int64_t p0 = (int64_t)blockIdx.x << p.log_run;
+    const int n = p.nlong - p0 < run ? (int)(p.nlong - p0) : run;   // positions of this workgroup
+    const int vecs = S << (p.log_run - LV);
+    const int flat = n * S;                                         // elements of the side without gaps
+    const int64_t gapless = p0 * S;
+    auto run_of = [&](int v) { return v >> (p.log_run - LV); };
+    auto pos_of = [&](int v) { return (v << LV) & (run - 1); };
+    auto spot = [&](int e) {                                        // element e of the side without gaps
+        const int at = (int)(((uint32_t)e * p.magic) >> 20);
+        return (e - at * S) * K + at;
+    };
+    Pack<T, VEC> x[kThinVecs];
+    if constexpr (THIN_OUT) {
+        // a vector past the end of its run is moved back to end with it (nlong >= VEC)
+        const T *const src = in + oi + p0;
+        const int64_t last = p.nlong - VEC - p0;
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int v = k * kBlock + tid;
+            if (v < vecs) x[k] = load_pack<T, VEC, streams_loads(MEM)>(src + run_of(v) * p.pitch + (pos_of(v) < last ? pos_of(v) : last));
+        }
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int v = k * kBlock + tid;
+            if (v >= vecs) continue;
+            T *const row = lds + run_of(v) * K;
+            if (pos_of(v) <= last) {
+                store_pack<T, VEC, false>(row + pos_of(v), x[k]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; j++)
+                    if (last + j >= 0) row[(int)last + j] = x[k].v[j];
+            }
+        }
+        __syncthreads();
+        T *const dst = out + oo + gapless;
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int e = (k * kBlock + tid) * VEC;
+            if (e >= flat) continue;
+#pragma unroll
+            for (int j = 0; j < VEC; j++) x[k].v[j] = lds[spot(e + j < flat ? e + j : e)];
+            if (e + VEC <= flat) {
+                store_mem<T, VEC, MEM, true>(dst + e, x[k]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; j++)
+                    if (e + j < flat) dst[e + j] = x[k].v[j];
+            }
+        }
+    } else {
+        const T *const src = in + oi + gapless;
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int e = (k * kBlock + tid) * VEC;
+            if (e + VEC <= flat) {
+                x[k] = load_pack<T, VEC, streams_loads(MEM)>(src + e);
+            } else if (e < flat) {
+#pragma unroll
+                for (int j = 0; j < VEC; j++) x[k].v[j] = src[e + j < flat ? e + j : e];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int e = (k * kBlock + tid) * VEC;
+#pragma unroll
+            for (int j = 0; j < VEC; j++)
+                if (e + j < flat) lds[spot(e + j)] = x[k].v[j];
+        }
+        __syncthreads();
+        T *const dst = out + oo + p0;
+#pragma unroll
+        for (int k = 0; k < kThinVecs; k++) {
+            const int v = k * kBlock + tid;
+            if (v >= vecs || pos_of(v) >= n) continue;
+            const Pack<T, VEC> z = load_pack<T, VEC, false>(lds + run_of(v) * K + pos_of(v));
+            T *const row = dst + run_of(v) * p.pitch + pos_of(v);
+            if (pos_of(v) + VEC <= n) {
+                store_mem<T, VEC, MEM, true>(row, z);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; j++)
+                    if (pos_of(v) + j < n) row[j] = z.v[j];
+            }
+        }
+    }
+}
+
 // ---- kernel 4: strided rows (anything else) ----------------------------------------------------------
 // Operands whose innermost (collapsed) dim has any stride: a strided destination (out[:, ::2] = ...),
 // gathers (a[:, ::2] + b), views without a unit-stride dim.  The threads of a workgroup form
@@ -1208,6 +1328,35 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
             }
             tp.trans_a = trans[1];
             tp.trans_b = nin == 2 ? trans[2] : 0;
+            // a short side, the output's rows or the input's: see ew_thin_kernel
+            if constexpr (IsCopy<F>::value) {
+                const bool thin_out = tp.C <= kThinMax && tp.ldr[0] == tp.C && tp.R >= 64;
+                const bool thin_in = tp.R <= kThinMax && tp.ldc[1] == tp.R && tp.C >= 64;
+                if ((thin_out || thin_in) && tp.nbatch <= 65535 && tp.nbatch * (thin_out ? tp.R : tp.C) > kThinPositions) {
+                    ThinParams q;
+                    q.outer = tp.outer;
+                    q.nlong = thin_out ? tp.R : tp.C;
+                    q.pitch = thin_out ? tp.ldc[1] : tp.ldr[0];
+                    q.nshort = (int)(thin_out ? tp.C : tp.R);
+                    q.magic = ((1u << 20) + (uint32_t)q.nshort - 1) / (uint32_t)q.nshort;
+                    // positions per workgroup: what fills its 16 KB, less where the chip would stay empty
+                    q.log_run = 6;
+                    while ((int64_t)q.nshort * (int64_t)sizeof(T) << (q.log_run + 1) <= kThinBytes) q.log_run++;
+                    while (q.log_run > 6 && tp.nbatch * ((q.nlong + ((int64_t)1 << q.log_run) - 1) >> q.log_run) < 4 * (int64_t)device_info().num_cus) q.log_run--;
+                    const int64_t tiles = (q.nlong + ((int64_t)1 << q.log_run) - 1) >> q.log_run;
+                    q.lds_pitch = (1 << q.log_run) + ((64 / q.nshort + 3) & ~3);
+                    if (tiles <= 0x7fffffffLL) {
+                        const dim3 g((unsigned)tiles, (unsigned)tp.nbatch);
+                        const size_t lds = (size_t)q.nshort * q.lds_pitch * sizeof(T);
+                        with_mem(std::false_type(), [&](auto mem) {
+                            if (thin_out) ew_thin_kernel<T, decltype(mem)::value, true><<<g, kBlock, lds, stream>>>(out, a, q);
+                            else          ew_thin_kernel<T, decltype(mem)::value, false><<<g, kBlock, lds, stream>>>(out, a, q);
+                        });
+                        ZENU_LAUNCH_CHECK();
+                        return ZENU_OK;
+                    }
+                }
+            }
             bool vec = true;
             // the vector path reads whole vectors along C from the inputs that are not transposed: one
             // that is broadcast along C (a column beside a transposed operand) takes the element path
