@@ -225,6 +225,23 @@ def test_softmax_kernel_edges(hip, dtype, shape):
     assert np.all(ends[:2] == 0) and np.all(ends[-5:] == 7)
 
 
+# rows that are turned in LDS: odd and even lengths, one to eight wavefronts a row, a last workgroup of 1 .. 63 rows, the line
+# between them and the direct kernel; lines of which y is read twice (f64 beyond 256 elements)
+STAGED_SHAPES = [(1, 40, 1), (64, 33, 1), (65, 34, 1), (257, 64, 1), (321, 63, 1), (32767, 8, 1), (32769, 8, 1), (30001, 9, 1), (16385, 16, 1),
+                 (20001, 31, 1), (9000, 32, 1), (33000, 7, 1), (3, 257, 65), (2, 288, 64), (1, 289, 130), (2, 511, 33), (1, 512, 70)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", STAGED_SHAPES, ids=str)
+def test_softmax_staged_rows(hip, dtype, shape):
+    test_softmax_kernel_edges(hip, dtype, shape)
+    x = np.random.default_rng(1).standard_normal(shape).astype(dtype)
+    m, out = hip.Matrix.from_numpy(x), hip.Matrix.from_numpy(np.zeros_like(x))
+    out.softmax_assign(m, 1)
+    m.softmax_assign(m, 1)                                 # in place
+    assert np.array_equal(m.to_numpy(), out.to_numpy())
+
+
 # Rows for the exact test below: few and many, around each limit of a wavefront, of 256 threads (single elements and
 # vectors) and of larger workgroups, totals below and above the streaming size.  Powers of two of them, see below.
 EXACT_ROWS = [(4, 65), (512, 127), (1024, 128), (2048, 255), (512, 256), (1024, 300), (512, 511), (2048, 512), (2048, 513), (4, 600),

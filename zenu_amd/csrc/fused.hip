@@ -91,7 +91,8 @@ template <typename T> __device__ __forceinline__ T quotient(T a, T sum, T rcp)
 // lines, wavefront w of them holds elements [w OWN, (w + 1) OWN) of each of its lines in registers.
 struct LineSpot {
     int64_t line, base;   // base: offset of the line's element 0 (of line 0 past the end)
-    int w, group;
+    int64_t first;        // the workgroup's first line
+    int w, group, lines_here;
     bool active;
     __device__ __forceinline__ LineSpot(int64_t lines, int64_t R, int64_t inner, int waves)
     {
@@ -99,7 +100,9 @@ struct LineSpot {
         group = wave / waves;
         w = wave - group * waves;
         const int groups = (int)(blockDim.x >> 6) / waves;
-        line = ((int64_t)blockIdx.x * groups + group) * 64 + (threadIdx.x & 63);
+        first = (int64_t)blockIdx.x * groups * 64;
+        lines_here = (int)min((int64_t)groups * 64, lines - first);
+        line = first + group * 64 + (threadIdx.x & 63);
         active = line < lines;
         const int64_t l = active ? line : 0;
         if (inner == 1) {
@@ -131,6 +134,61 @@ __device__ __forceinline__ T sum_in_order(const T (&x)[OWN], int valid, const Li
     return waves > 1 ? *mine : sum;
 }
 
+// Rows of the last axis with a lane per row: a wavefront's accesses would lie a row apart, 64 lines of the cache for 4
+// or 8 bytes each.  The rows of a workgroup are one piece of memory: it is read and written in vectors, OWN elements
+// per thread, and turned in LDS, where rows start an odd number of elements apart.
+template <typename T, int OWN> struct StagedRows {
+    static constexpr int VEC = VecOf<T>::N;
+    Pack<T, VEC> x[OWN / VEC];
+    int n, even;
+    uint32_t magic;     // ceil(2^20 / R), as n R <= 2^20: 256 rows of 64 elements
+    static __host__ __device__ __forceinline__ int pitch(int R) { return R | 1; }
+    __device__ __forceinline__ StagedRows(int rows, int R) : n(rows * R), even(~R & 1), magic(((1u << 20) + R - 1) / R) {}
+    __device__ __forceinline__ int first(int k) const { return (k * (int)blockDim.x + (int)threadIdx.x) * VEC; }
+    __device__ __forceinline__ int spot(int e) const { return even ? e + (int)(((uint32_t)e * magic) >> 20) : e; }
+    __device__ __forceinline__ void load(const T *p)
+    {
+#pragma unroll
+        for (int k = 0; k < OWN / VEC; k++) {
+            const int e = first(k);
+            if (e + VEC <= n) {
+                x[k] = load_pack<T, VEC, false>(p + e);
+            } else if (e < n) {
+#pragma unroll
+                for (int j = 0; j < VEC; j++) x[k].v[j] = p[e + j < n ? e + j : e];
+            }
+        }
+    }
+    __device__ __forceinline__ void put(T *lds) const
+    {
+#pragma unroll
+        for (int k = 0; k < OWN / VEC; k++) {
+            const int e = first(k);
+#pragma unroll
+            for (int j = 0; j < VEC; j++)
+                if (e + j < n) lds[spot(e + j)] = x[k].v[j];
+        }
+    }
+    __device__ __forceinline__ void store(T *p, const T *lds)
+    {
+#pragma unroll
+        for (int k = 0; k < OWN / VEC; k++) {
+            const int e = first(k);
+            if (e >= n) continue;
+#pragma unroll
+            for (int j = 0; j < VEC; j++) x[k].v[j] = lds[spot(e + j < n ? e + j : e)];
+            if (e + VEC <= n) {
+                store_pack<T, VEC, false>(p + e, x[k]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; j++)
+                    if (e + j < n) p[e + j] = x[k].v[j];
+            }
+        }
+    }
+};
+extern __shared__ __align__(16) unsigned char staged_raw[];
+
 // The softmax axis is not the last one, or is short: a lane per line, and as many wavefronts along the line as it
 // takes to hold it in registers, so that it is read and written once with all its loads in flight together.  The
 // sums run over the line in index order exactly as sum.rs:20-25 adds (they are handed from wavefront to wavefront).
@@ -138,7 +196,8 @@ __device__ __forceinline__ T sum_in_order(const T (&x)[OWN], int valid, const Li
 // walked a line three times, one load in flight; its backward pass 11.1 us, 20.5.
 // With `loss` set (cross-entropy, every line in this one workgroup) the kernel also folds the row
 // terms and divides by -N, in the order of ce_finalize_kernel: the whole loss in one launch.
-template <typename T, bool CE, int OWN>
+// STAGED (inner == 1): through StagedRows.
+template <typename T, bool CE, int OWN, bool STAGED>
 __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T *x, T *y, int64_t lines, int R,
                                                                          int64_t inner, int waves, const T *target,
                                                                          T *rowloss, T *loss, T neg_n)
@@ -148,19 +207,29 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T 
     const int lane = threadIdx.x & 63;
     const int r0 = at.w * OWN;
     const int valid = R - r0;              // uniform; at least 1
-    const T *const xl = x + at.base + r0 * inner;
-    T *const yl = y + at.base + r0 * inner;
+    zmath::ExpLog<T> ml;
+    StagedRows<T, OWN> rows(at.lines_here, R);
+    T *const staged = reinterpret_cast<T *>(staged_raw);
+    T *const row = staged + (at.active ? at.group * 64 + lane : 0) * rows.pitch(R);
+    if constexpr (STAGED) {
+        rows.load(x + at.first * R);
+        ml.init(true, CE);
+        rows.put(staged);
+        __syncthreads();
+    }
+    const int64_t step = STAGED ? 1 : inner;
+    const T *const xl = STAGED ? row + r0 : x + at.base + r0 * inner;
+    T *const yl = STAGED ? row + r0 : y + at.base + r0 * inner;
     T v[OWN];
 #pragma unroll
     for (int i = 0; i < OWN; i += 4) {
         if (i < valid) {
 #pragma unroll
-            for (int j = i; j < i + 4; j++) v[j] = xl[(j < valid ? j : 0) * inner];
+            for (int j = i; j < i + 4; j++) v[j] = xl[(j < valid ? j : 0) * step];
         }
     }
-    const T x0 = waves > 1 ? x[at.base] : v[0];
-    zmath::ExpLog<T> ml;
-    ml.init(true, CE);
+    const T x0 = waves > 1 ? (STAGED ? row[0] : x[at.base]) : v[0];
+    if constexpr (!STAGED) ml.init(true, CE);
     // max_axis: strict '>' from element 0 (max.rs:19-34): a NaN there stays, a NaN elsewhere never replaces
     T m = -INFINITY;
 #pragma unroll
@@ -188,13 +257,17 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T 
         for (int i = 0; i < OWN; i++) {
             if (i < valid) {
                 const T s = decltype(by_reciprocal)::value ? quotient<T>(v[i], sum, rcp) : v[i] / sum;
-                if (at.active) yl[i * inner] = s;
+                if (at.active) yl[i * step] = s;
                 if constexpr (CE) v[i] = target[at.base + r0 + i] * ml.log(s);
             }
         }
     };
     if (divides_by_reciprocal<T>(least, sum)) finish(std::true_type());
     else finish(std::false_type());
+    if constexpr (STAGED) {
+        __syncthreads();
+        rows.store(y + at.first * R, staged);
+    }
     if constexpr (CE) {
         if (waves > 1) __syncthreads();        // the sum of the exponentials has been read
         const T term = sum_in_order<T, OWN>(v, valid, at, waves, shared);
@@ -559,11 +632,16 @@ __global__ __launch_bounds__(kBlock) void ce_finalize_kernel(const T *rowloss, i
 }
 
 // ---- backward --------------------------------------------------------------------------------------------
+// elements per thread of the largest workgroups, which leave a thread 128 registers: y and t of the backward pass, or
+// the terms of the forward pass with the constants of exp, in 64 of them (f64 with 32 elements spills)
+template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
+
 // gx = t - y * sum(t), t = y * gy.  CE: gy = (target * g_total) / y with g_total = gout / (-N), the
 // chain div -> sum_to -> mul -> log backward of cross_entropy.rs:18-22.
 
-// lines in registers, as in softmax_lines_kernel; the sum of t in index order
-template <typename T, bool CE, int OWN>
+// lines in registers, as in softmax_lines_kernel; the sum of t in index order.  Where t alone fills the registers of a
+// workgroup of 1024 threads (f64 lines of 257 - 512 elements), y is read a second time.
+template <typename T, bool CE, int OWN, bool STAGED>
 __global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(const T *y, const T *gy_or_target, T *gx,
                                                                              int64_t lines, int R, int64_t inner,
                                                                              int waves, const T *gout, T neg_n)
@@ -574,26 +652,81 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(cons
     const int r0 = at.w * OWN;
     const int valid = R - r0;
     const int64_t base = at.base + r0 * inner;
-    T yv[OWN], t[OWN];
+    constexpr bool kHold = OWN <= kMost<T>;
+    T yv[kHold ? OWN : 1], t[OWN];
+    StagedRows<T, OWN> rows(at.lines_here, R);
+    T *const staged = reinterpret_cast<T *>(staged_raw);
+    T *const mine = staged + (at.active ? at.group * 64 + (threadIdx.x & 63) : 0) * rows.pitch(R) + r0;
+    auto product = [&](T yj, T g) { return yj * (CE ? (g * g_total) / yj : g); };
+    if constexpr (STAGED) {
+        static_assert(kHold, "short rows");
+        StagedRows<T, OWN> second(at.lines_here, R);
+        rows.load(y + at.first * R);
+        second.load(gy_or_target + at.first * R);
+        rows.put(staged);
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < OWN; i += 4) {
-        if (i < valid) {
+        for (int i = 0; i < OWN; i++)
+            if (i < valid) yv[i] = mine[i];
+        __syncthreads();
+        second.put(staged);
+        __syncthreads();
 #pragma unroll
-            for (int j = i; j < i + 4; j++) {
-                const int64_t off = base + (j < valid ? j : 0) * inner;
-                yv[j] = y[off];
-                t[j] = gy_or_target[off];
+        for (int i = 0; i < OWN; i++)
+            if (i < valid) t[i] = product(yv[i], mine[i]);
+    } else {
+        T once[OWN];
+#pragma unroll
+        for (int i = 0; i < OWN; i += 4) {
+            if (i < valid) {
+#pragma unroll
+                for (int j = i; j < i + 4; j++) {
+                    const int64_t off = base + (j < valid ? j : 0) * inner;
+                    once[j] = y[off];
+                    t[j] = gy_or_target[off];
+                }
+                if constexpr (!kHold) {
+#pragma unroll
+                    for (int j = i; j < i + 4; j++) t[j] = product(once[j], t[j]);
+                }
+            }
+        }
+        if constexpr (kHold) {
+#pragma unroll
+            for (int i = 0; i < OWN; i++) {
+                if (i < valid) {
+                    yv[i] = once[i];
+                    t[i] = product(yv[i], t[i]);
+                }
             }
         }
     }
-#pragma unroll
-    for (int i = 0; i < OWN; i++)
-        if (i < valid) t[i] = yv[i] * (CE ? (t[i] * g_total) / yv[i] : t[i]);
     const T sum = sum_in_order<T, OWN>(t, valid, at, waves, carry);
-    if (!at.active) return;
+    if constexpr (STAGED) {
+        if (waves == 1) __syncthreads();       // every row has been read (sum_in_order's barriers, otherwise)
+        if (at.active) {
 #pragma unroll
-    for (int i = 0; i < OWN; i++)
-        if (i < valid) gx[base + i * inner] = t[i] - yv[i] * sum;
+            for (int i = 0; i < OWN; i++)
+                if (i < valid) mine[i] = t[i] - yv[i] * sum;
+        }
+        __syncthreads();
+        rows.store(gx + at.first * R, staged);
+    } else if (at.active) {
+#pragma unroll
+        for (int i = 0; i < OWN; i += 4) {
+            if (i < valid) {
+                T again[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if constexpr (kHold) again[j] = yv[i + j];
+                    else again[j] = y[base + (i + j < valid ? i + j : 0) * inner];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (i + j < valid) gx[base + (i + j) * inner] = t[i + j] - again[j] * sum;
+            }
+        }
+    }
 }
 
 // lines longer than that, the softmax axis not the last one
@@ -1013,6 +1146,14 @@ template <typename T, bool CE> inline int line_most(const Geometry &g)
     if (g.inner > 1 || g.R <= 16) return 32;
     return CE ? 8 : sizeof(T) == 8 ? 16 : 32;
 }
+// Rows that go through StagedRows (us without / with, softmax and its backward pass): f32 [60000,33] 15.6 / 9.0 and 19.6 / 8.3,
+// [65536,64] 31 / 16 and 40 / 16, [65536,16] 10.1 / 5.5 and 10.0 / 4.8, [300,50] 6.3 / 5.2 and 5.4 / 4.5, [20000,21] 6.4 / 5.1 and
+// 5.4 / 4.4; f64 [65536,64] 36 / 25 and 50 / 20.  Short rows of a small tensor, which the first cache holds, lose by the turn in
+// LDS ([5000,10] 4.1 / 4.3 and 3.0 / 3.9), very short ones always ([65536,2] 2.7 / 3.3).
+inline bool staged_rows(const Geometry &g)
+{
+    return g.inner == 1 && g.R <= kLineMaxR && (g.R > 32 || (g.R >= 8 && g.outer * g.R >= 1 << 18));
+}
 // calls go(own) with `own` as a constant
 template <int MOST, typename Go> int with_own(int own, Go go)
 {
@@ -1034,11 +1175,11 @@ struct LineGrid {
         blocks = (all + groups - 1) / groups;
     }
     unsigned threads() const { return (unsigned)(64 * waves * groups); }
+    template <typename T, int OWN> size_t staged_bytes(int64_t R) const
+    {
+        return (size_t)(64 * groups) * StagedRows<T, OWN>::pitch((int)R) * sizeof(T);   // at most 35 KB: four groups only where R <= OWN
+    }
 };
-
-// elements per thread of the largest workgroups, which leave a thread 128 registers: y and t of the backward pass, or
-// the terms of the forward pass with the constants of exp, in 64 of them (f64 with 32 elements spills)
-template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
 
 // Threads per row and elements per thread of the rows kernels by row length (a streaming row
 // is cut at cache lines where the registers leave room for it).  go(lanes, elements, long) gets constants.
@@ -1105,7 +1246,15 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
             const LineGrid lg(lines, g.R, own, CE && loss);
             if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
             with_own<32>(own, [&](auto o) {
-                softmax_lines_kernel<T, CE, decltype(o)::value><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
+                constexpr int OWN = decltype(o)::value;
+                if constexpr (!CE) {
+                    if (staged_rows(g)) {
+                        softmax_lines_kernel<T, CE, OWN, true><<<(unsigned)lg.blocks, lg.threads(), lg.template staged_bytes<T, OWN>(g.R), s>>>(
+                            x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
+                        return 0;
+                    }
+                }
+                softmax_lines_kernel<T, CE, OWN, false><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
                     x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
                 return 0;
             });
@@ -1177,7 +1326,8 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
         }
     }
     if (g.inner != 1 || g.R <= kLineMaxR) {
-        const int own = line_own(lines, g.R, kMost<T>);
+        int own = line_own(lines, g.R, kMost<T>);
+        if (own == 0) own = line_own(lines, g.R, 32);
         if (own == 0) {
             const int64_t blocks = (lines + kBlock - 1) / kBlock;
             if (!grid_ok(blocks)) return ZENU_ERR_UNSUPPORTED;
@@ -1185,8 +1335,16 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
         } else {
             const LineGrid lg(lines, g.R, own, false);
             if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
-            with_own<kMost<T>>(own, [&](auto o) {
-                softmax_bwd_lines_kernel<T, CE, decltype(o)::value><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
+            with_own<32>(own, [&](auto o) {
+                constexpr int OWN = decltype(o)::value;
+                if constexpr (!CE && OWN <= kMost<T>) {
+                    if (staged_rows(g)) {
+                        softmax_bwd_lines_kernel<T, CE, OWN, true><<<(unsigned)lg.blocks, lg.threads(), lg.template staged_bytes<T, OWN>(g.R), s>>>(
+                            y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
+                        return 0;
+                    }
+                }
+                softmax_bwd_lines_kernel<T, CE, OWN, false><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
                     y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
                 return 0;
             });
