@@ -366,3 +366,27 @@ def test_copies_with_one_short_side(hip, dtype, shape):
         same(wide.to_numpy(), exp, ("into part of longer runs", shape, off))
         out.copy_from(wide.slice(slice(0, n), slice(0, short), slice(1, long + 1)).transpose())
         same(out.to_numpy(), exp[:, :, 1:long + 1].transpose(0, 2, 1), ("from part of longer runs", shape, off))
+
+
+# column sums whose splits are folded by a launch of their own: 8 to 64 row lanes, two splits to a hundred, outputs that are no
+# whole number of its workgroups, sources just below and above the size from which it is used.  Small whole numbers: every sum is exact
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", [(16383, 64), (16384, 64), (70001, 16), (65536, 33), (30000, 65), (4097, 257), (3000, 400), (1001, 1500), (517, 4100)],
+                         ids=str)
+def test_column_sums_folded_by_a_second_launch(hip, dtype, shape):
+    r = np.random.default_rng(shape[0])
+    a = r.integers(-3, 4, shape).astype(dtype)
+    x = r.integers(-1, 2, shape).astype(dtype)
+    rows, cols = shape
+    for off in (0, 1):
+        A, X = offset_matrix(hip, a, off), offset_matrix(hip, x, off)
+        out = hip.Matrix.from_numpy(np.full(cols + 2, 7, dtype))
+        hip.sum_to(A, hip.Matrix(out.buf, 1, (cols,), (1,), dtype))
+        exp = np.full(cols + 2, 7, dtype)
+        exp[1:-1] = a.sum(0, dtype=np.float64)
+        same(out.to_numpy(), exp, ("column sums", shape, off))
+        gx, gb = offset_matrix(hip, np.zeros(shape, dtype), off), hip.Matrix.from_numpy(np.zeros(cols, dtype))
+        gx.relu_backward_bias_grad(gb, A, X, 0.0)
+        g = np.where(x > 0, a, 0).astype(dtype)
+        same(np.abs(gx.to_numpy()), np.abs(g), ("ReLU gradient", shape, off))
+        same(gb.to_numpy(), g.sum(0, dtype=np.float64).astype(dtype), ("bias gradient", shape, off))

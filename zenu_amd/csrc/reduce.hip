@@ -778,6 +778,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
     }
     if (ty == 0)
         ZENU_FOR_COLS(j) emit_partial<T, Tr>(p, (int64_t)split * p.nout + o0 + j, acc[j]);
+    if (!p.counters) return;   // fold_cols_kernel follows
     if (!arrive_last(p.counters + group * p.cstride, split, p.splits, p.fan)) return;
     // fold this column tile: row lane ty takes splits ty, ty + ty_n, ...; then the fixed LDS order
 #pragma unroll
@@ -881,6 +882,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
         for (int j = 0; j < VEC; j++) emit_partial<T, Tr>(p, (int64_t)split * p.nout + o0 + j, acc.a[j]);
     }
     const int64_t group = q * gridDim.x + blockIdx.x;
+    if (!p.counters) return;   // fold_cols_kernel follows
     if (!arrive_last(p.counters + group, split, splits, splits)) return;
     // fold this column tile: row lane ty takes splits ty, ty + TY, ... two at a time, then the LDS order
 #pragma unroll
@@ -917,6 +919,41 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
         }
     }
     if (threadIdx.x == 0) store_agent(p.counters + group, 0);
+}
+
+// The splits of a column sum, added as the folding workgroup of kernel B adds them (`lanes` is its number of row lanes).
+constexpr int kFoldCols = 16;
+template <typename T>
+__global__ __launch_bounds__(1024) void fold_cols_kernel(const T *part, T *out, int64_t nout, int splits, int lanes)
+{
+    __shared__ T lds[1024];
+    const int tx = threadIdx.x % kFoldCols, ty = threadIdx.x / kFoldCols;
+    const int64_t o = (int64_t)blockIdx.x * kFoldCols + tx;
+    const T *const src = part + (o < nout ? o : nout - 1);
+    T acc = (T)0;
+    for (int s0 = ty; s0 < splits; s0 += 8 * lanes) {
+        T t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int s = s0 + u * lanes;
+            t[u] = src[(int64_t)(s < splits ? s : s0) * nout];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc = acc + (s0 + u * lanes < splits ? t[u] : (T)0);
+    }
+    lds[threadIdx.x] = acc;
+    __syncthreads();
+    if (lanes > 8) {
+        if (ty < 8)
+            for (int w = ty + 8; w < lanes; w += 8) acc = acc + lds[w * kFoldCols + tx];
+        __syncthreads();
+        if (ty < 8) lds[threadIdx.x] = acc;
+        __syncthreads();
+    }
+    if (ty == 0) {
+        for (int w = 1; w < (lanes < 8 ? lanes : 8); w++) acc = acc + lds[w * kFoldCols + tx];
+        if (o < nout) out[o] = acc;
+    }
 }
 
 // ---- kernel C: pieces -----------------------------------------------------------------------------------------
@@ -1025,6 +1062,7 @@ int launch_rows(const RedParams<T> &p, hipStream_t s)
 
 // threads along the columns for a cols launch: a power of two covering the row, at most kColsTx
 constexpr int64_t kSmallColsRows = 512, kSmallColsBytes = 4 << 20;   // see reduce_strided
+constexpr int64_t kFoldBytes = 4 << 20;   // see reduce_strided
 constexpr int kColsTx = 32;  // 32 lanes x 16 B = 512 B of a source row per wavefront half (measured best of 8..256)
 inline int cols_tx_shift(int64_t inner, int v)
 {
@@ -1185,6 +1223,30 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
 
     if (splits == 1) return use_cols ? launch_cols<T, Tr>(p, s) : launch_rows<T, Tr>(p, s);
 
+    if constexpr (std::is_same<Tr, SumTr<T>>::value) {
+        // Column sums: a second launch folds the splits.  The hand-over inside one launch is a chain of five round trips to
+        // memory (partials written through, two levels of counters, partials read) that the last workgroup of every column
+        // tile waits for, about 5 us; a launch behind another takes 1 - 2.  us, one launch / two: f32 [14252,542] 15.1 /
+        // 10.0, [10007,1003] 13.4 / 10.3, [4096,1024] 10.6 / 6.8, [16384,64] 7.1 / 5.5, [1000,1500] 6.8 / 5.6; f64 [10007,1003]
+        // 16.6 / 15.4 (80 MB, 5.2 TB/s), [4096,1024] 11.0 / 8.7, [1000,4000] 10.0 / 9.5.  Up to 16 splits of a large source,
+        // one level of counters, stream better through one launch: f32 [8192,4096] 23.0 / 23.4, f64 [4001,4001] 26.5 / 27.5.
+        // Small sources wait for the host, to which a launch is 2.3 us.
+        const int64_t bytes_in = outer * R * inner * (int64_t)sizeof(T);
+        if (use_cols && bytes_in >= kFoldBytes && (splits > 16 || bytes_in < kStreamBytes)) {
+            const size_t bytes = (size_t)nout * splits * sizeof(T);
+            if (fixed && bytes > fixed->partial_bytes) return ZENU_ERR_SCRATCH_LIMIT;
+            Workspace ws(fixed ? 0 : bytes, s);
+            if (ws.status) return ws.status;
+            p.part_key = static_cast<T *>(fixed ? fixed->partials : ws.ptr);
+            p.fan = (int)splits;
+            const int rc = launch_cols<T, Tr>(p, s);
+            if (rc) return rc;
+            const int lanes = kBlock >> p.cols_shift;
+            fold_cols_kernel<T><<<(unsigned)((nout + kFoldCols - 1) / kFoldCols), kFoldCols * lanes, 0, s>>>(p.part_key, out_val, nout, (int)splits, lanes);
+            ZENU_LAUNCH_CHECK();
+            return ZENU_OK;
+        }
+    }
     // one launch: partials in a workspace, folded by the last workgroup of each group to arrive
     // arrival tree: eight splits per leaf once a flat counter would serialise
     int fan = (int)splits, cstride = 1;
