@@ -571,6 +571,16 @@ def test_relu_backward_bias_grad(hip, dtype, shape, alpha):
     assert bits_equal(GY.to_numpy(), gx.to_numpy()) and bits_equal(gb3.to_numpy(), gb.to_numpy())
 
 
+# rows that are no whole number of vectors: a last vector of 1 .. 3 own elements in a full, a partial and a tile of its own,
+# one split and many, on both sides of the line to two launches (narrow and few rows) and of the fold's
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", [(5, 131), (402, 1497), (300, 127), (1025, 17), (2000, 65), (1030, 67), (64, 1025), (700, 129), (3000, 1403), (7, 20, 257)],
+                         ids=str)
+@pytest.mark.parametrize("alpha", [0.0, 0.2])
+def test_relu_backward_bias_grad_ragged(hip, dtype, shape, alpha):
+    test_relu_backward_bias_grad(hip, dtype, shape, alpha)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("n,c", [(1025, 64), (1100, 128), (4096, 32), (10007, 256), (30000, 16), (2000, 192)])
 def test_bias_gradient_has_the_bits_of_sum_to(hip, dtype, n, c):

@@ -341,12 +341,20 @@ template <typename T, int VEC, bool PRE> struct SrcVec {
         g = load_pack<T, VEC, NT>(ptr);
         if constexpr (PRE) x = load_pack<T, VEC, NT>(p.pre_x + (ptr - p.in));
     }
-    template <bool NT> __device__ __forceinline__ void apply(const RedParams<T> &p, const T *ptr)
+    // skip: leading elements that another thread writes
+    template <bool NT> __device__ __forceinline__ void apply(const RedParams<T> &p, const T *ptr, int skip)
     {
         if constexpr (PRE) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) g.v[j] = g.v[j] * ((x.v[j] > (T)0) ? (T)1 : p.pre_alpha * (T)-1);
-            store_pack<T, VEC, NT>(p.pre_out + (ptr - p.in), g);
+            T *const out = p.pre_out + (ptr - p.in);
+            if (skip == 0) {
+                store_pack<T, VEC, NT>(out, g);
+            } else {
+#pragma unroll
+                for (int j = 1; j < VEC; j++)
+                    if (j >= skip) out[j] = g.v[j];
+            }
         }
     }
 };
@@ -642,7 +650,8 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(RedParams<T> p)
 // which sits in host memory: 2-10 us before the first load (measured on the arg-max kernel).
 #define ZENU_FOR_COLS(j) _Pragma("unroll") for (int j = 0; j < VEC; j++) if (j < ncol)
 
-template <typename T, typename Tr, int VEC, bool NT, bool PRE = false>
+// RAGGED (with PRE): rows are no whole number of vectors.
+template <typename T, typename Tr, int VEC, bool NT, bool PRE = false, bool RAGGED = false>
 __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uint32_t col_tiles, int tx_shift, int grid3d, int banded)
 {
     typedef typename Tr::Acc A;
@@ -684,11 +693,12 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
     const int64_t q = q_u;
     const int64_t group = q * col_tiles + ct;   // the workgroups that share these outputs
     // A thread whose vector would run past the end of the row takes the row's last VEC columns instead; those that
-    // its neighbour has as well come to the same bits and are written twice.  (With PRE inner % VEC == 0: no element
-    // of pre_out has two writers.)
+    // its neighbour has as well come to the same bits and are written twice.  With PRE they are left to the neighbour,
+    // outputs and sums: pre_out may be the source, of which the neighbour may have written them already.
     const int64_t c0 = ((int64_t)ct * tx_n + tx) * VEC;
     const int64_t c = c0 + VEC <= p.inner ? c0 : p.inner - VEC;
     const int ncol = c0 < p.inner ? VEC : 0;
+    const int skip = RAGGED ? (int)(c0 - c) : 0;
     const T *src = p.in + q * p.outer_stride + c;
     constexpr int U = 4;
     const int64_t R = p.R;
@@ -747,7 +757,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
                     for (int u = 0; u < U; u++) x[u].template load<NT>(p, ptr + u * row_step);
 #pragma unroll
                     for (int u = 0; u < U; u++) {
-                        x[u].template apply<NT>(p, ptr + u * row_step);
+                        x[u].template apply<NT>(p, ptr + u * row_step, skip);
 #pragma unroll
                         for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x[u].g.v[j], r + u * ty_n);
                     }
@@ -756,7 +766,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
                     for (int64_t rr = r; rr < R; rr += ty_n, pt += row_step) {
                         SrcVec<T, VEC, PRE> x;
                         x.template load<false>(p, pt);
-                        x.template apply<false>(p, pt);
+                        x.template apply<false>(p, pt, skip);
 #pragma unroll
                         for (int j = 0; j < VEC; j++) acc[j] = Tr::update(acc[j], x.g.v[j], rr);
                     }
@@ -773,11 +783,11 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
     const int64_t o0 = q * p.inner + c;
     if (p.splits == 1) {
         if (ty == 0)
-            ZENU_FOR_COLS(j) emit_final<T, Tr>(p, o0 + j, acc[j]);
+            ZENU_FOR_COLS(j) if (j >= skip) emit_final<T, Tr>(p, o0 + j, acc[j]);
         return;
     }
     if (ty == 0)
-        ZENU_FOR_COLS(j) emit_partial<T, Tr>(p, (int64_t)split * p.nout + o0 + j, acc[j]);
+        ZENU_FOR_COLS(j) if (j >= skip) emit_partial<T, Tr>(p, (int64_t)split * p.nout + o0 + j, acc[j]);
     if (!p.counters) return;   // fold_cols_kernel follows
     if (!arrive_last(p.counters + group * p.cstride, split, p.splits, p.fan)) return;
     // fold this column tile: row lane ty takes splits ty, ty + ty_n, ...; then the fixed LDS order
@@ -801,7 +811,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(RedParams<T> p, uin
     }
     combine_rows(acc);
     if (ty == 0)
-        ZENU_FOR_COLS(j) emit_final<T, Tr>(p, o0 + j, acc[j]);
+        ZENU_FOR_COLS(j) if (j >= skip) emit_final<T, Tr>(p, o0 + j, acc[j]);
     if (threadIdx.x == 0) store_agent(p.counters + group * p.cstride, 0);
 }
 
@@ -856,7 +866,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
             for (int u = 0; u < U; u++) x[u].template load<NT>(p, src + (r + u * TY) * es);
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                x[u].template apply<NT>(p, src + (r + u * TY) * es);
+                x[u].template apply<NT>(p, src + (r + u * TY) * es, 0);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x[u].g.v[j], r + u * TY);
             }
@@ -864,7 +874,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_regular_kernel(RedParams<T
             for (int64_t rr = r; rr < R; rr += TY) {
                 SrcVec<T, VEC, PRE> x;
                 x.template load<false>(p, src + rr * es);
-                x.template apply<false>(p, src + rr * es);
+                x.template apply<false>(p, src + rr * es, 0);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) acc.a[j] = Tr::update(acc.a[j], x.g.v[j], rr);
             }
@@ -1063,6 +1073,7 @@ int launch_rows(const RedParams<T> &p, hipStream_t s)
 // threads along the columns for a cols launch: a power of two covering the row, at most kColsTx
 constexpr int64_t kSmallColsRows = 512, kSmallColsBytes = 4 << 20;   // see reduce_strided
 constexpr int64_t kFoldBytes = 4 << 20;   // see reduce_strided
+constexpr int64_t kNarrowRows = 1024;   // see reduce_strided
 constexpr int kColsTx = 32;  // 32 lanes x 16 B = 512 B of a source row per wavefront half (measured best of 8..256)
 inline int cols_tx_shift(int64_t inner, int v)
 {
@@ -1095,8 +1106,10 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
     // the regular geometry: full vector tiles of 32 x 8 threads, a split axis with a flat counter
     const bool regular = g3 && p.cols_vec == VEC && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
     if constexpr (!Tr::kHasIdx && std::is_same<Tr, SumTr<T>>::value) {
-        if (p.pre_x) {   // (the caller has checked that a row is a whole number of vectors)
-            if (regular) {
+        if (p.pre_x) {
+            if (p.inner % VEC) {   // (below the streaming sizes: zenu_hip_relu_backward_bias_grad)
+                reduce_cols_kernel<T, Tr, VEC, false, true, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
+            } else if (regular) {
                 if (nt) reduce_cols_regular_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p);
                 else    reduce_cols_regular_kernel<T, Tr, VEC, false, true><<<g, kBlock, 0, s>>>(p);
             } else {
@@ -1168,7 +1181,7 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
     p.g_elem_stride = elem_stride;
 
     const bool use_cols = inner >= 16;
-    if (pre_x && (!use_cols || inner % VEC)) return ZENU_ERR_UNSUPPORTED;   // the caller falls back to two launches
+    if (pre_x && !use_cols) return ZENU_ERR_UNSUPPORTED;   // the caller falls back to two launches
     int64_t splits = 1, groups = nout;
     p.cols_shift = 0;
     p.cols_vec = VEC;
@@ -1183,7 +1196,7 @@ int reduce_strided(const T *src, int64_t outer, int64_t R, int64_t inner, int64_
         const bool whole = aligned16(src) && inner % VEC == 0 && outer_stride % VEC == 0 && elem_stride % VEC == 0;
         const int64_t bytes = nout * R * (int64_t)sizeof(T);
         const bool narrow = inner < kColsTx * VEC;
-        if (!pre_x && (Tr::kHasIdx ? bytes < kStreamBytes && (inner >= 2 * kColsTx || R <= 4096) && (VEC == 4 || inner <= 512) : !whole && narrow && R <= 1024)) p.cols_vec = 1;
+        if (!pre_x && (Tr::kHasIdx ? bytes < kStreamBytes && (inner >= 2 * kColsTx || R <= 4096) && (VEC == 4 || inner <= 512) : !whole && narrow && R <= kNarrowRows)) p.cols_vec = 1;
         const int v = p.cols_vec;
         int shift = cols_tx_shift(inner, v);
         auto tiles_at = [&](int sh) { return (inner + (((int64_t)1 << sh) * v) - 1) / (((int64_t)1 << sh) * v); };
@@ -1703,11 +1716,16 @@ int zenu_hip_relu_backward_bias_grad(int dtype, const zenu_tensor_t *gx, const z
     // one launch when the gradient is a whole [.., N] tensor and the bias gradient its [N] (or [1, .., N])
     // column sums; anything else is the two calls it stands for
     bool fused = gx->ndim >= 2 && gbias->ndim >= 1 && num_elm(*gy) > 0 && is_default_stride_strict(*gx) &&
-                 is_default_stride_strict(*gy) && is_default_stride_strict(*x) && is_default_stride_strict(*gbias) &&
-                 aligned16(gx->ptr) && aligned16(x->ptr) && aligned16(gy->ptr);
+                 is_default_stride_strict(*gy) && is_default_stride_strict(*x) && is_default_stride_strict(*gbias);
     if (fused) {
-        const int64_t n = gx->shape[gx->ndim - 1];
-        fused = gbias->shape[gbias->ndim - 1] == n && num_elm(*gbias) == n;
+        // Whole aligned vectors; or any rows of which the sums take vectors of columns as well (the bias gradient has the
+        // bits of sum_to, see kNarrowRows), below the streaming sizes, where lines shared by two rows cost more: f32, us
+        // as two calls / in one launch, [402,1497] 7.5 / 5.4, [724,1397] 9.7 / 7.7, [1000,1499] 10.1 / 8.9, [500,301] 7.0 / 5.2;
+        // f64 [1000,1499] 14.0 / 11.3; but f32 [30000,1499] 123 / 141.
+        const int64_t n = gx->shape[gx->ndim - 1], vec = 16 / (int64_t)esz;
+        const bool whole = n % vec == 0 && aligned16(gx->ptr) && aligned16(x->ptr) && aligned16(gy->ptr);
+        const bool ragged = (n >= kColsTx * vec || (n >= vec && num_elm(*gy) / n > kNarrowRows)) && num_elm(*gy) * (int64_t)esz < kStreamSource;
+        fused = gbias->shape[gbias->ndim - 1] == n && num_elm(*gbias) == n && (whole || ragged);
     }
     if (fused) {
         rc = dtype == ZENU_F32 ? relu_backward_bias_grad_t<float>(*gx, *gbias, *gy, *x, alpha, as_stream(stream))
