@@ -622,13 +622,20 @@ __global__ __launch_bounds__(kBlock) void ew_rows_kernel(T *out, const T *a, con
 // long chain; with a quarter of the tile per workgroup a transposed copy of [256,512] f32 takes 2.8 us
 // against 3.3 us, of [784,512] 3.4 against 3.6 (the MLP step of a 512-wide layer issues eleven of them).
 // Operands that stay in the caches take them at every size, see launch_ew.
-template <typename T, bool SMALL = false> struct TileOf { static constexpr int N = (sizeof(T) == 4 ? 64 : 32) / (SMALL ? 2 : 1); };
+// Tile shapes: whole tiles, small ones, and small ones with two vectors per thread for copies of up to 96 MB, which wait for
+// the loads that are in flight: half the threads per workgroup, twice as many workgroups on a CU, two loads in each
+// thread.  us with one vector / two: [1500,1433] f32 5.2 / 4.9, [1500,1000] 4.2 / 4.0, NCHW -> NHWC [64,512,14,14] 9.6 / 9.0,
+// [4,166,75,76] 8.7 / 7.1, [40,124,29,30] 9.2 / 7.3, [92,51,22,22] 7.4 / 6.1; f64 [1500,1500] 7.8 / 7.2 (5.0 TB/s), [40,124,29,30]
+// 17.2 / 16.1.  Not other functions of one input (sine of a transposed [500,500] 2.7 / 3.1), two inputs (a + b^T
+// [3001,2047] 12.6 / 12.9) nor larger copies ([4099,4097] 31 / 33, f64 65 / 71).
+enum { kTileWhole, kTileSmall, kTileSmallPairs };
+template <typename T, int SMALL = kTileWhole> struct TileOf { static constexpr int N = (sizeof(T) == 4 ? 64 : 32) / (SMALL ? 2 : 1); };
 // With two inputs (three streams, a + b^T) two vectors per thread and operand at 512 threads are the
 // fastest (stand-alone probe: 36.2 us with four at 256 threads, 35.5 us with two at 512, 35.7 us with
 // one at 1024).
-template <typename T, typename F, bool SMALL = false> struct TileThreads {
+template <typename T, typename F, int SMALL = kTileWhole> struct TileThreads {
     static constexpr int kVecs = TileOf<T, SMALL>::N * TileOf<T, SMALL>::N / VecOf<T>::N;   // vectors per tile and operand
-    static constexpr int value = (F::NIN == 1 || kVecs < 512) ? kVecs : 512;
+    static constexpr int value = SMALL == kTileSmallPairs ? kVecs / 2 : (F::NIN == 1 || kVecs < 512) ? kVecs : 512;
 };
 
 enum { kWalkRows = 0, kWalkCols = 1, kWalkDiagonal = 2, kWalkBands = 3 };
@@ -647,7 +654,7 @@ struct TileParams {
     uint32_t tiles_r_magic;     // min(floor(2^32 / tiles_r), 2^32 - 1): x mod tiles_r from one high multiply and a fix-up
 };
 
-template <typename T, int MEM, typename F, bool SMALL = false>
+template <typename T, int MEM, typename F, int SMALL = kTileWhole>
 __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_kernel(T *out, const T *a, const T *b,
                                                                                   TileParams p, F f)
 {
@@ -1384,7 +1391,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
             const bool large = stream_tiles && full_tiles >= 2 * (int64_t)device_info().num_cus &&
                                full_tiles * (kFullTile * kFullTile) <= p.numel + p.numel / 25;
             auto launch_tiles = [&](auto small_c, auto nt_c) -> int {
-                constexpr bool SMALL = decltype(small_c)::value;
+                constexpr int SMALL = decltype(small_c)::value;
                 constexpr bool NT = decltype(nt_c)::value;
                 constexpr int kTile = TileOf<T, SMALL>::N;
                 tp.tiles_r = (tp.R + kTile - 1) / kTile;
@@ -1421,9 +1428,14 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                 else ew_tile_kernel<T, kMemStream, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
                 return ZENU_OK;
             };
-            const int rc_tiles = large          ? launch_tiles(std::false_type(), std::true_type())
-                                 : stream_tiles ? launch_tiles(std::true_type(), std::true_type())
-                                                : launch_tiles(std::true_type(), std::false_type());
+            typedef std::integral_constant<int, kTileWhole> Whole;
+            typedef std::integral_constant<int, kTileSmall> Small;
+            // (copies have the pairs in place of the small tiles without the hint, but for those that are too large)
+            const bool pairs = IsCopy<F>::value && bytes < 3 * kStreamBytes;
+            const int rc_tiles = large          ? launch_tiles(Whole(), std::true_type())
+                                 : stream_tiles ? launch_tiles(Small(), std::true_type())
+                                 : pairs        ? launch_tiles(std::integral_constant<int, IsCopy<F>::value ? kTileSmallPairs : kTileSmall>(), std::false_type())
+                                                : launch_tiles(Small(), std::false_type());
             if (rc_tiles) return rc_tiles;
             ZENU_LAUNCH_CHECK();
             return ZENU_OK;
