@@ -178,7 +178,7 @@ template <typename T, int OWN> struct StagedRows {
 #pragma unroll
             for (int j = 0; j < VEC; j++) x[k].v[j] = lds[spot(e + j < n ? e + j : e)];
             if (e + VEC <= n) {
-                store_pack<T, VEC, false>(p + e, x[k]);
+                store_pack_through<T, VEC>(p + e, x[k]);
             } else {
 #pragma unroll
                 for (int j = 0; j < VEC; j++)
@@ -192,12 +192,18 @@ extern __shared__ __align__(16) unsigned char staged_raw[];
 // The softmax axis is not the last one, or is short: a lane per line, and as many wavefronts along the line as it
 // takes to hold it in registers, so that it is read and written once with all its loads in flight together.  The
 // sums run over the line in index order exactly as sum.rs:20-25 adds (they are handed from wavefront to wavefront).
-// Bound by the passes over memory: [16,21,16384] f32 (22 MB each way, cached) 14.9 us, 26.1 when one thread
-// walked a line three times, one load in flight; its backward pass 11.1 us, 20.5.
+// Bound by the passes over memory and the f64 arithmetic of the exact exp between them: [16,21,16384] f32 (22 MB each way,
+// cached) 12.5 us, 26.1 when one thread walked a line three times, one load in flight; its backward pass 10.9 us, 20.5.
 // With `loss` set (cross-entropy, every line in this one workgroup) the kernel also folds the row
 // terms and divides by -N, in the order of ce_finalize_kernel: the whole loss in one launch.
-// STAGED (inner == 1): through StagedRows.
-template <typename T, bool CE, int OWN, bool STAGED>
+// MODE: kLinesStaged (inner == 1) through StagedRows; kLinesThrough writes the result through, see line_mode.
+enum { kLinesDirect, kLinesThrough, kLinesStaged };
+template <typename T, int MODE> __device__ __forceinline__ void store_line(T *p, T v)
+{
+    if constexpr (MODE == kLinesThrough) store_through<T>(p, v);
+    else *p = v;
+}
+template <typename T, bool CE, int OWN, int MODE>
 __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T *x, T *y, int64_t lines, int R,
                                                                          int64_t inner, int waves, const T *target,
                                                                          T *rowloss, T *loss, T neg_n)
@@ -207,6 +213,7 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T 
     const int lane = threadIdx.x & 63;
     const int r0 = at.w * OWN;
     const int valid = R - r0;              // uniform; at least 1
+    constexpr bool STAGED = MODE == kLinesStaged;
     zmath::ExpLog<T> ml;
     StagedRows<T, OWN> rows(at.lines_here, R);
     T *const staged = reinterpret_cast<T *>(staged_raw);
@@ -257,7 +264,7 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_lines_kernel(const T 
         for (int i = 0; i < OWN; i++) {
             if (i < valid) {
                 const T s = decltype(by_reciprocal)::value ? quotient<T>(v[i], sum, rcp) : v[i] / sum;
-                if (at.active) yl[i * step] = s;
+                if (at.active) store_line<T, MODE>(yl + i * step, s);
                 if constexpr (CE) v[i] = target[at.base + r0 + i] * ml.log(s);
             }
         }
@@ -641,7 +648,7 @@ template <typename T> constexpr int kMost = 128 / (int)sizeof(T);
 
 // lines in registers, as in softmax_lines_kernel; the sum of t in index order.  Where t alone fills the registers of a
 // workgroup of 1024 threads (f64 lines of 257 - 512 elements), y is read a second time.
-template <typename T, bool CE, int OWN, bool STAGED>
+template <typename T, bool CE, int OWN, int MODE>
 __global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(const T *y, const T *gy_or_target, T *gx,
                                                                              int64_t lines, int R, int64_t inner,
                                                                              int waves, const T *gout, T neg_n)
@@ -652,7 +659,7 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(cons
     const int r0 = at.w * OWN;
     const int valid = R - r0;
     const int64_t base = at.base + r0 * inner;
-    constexpr bool kHold = OWN <= kMost<T>;
+    constexpr bool kHold = OWN <= kMost<T>, STAGED = MODE == kLinesStaged;
     T yv[kHold ? OWN : 1], t[OWN];
     StagedRows<T, OWN> rows(at.lines_here, R);
     T *const staged = reinterpret_cast<T *>(staged_raw);
@@ -723,7 +730,9 @@ __global__ __launch_bounds__(kLineWaves * 64) void softmax_bwd_lines_kernel(cons
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    if (i + j < valid) gx[base + (i + j) * inner] = t[i + j] - again[j] * sum;
+                    if (i + j < valid) {
+                        store_line<T, MODE>(gx + base + (i + j) * inner, t[i + j] - again[j] * sum);
+                    }
             }
         }
     }
@@ -1131,6 +1140,7 @@ inline int line_own(int64_t lines, int64_t R, int most)
 {
     const int64_t groups = (lines + 63) / 64;
     const int64_t want = 8 * (int64_t)device_info().num_cus;
+    while (most > 8 && most / 2 >= R) most /= 2;   // (no registers for elements that no line has: [128,5,12544] f32 25.8 -> 16.0 us)
     for (int own = most; own >= 8; own /= 2) {
         if (R > (int64_t)own * kLineWaves) return own == most ? 0 : 2 * own;
         if (groups * ((R + own - 1) / own) >= want) return own;
@@ -1146,13 +1156,30 @@ template <typename T, bool CE> inline int line_most(const Geometry &g)
     if (g.inner > 1 || g.R <= 16) return 32;
     return CE ? 8 : sizeof(T) == 8 ? 16 : 32;
 }
-// Rows that go through StagedRows (us without / with, softmax and its backward pass): f32 [60000,33] 15.6 / 9.0 and 19.6 / 8.3,
-// [65536,64] 31 / 16 and 40 / 16, [65536,16] 10.1 / 5.5 and 10.0 / 4.8, [300,50] 6.3 / 5.2 and 5.4 / 4.5, [20000,21] 6.4 / 5.1 and
-// 5.4 / 4.4; f64 [65536,64] 36 / 25 and 50 / 20.  Short rows of a small tensor, which the first cache holds, lose by the turn in
+// Rows that go through StagedRows (us without / with, softmax and its backward pass): f32 [60000,33] 15.6 / 8.2 and 19.6 / 7.4,
+// [65536,64] 31 / 14 and 40 / 14, [65536,16] 10.1 / 5.1 and 10.0 / 4.5, [300,50] 6.3 / 5.2 and 5.4 / 4.5, [20000,21] 6.4 / 5.1 and
+// 5.4 / 4.4; f64 [65536,64] 36 / 23 and 50 / 19.  Short rows of a small tensor, which the first cache holds, lose by the turn in
 // LDS ([5000,10] 4.1 / 4.3 and 3.0 / 3.9), very short ones always ([65536,2] 2.7 / 3.3).
 inline bool staged_rows(const Geometry &g)
 {
     return g.inner == 1 && g.R <= kLineMaxR && (g.R > 32 || (g.R >= 8 && g.outer * g.R >= 1 << 18));
+}
+// How the lines kernels write (us, left in the L2 / written through): all wavefronts of a launch store at about the same
+// time, and what is dirty in the L2 then is written back behind the last of them.  Softmax [16,21,16384] f32 14.8 / 12.5,
+// [2,32,16083] 5.4 / 4.7, [32,120,3136] 25.9 / 23.7, f64 [16,21,8000] 15.6 / 13.7; backward 11.4 / 10.9, 4.1 / 3.6, f64 11.4 /
+// 10.9, but larger results stream better through the L2 ([8,21,50000] 17.5 / 17.8).  Staged rows: [65536,64] 16.3 / 14.1 and
+// 15.8 / 13.6.  Where neighbouring lanes do not write neighbouring elements the L2 has to collect them ([65536,3] 3.0 / 3.2).
+inline int line_mode(const Geometry &g, bool forward, size_t size)
+{
+    if (staged_rows(g)) return kLinesStaged;
+    return g.inner >= 32 && (forward || g.outer * g.R * g.inner * (int64_t)size < kStreamBytes) ? kLinesThrough : kLinesDirect;
+}
+template <bool MAY_STAGE, typename Go> void with_line_mode(int mode, Go go)
+{
+    if constexpr (MAY_STAGE)
+        if (mode == kLinesStaged) return go(std::integral_constant<int, kLinesStaged>());
+    if (mode == kLinesThrough) go(std::integral_constant<int, kLinesThrough>());
+    else go(std::integral_constant<int, kLinesDirect>());
 }
 // calls go(own) with `own` as a constant
 template <int MOST, typename Go> int with_own(int own, Go go)
@@ -1247,15 +1274,13 @@ int softmax_forward_launch(const T *x, T *y, Geometry g, const T *target, T *row
             if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
             with_own<32>(own, [&](auto o) {
                 constexpr int OWN = decltype(o)::value;
-                if constexpr (!CE) {
-                    if (staged_rows(g)) {
-                        softmax_lines_kernel<T, CE, OWN, true><<<(unsigned)lg.blocks, lg.threads(), lg.template staged_bytes<T, OWN>(g.R), s>>>(
-                            x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
-                        return 0;
-                    }
-                }
-                softmax_lines_kernel<T, CE, OWN, false><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
-                    x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
+                auto go = [&](auto mode_c) {
+                    constexpr int MODE = decltype(mode_c)::value;
+                    softmax_lines_kernel<T, CE, OWN, MODE><<<(unsigned)lg.blocks, lg.threads(), MODE == kLinesStaged ? lg.template staged_bytes<T, OWN>(g.R) : 0, s>>>(
+                        x, y, lines, (int)g.R, g.inner, lg.waves, target, rowloss, loss, neg_n);
+                };
+                if constexpr (CE) go(std::integral_constant<int, kLinesDirect>());   // (the loss: inner == 1)
+                else with_line_mode<true>(line_mode(g, true, sizeof(T)), go);
                 return 0;
             });
         }
@@ -1337,15 +1362,13 @@ int softmax_backward_launch(const T *y, const T *gy_or_target, T *gx, Geometry g
             if (!grid_ok(lg.blocks)) return ZENU_ERR_UNSUPPORTED;
             with_own<32>(own, [&](auto o) {
                 constexpr int OWN = decltype(o)::value;
-                if constexpr (!CE && OWN <= kMost<T>) {
-                    if (staged_rows(g)) {
-                        softmax_bwd_lines_kernel<T, CE, OWN, true><<<(unsigned)lg.blocks, lg.threads(), lg.template staged_bytes<T, OWN>(g.R), s>>>(
-                            y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
-                        return 0;
-                    }
-                }
-                softmax_bwd_lines_kernel<T, CE, OWN, false><<<(unsigned)lg.blocks, lg.threads(), 0, s>>>(
-                    y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
+                auto go = [&](auto mode_c) {
+                    constexpr int MODE = decltype(mode_c)::value;
+                    softmax_bwd_lines_kernel<T, CE, OWN, MODE><<<(unsigned)lg.blocks, lg.threads(), MODE == kLinesStaged ? lg.template staged_bytes<T, OWN>(g.R) : 0, s>>>(
+                        y, gy_or_target, gx, lines, (int)g.R, g.inner, lg.waves, gout, neg_n);
+                };
+                if constexpr (CE) go(std::integral_constant<int, kLinesDirect>());
+                else with_line_mode<OWN <= kMost<T>>(line_mode(g, false, sizeof(T)), go);   // (staged rows are short)
                 return 0;
             });
         }

@@ -78,6 +78,13 @@ template <typename T, int N> __device__ __forceinline__ void store_pack_through(
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(reinterpret_cast<V *>(p)), "v"(x) : "memory");
 }
 
+// one element written through, for kernels whose lanes store neighbouring elements
+template <typename T> __device__ __forceinline__ void store_through(T *p, T v)
+{
+    if constexpr (sizeof(T) == 4) asm volatile("global_store_dword %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
 // the same at row + at, `row` being the same in the whole wavefront and 0 <= at * sizeof(T) < 2^31: one address
 // register.  The five wait states in front are what a memory instruction needs after a vector instruction has written
 // one of its scalar registers (v_readfirstlane, or v_readlane where a spilled one is taken back); the compiler counts
