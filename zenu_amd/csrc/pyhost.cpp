@@ -130,7 +130,9 @@ bool as_tensor(PyObject *m, zenu_tensor_t &t, int &code)
         t.shape[i] = a;
         t.stride[i] = b;
     }
+    Py_INCREF(buf);   // (ptr may be a property: its code could take the buffer out of the Matrix)
     PyObject *ptr = PyObject_GetAttr(buf, s_ptr);
+    Py_DECREF(buf);
     if (!ptr) {
         PyErr_Clear();
         return false;
@@ -326,6 +328,8 @@ struct Update {
         zenu_tensor_t t;
         for (int k = 0; k < kinds; k++) {
             int c;
+            Py_INCREF(matrices[k]);
+            held.push_back(matrices[k]);
             if (!as_tensor(matrices[k], t, c) || !default_stride(t)) return false;
             if (code < 0) code = c;
             if (c != code) return false;
@@ -335,8 +339,6 @@ struct Update {
                 for (int i = 0; i < t.ndim; i++) n *= t.shape[i];
                 sizes.push_back(n);
             }
-            Py_INCREF(matrices[k]);
-            held.push_back(matrices[k]);
         }
         return true;
     }
