@@ -22,7 +22,8 @@
 // many workgroups share an output) and the one that arrives last folds the partials of its
 // outputs, always in split order.  No workgroup waits for another and no atomic touches data:
 // the combination tree is fixed by the launch geometry, so results are bit-reproducible, and
-// the whole reduction is ONE launch.
+// the whole reduction is ONE launch -- but for column sums of 4 MB or more over many splits,
+// which a second launch folds in the same order (fold_cols_kernel), faster than the counters.
 //
 // Arg-max follows MaxIdx for Cpu (max.rs:19-34): start from element 0 and replace on strict '>'.
 // That is "largest value, lowest index on ties", except for NaN: a NaN at position 0 is never
