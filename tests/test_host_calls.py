@@ -1,6 +1,8 @@
 """The native host side of a call (csrc/pyhost.cpp) against the ctypes one beside it: the same descriptors, the same
 results, the same errors, and what it does not take goes the ctypes way unchanged."""
 import ctypes as C
+import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -53,6 +55,40 @@ def test_transposed_view():
     assert _pyhost.transpose(Derived(Memory(4096), 0, (2, 3), (3, 1), np.float32)) is None
     u = Derived(Memory(4096), 0, (2, 3), (3, 1), np.float32).transpose()
     assert (u.shape, u.stride) == ((3, 2), (1, 3))
+
+
+def test_optimizer_operands_are_held_while_they_are_read():
+    """reading a buffer's address can run code that takes the entry, its moments and its name away"""
+    zenu_amd.lib()
+
+    def matrix(memory, stride=(3, 1)):
+        return Matrix(memory, 0, (2, 3), stride, np.float32)
+
+    for kinds in (2, 4):
+        alive = []
+
+        class Taking:
+            @property
+            def ptr(self):
+                for d in (params, m, v, weights):
+                    d.clear()
+                gc.collect()
+                alive.append([r() is not None for r in refs])
+                return 4096
+
+        # the last matrix that is read has another stride: the call is declined after all of them
+        last = (1, 2)
+        g, first, second = matrix(Memory(4096), last if kinds == 2 else (3, 1)), matrix(Memory(4096)), matrix(Memory(4096), last)
+        refs = [weakref.ref(x) for x in (g, first, second)[:kinds - 1]]
+        name = "".join(["layer", ".", "weight"])
+        params, m, v, weights = {name: (matrix(Taking()), g)}, {name: first}, {name: second}, {name}
+        del g, first, second, name
+        if kinds == 2:
+            assert _pyhost.sgd_step_multi(params, 1e-3, None) is False
+        else:
+            assert _pyhost.adam_step_multi(params, m, v, weights, 1e-3, 0.9, 0.999, 1e-8, 0.0, 1, None) is False
+        assert alive == [[True] * (kinds - 1)]
+        assert not params and all(r() is None for r in refs)      # and let go afterwards
 
 
 def test_other_forms_are_left_to_ctypes():

@@ -314,7 +314,9 @@ ZENU_PY_END
 // ---- optimizers ----------------------------------------------------------------------------------------------------
 
 // The tensors of an update in the order of the mapping: per entry with a gradient `kinds` matrices of one dtype in default
-// stride.  Holds a reference to each while the GIL is released, as the argument lists of the general path do.
+// stride.  Reading a matrix can run Python code (ptr may be a property, and another thread may get the GIL in it) that
+// takes entries out of the mapping or of a dictionary of moments, so everything is held first and read afterwards; the
+// matrices stay held while the GIL is released, as the argument lists of the general path hold them.
 struct Update {
     std::vector<void *> ptr[4];
     std::vector<int64_t> sizes;
@@ -323,13 +325,16 @@ struct Update {
     int code = -1;
     ~Update() { for (PyObject *o : held) Py_DECREF(o); }
 
+    void hold(PyObject *o)
+    {
+        held.push_back(o);
+        Py_INCREF(o);
+    }
     bool add(PyObject *const *matrices, int kinds)
     {
         zenu_tensor_t t;
         for (int k = 0; k < kinds; k++) {
             int c;
-            Py_INCREF(matrices[k]);
-            held.push_back(matrices[k]);
             if (!as_tensor(matrices[k], t, c) || !default_stride(t)) return false;
             if (code < 0) code = c;
             if (c != code) return false;
@@ -351,31 +356,45 @@ struct Update {
         for (auto &p : ptr) p.reserve(most);
         sizes.reserve(most);
         decay.reserve(most);
-        held.reserve(4 * most);
+        held.reserve((m ? 5 : 3) * most);
         PyObject *key, *value;
         Py_ssize_t at = 0;
-        while (PyDict_Next(parameters, &at, &key, &value)) {
+        while (PyDict_Next(parameters, &at, &key, &value)) {   // nothing in this loop runs Python code
             if (!PyUnicode_CheckExact(key) || !PyTuple_CheckExact(value) || PyTuple_GET_SIZE(value) != 2) return false;
-            PyObject *matrices[4] = {PyTuple_GET_ITEM(value, 0), PyTuple_GET_ITEM(value, 1), nullptr, nullptr};
-            if (matrices[1] == Py_None) continue;
-            if (m) {
-                matrices[2] = PyDict_GetItemWithError(m, key);
-                matrices[3] = PyDict_GetItemWithError(v, key);
-                if (!matrices[2] || !matrices[3]) {
-                    PyErr_Clear();
-                    return false;
+            if (PyTuple_GET_ITEM(value, 1) == Py_None) continue;
+            hold(key);
+            hold(PyTuple_GET_ITEM(value, 0));
+            hold(PyTuple_GET_ITEM(value, 1));
+        }
+        const size_t entries = held.size() / 3;
+        if (m) {
+            for (size_t e = 0; e < entries; e++) {
+                for (PyObject *moments : {m, v}) {
+                    PyObject *moment = PyDict_GetItemWithError(moments, held[3 * e]);
+                    if (!moment) {
+                        PyErr_Clear();
+                        return false;
+                    }
+                    hold(moment);
                 }
+            }
+        }
+        for (size_t e = 0; e < entries; e++) {
+            PyObject *matrices[4] = {held[3 * e + 1], held[3 * e + 2], nullptr, nullptr};
+            if (m) {
+                matrices[2] = held[3 * entries + 2 * e];
+                matrices[3] = held[3 * entries + 2 * e + 1];
             }
             if (!add(matrices, m ? 4 : 2)) return false;
             int in = 0;
-            if (weights && weights != Py_None) in = PySet_Contains(weights, key);
+            if (weights && weights != Py_None) in = PySet_Contains(weights, held[3 * e]);
             if (in < 0) {
                 PyErr_Clear();
                 return false;
             }
             decay.push_back(in);
         }
-        return sizes.size() <= (size_t)INT_MAX;
+        return entries <= (size_t)INT_MAX;
     }
 };
 
