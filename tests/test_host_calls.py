@@ -91,6 +91,26 @@ def test_optimizer_operands_are_held_while_they_are_read():
         assert not params and all(r() is None for r in refs)      # and let go afterwards
 
 
+def test_transposed_view_holds_what_it_copies():
+    """an allocation can start the collector, and a finalizer can replace the attributes that the view takes"""
+    m = Matrix(Memory(4096), 0, (2, 3), (3, 1), np.float32)
+    ref, old = weakref.ref(m.buf), gc.get_threshold()
+
+    def replace(phase, info):
+        m.buf, m.shape, m.stride = Memory(0), (9, 9), (9, 1)
+
+    gc.collect()
+    gc.callbacks.append(replace)
+    gc.set_threshold(1)
+    try:
+        t = _pyhost.transpose(m)
+    finally:
+        gc.set_threshold(*old)
+        gc.callbacks.remove(replace)
+    assert (t.shape, t.stride) in (((3, 2), (1, 3)), ((9, 9), (1, 9)))     # one state or the other, whole
+    assert t.buf is ref() if t.shape == (3, 2) else t.buf is m.buf
+
+
 def test_other_forms_are_left_to_ctypes():
     m = Matrix(Memory(4096), 0, (2, 3), (3, 1), np.float32)
     odd = [Derived(Memory(4096), 0, (2, 3), (3, 1), np.float32), Matrix(Memory(4096), 0, (2, 3), (3, 1), np.int64),

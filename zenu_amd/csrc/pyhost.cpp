@@ -460,33 +460,28 @@ PyObject *py_transpose(PyObject *, PyObject *m)
     }
     for (int i = 2; i < 4; i++)
         if (!PyTuple_CheckExact(v[i]) || PyTuple_GET_SIZE(v[i]) < 2 || PyTuple_GET_SIZE(v[i]) != PyTuple_GET_SIZE(v[2])) Py_RETURN_NONE;
+    for (PyObject *x : v) Py_INCREF(x);   // (an allocation can start the collector, whose finalizers may take them out of the Matrix)
     PyObject *view = g_matrix->tp_alloc(g_matrix, 0);
-    if (!view) return nullptr;
-    for (int i = 0; i < 5; i++) {
-        PyObject *x = v[i];
-        Py_INCREF(x);
-        if (i == 2 || i == 3) {
-            const Py_ssize_t n = PyTuple_GET_SIZE(x);
-            PyObject *turned = PyTuple_New(n);
-            if (!turned) {
-                Py_DECREF(x);
-                Py_DECREF(view);
-                return nullptr;
-            }
-            for (Py_ssize_t k = 0; k < n; k++) {
-                PyObject *e = PyTuple_GET_ITEM(x, k == n - 1 ? n - 2 : k == n - 2 ? n - 1 : k);
-                Py_INCREF(e);
-                PyTuple_SET_ITEM(turned, k, e);
-            }
-            Py_DECREF(x);
-            x = turned;
+    bool ok = view != nullptr;
+    for (int i = 2; i < 4 && ok; i++) {
+        const Py_ssize_t n = PyTuple_GET_SIZE(v[i]);
+        PyObject *turned = PyTuple_New(n);
+        if (!turned) {
+            ok = false;
+            break;
         }
-        const int rc = PyObject_SetAttr(view, names[i], x);
-        Py_DECREF(x);
-        if (rc) {
-            Py_DECREF(view);
-            return nullptr;
+        for (Py_ssize_t k = 0; k < n; k++) {
+            PyObject *e = PyTuple_GET_ITEM(v[i], k == n - 1 ? n - 2 : k == n - 2 ? n - 1 : k);
+            Py_INCREF(e);
+            PyTuple_SET_ITEM(turned, k, e);
         }
+        Py_SETREF(v[i], turned);
+    }
+    for (int i = 0; i < 5 && ok; i++) ok = PyObject_SetAttr(view, names[i], v[i]) == 0;
+    for (PyObject *x : v) Py_DECREF(x);
+    if (!ok) {
+        Py_XDECREF(view);
+        return nullptr;
     }
     return view;
 }
