@@ -581,6 +581,24 @@ def test_relu_backward_bias_grad_ragged(hip, dtype, shape, alpha):
     test_relu_backward_bias_grad(hip, dtype, shape, alpha)
 
 
+# a gradient that shares memory with the incoming one other than as the same view: whole aligned rows, and the shifts that rows
+# of any length and address allow
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("rows,cols,shift", [(64, 256, 256), (64, 256, 1), (64, 257, 257), (64, 257, 1), (1100, 33, 4), (8, 24, 24)])
+def test_relu_backward_bias_grad_refuses_shifted_operands(hip, dtype, rows, cols, shift):
+    from zenu_amd import _lib
+    M, n = hip.Matrix, rows * cols
+    a = np.random.default_rng(n).standard_normal(n + shift).astype(dtype)
+    whole, x = M.from_numpy(a), M.from_numpy(np.ones((rows, cols), dtype))
+    low, high = (M(whole.buf, at, (rows, cols), (cols, 1), dtype) for at in (0, shift))
+    gb = M.from_numpy(np.full(cols, 7, dtype))
+    for gx, gy, other in ((low, high, x), (high, low, x), (low, x, high), (high, x, low)):
+        with pytest.raises(hip.ZenuHipError) as e:
+            gx.relu_backward_bias_grad(gb, gy, other, 0.1)
+        assert e.value.status == _lib.ERR_ARG
+        assert bits_equal(whole.to_numpy(), a) and np.all(gb.to_numpy() == 7), "a refused call wrote something"
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("n,c", [(1025, 64), (1100, 128), (4096, 32), (10007, 256), (30000, 16), (2000, 192)])
 def test_bias_gradient_has_the_bits_of_sum_to(hip, dtype, n, c):

@@ -1712,7 +1712,8 @@ int zenu_hip_relu_backward_bias_grad(int dtype, const zenu_tensor_t *gx, const z
     const size_t esz = dtype == ZENU_F32 ? 4 : 8;
     if (view_overlaps(*gx, esz, gbias->ptr, (size_t)num_elm(*gbias) * esz) ||
         view_overlaps(*gy, esz, gbias->ptr, (size_t)num_elm(*gbias) * esz) ||
-        view_overlaps(*x, esz, gbias->ptr, (size_t)num_elm(*gbias) * esz) || check_output_alias(*gx, *x, esz))
+        view_overlaps(*x, esz, gbias->ptr, (size_t)num_elm(*gbias) * esz) || check_output_alias(*gx, *x, esz) ||
+        check_output_alias(*gx, *gy, esz))
         return ZENU_ERR_ARG;
     // one launch when the gradient is a whole [.., N] tensor and the bias gradient its [N] (or [1, .., N])
     // column sums; anything else is the two calls it stands for
