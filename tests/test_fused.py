@@ -581,6 +581,34 @@ def test_relu_backward_bias_grad_ragged(hip, dtype, shape, alpha):
     test_relu_backward_bias_grad(hip, dtype, shape, alpha)
 
 
+# every form of the bias gradient for rows that are no whole number of vectors: what the two calls give, the sign of a zero
+# included, and what they refuse
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", [(402, 131), (1, 1031), (2, 131), (7, 60, 257), (1, 7, 257), (1, 1, 257)], ids=str)
+def test_relu_backward_bias_grad_is_the_two_calls(hip, dtype, shape):
+    M, n = hip.Matrix, shape[-1]
+    r = np.random.default_rng(n)
+    x, gy = r.standard_normal(shape).astype(dtype), r.standard_normal(shape).astype(dtype)
+    x[..., :8] = -1                                        # gradients that are zero, of either sign
+    X, GY = M.from_numpy(x), M.from_numpy(gy)
+    for form in ((n,), (1, n), (1, 1, n), (1, 1, 1, n)):
+        gx, gx2 = M.zeros(shape, dtype), M.zeros(shape, dtype)
+        gb, gb2 = (M.from_numpy(np.full(form, 7, dtype)) for _ in range(2))
+        gx2.relu_backward(GY, X, 0.0)
+        try:
+            hip.sum_to(gx2, gb2)
+            expect = None
+        except hip.ZenuHipError as e:
+            expect = e.status
+        try:
+            gx.relu_backward_bias_grad(gb, GY, X, 0.0)
+            got = None
+        except hip.ZenuHipError as e:
+            got = e.status
+        assert got == expect, form
+        assert bits_equal(gx.to_numpy(), gx2.to_numpy()) and bits_equal(gb.to_numpy(), gb2.to_numpy()), form
+
+
 # a gradient that shares memory with the incoming one other than as the same view: whole aligned rows, and the shifts that rows
 # of any length and address allow
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])

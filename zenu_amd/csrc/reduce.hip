@@ -1521,6 +1521,28 @@ int reduce_axis(int kind, int dtype, const zenu_tensor_t *out, int64_t *out_idx,
     return ZENU_ERR_ARG;
 }
 
+// The axes that sum_to reduces, in the order the reference reduces them (sum.rs:35-94), and which of them stay as 1; or what
+// is wrong with the shapes.
+int sum_to_axes(const zenu_tensor_t &src, const zenu_tensor_t &target, int *axes, int *keep, int &na)
+{
+    na = 0;
+    if (src.ndim < target.ndim) return ZENU_ERR_RANK;
+    const int diff = src.ndim - target.ndim;
+    if (diff == 0) {
+        for (int i = 0; i < src.ndim; i++) {
+            if (src.shape[i] == target.shape[i]) continue;
+            if (target.shape[i] != 1) return ZENU_ERR_SHAPE;
+            axes[na] = i; keep[na] = 1; na++;
+        }
+    } else {
+        // trailing dims must match exactly (is_include), leading axes are summed away
+        for (int i = 0; i < target.ndim; i++)
+            if (src.shape[diff + i] != target.shape[i]) return ZENU_ERR_SHAPE;
+        for (int i = 0; i < diff; i++) { axes[na] = 0; keep[na] = 0; na++; }
+    }
+    return ZENU_OK;
+}
+
 // whole-tensor reductions: view the (contiguous copy of the) source as one row
 int reduce_all(int kind, int dtype, void *out_val, int64_t *out_idx, const zenu_tensor_t *src, hipStream_t s)
 {
@@ -1726,7 +1748,10 @@ int zenu_hip_relu_backward_bias_grad(int dtype, const zenu_tensor_t *gx, const z
         // f64 [1000,1499] 14.0 / 11.3; but f32 [30000,1499] 123 / 141.
         const int64_t n = gx->shape[gx->ndim - 1], vec = 16 / (int64_t)esz;
         const bool whole = n % vec == 0 && aligned16(gx->ptr) && aligned16(x->ptr) && aligned16(gy->ptr);
-        const bool ragged = (n >= kColsTx * vec || (n >= vec && num_elm(*gy) / n > kNarrowRows)) && num_elm(*gy) * (int64_t)esz < kStreamSource;
+        // (sum_to has no sums to make, but a copy, where gbias has the shape of gx: it keeps the sign of a zero)
+        int axes[kMaxDim * 2], keep[kMaxDim * 2], na;
+        const bool ragged = (n >= kColsTx * vec || (n >= vec && num_elm(*gy) / n > kNarrowRows)) && num_elm(*gy) * (int64_t)esz < kStreamSource &&
+                            sum_to_axes(*gx, *gbias, axes, keep, na) == ZENU_OK && na > 0;
         fused = gbias->shape[gbias->ndim - 1] == n && num_elm(*gbias) == n && (whole || ragged);
     }
     if (fused) {
@@ -1747,26 +1772,13 @@ int zenu_hip_sum_to(int dtype, const zenu_tensor_t *target, const zenu_tensor_t 
     if (!rc) rc = ensure_init();
     if (rc) return rc;
     if (dtype != ZENU_F32 && dtype != ZENU_F64) return ZENU_ERR_ARG;
-    if (src->ndim < target->ndim) return ZENU_ERR_RANK;
     hipStream_t s = as_stream(stream);
     if (same_shape(*src, *target)) return zenu_hip_copy(dtype, target, src, stream);
     const size_t esz = dtype == ZENU_F32 ? 4 : 8;
     const int diff = src->ndim - target->ndim;
-
-    // list of axes to reduce, in the order the reference reduces them
     int axes[kMaxDim * 2], keep[kMaxDim * 2], na = 0;
-    if (diff == 0) {
-        for (int i = 0; i < src->ndim; i++) {
-            if (src->shape[i] == target->shape[i]) continue;
-            if (target->shape[i] != 1) return ZENU_ERR_SHAPE;
-            axes[na] = i; keep[na] = 1; na++;
-        }
-    } else {
-        // trailing dims must match exactly (is_include), leading axes are summed away
-        for (int i = 0; i < target->ndim; i++)
-            if (src->shape[diff + i] != target->shape[i]) return ZENU_ERR_SHAPE;
-        for (int i = 0; i < diff; i++) { axes[na] = 0; keep[na] = 0; na++; }
-    }
+    rc = sum_to_axes(*src, *target, axes, keep, na);
+    if (rc) return rc;
 
     // Two or more axes of a contiguous source that leave one run of kept dims in the middle, [N, C, I]: in one go.
     // (A target inside the source is written by the last of several launches only, as below.)
