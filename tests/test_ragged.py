@@ -390,3 +390,26 @@ def test_column_sums_folded_by_a_second_launch(hip, dtype, shape):
         g = np.where(x > 0, a, 0).astype(dtype)
         same(np.abs(gx.to_numpy()), np.abs(g), ("ReLU gradient", shape, off))
         same(gb.to_numpy(), g.sum(0, dtype=np.float64).astype(dtype), ("bias gradient", shape, off))
+
+
+# How many accumulators a lane has where workgroups share a row, on both sides of the 32 MB from which there are eight and of
+# the 128 MB from which the loads stream.  A value so large that single ones added to it are lost stands first; two ones
+# stand where the first lane meets them as well, one by one, if it has four accumulators, and another workgroup adds them
+# up first if it has eight.
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("mbytes,accumulators", [(31, 4), (32, 8), (100, 8), (127, 8), (128, 8), (160, 8)])
+def test_accumulators_of_shared_rows(hip, dtype, mbytes, accumulators):
+    size = np.dtype(dtype).itemsize
+    vec, large = 16 // size, dtype(2) ** (24 if size == 4 else 53)
+    splits = 512                                           # two workgroups on each of 256 CUs
+    for rows in (1, 4):
+        a = np.zeros((rows, mbytes * (1 << 20) // size // rows), dtype)
+        second = 4 * 256 * vec * (splits // rows)          # the first workgroup's second chunk with four accumulators
+        a[:, 0] = large
+        a[:, second:second + 2] = 1
+        assert second + 2 <= a.shape[1]
+        exp = np.full(rows, large + 2 if accumulators == 8 else large, dtype)
+        m = hip.Matrix.from_numpy(a)
+        same((m.sum(1) if rows > 1 else m.sum_all()).to_numpy().reshape(rows), exp, ("sum", rows))
+        if rows == 1:
+            assert m.asum() == exp[0]

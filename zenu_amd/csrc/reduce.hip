@@ -9,7 +9,7 @@
 //
 //   rows : inner < 16, normally 1 (the reduced axis is contiguous) -- one workgroup (or one
 //          wavefront when the row is short) per row, 128-bit loads, four independent
-//          accumulators per lane (eight when workgroups share a row), wave64 butterfly built
+//          accumulators per lane (eight when workgroups share a row of a source of 32 MB or more), wave64 butterfly built
 //          from DPP (quad_perm, row_half_mirror, row_mirror), ds_swizzle and one cross-half
 //          exchange, then a fixed-order combine of the 4 waves through LDS.
 //   cols : inner >= 16 -- a 32 x 8 thread tile: 32 lanes own 32 column vectors (512-byte row
@@ -1045,6 +1045,9 @@ int launch_rows(const RedParams<T> &p, hipStream_t s)
     // 12.9, [16384,255] 9.3 / 11.3, [1000,999] 2.7 / 3.3; f64: [10007,1003] 13.5 / 13.6, [1000,999] 3.3 / 4.3.
     const bool vec = p.elem_stride == 1 && p.inner == 1 && p.R >= VEC && p.R > kWave;
     const bool nt = vec && stream_source(p);
+    // Rows shared by workgroups have twice the loads in flight, and twice the accumulators, from the size of the L2 on.
+    // Not tied to the hint: the number of accumulators decides the bits of a sum.
+    const bool deep = vec && p.nout * p.R * (int64_t)sizeof(T) >= kStreamBytes;
     const bool wave_row = p.splits == 1 && p.R <= 1024;
     if (wave_row) {
         int64_t grid = (p.nout + kWaves - 1) / kWaves;
@@ -1058,9 +1061,10 @@ int launch_rows(const RedParams<T> &p, hipStream_t s)
         if (p.splits > 1) {
             if (p.nout > 65535) return ZENU_ERR_UNSUPPORTED;   // never: rows are split only when there are few of them
             const dim3 g((unsigned)p.splits, (unsigned)p.nout);
-            if (nt)       reduce_rows_kernel<T, Tr, VEC, kSplitRow, true, kSplitU><<<g, kBlock, 0, s>>>(p);
-            else if (vec) reduce_rows_kernel<T, Tr, VEC, kSplitRow, false, kRowsU><<<g, kBlock, 0, s>>>(p);
-            else          reduce_rows_kernel<T, Tr, 1, kSplitRow, false, kRowsU><<<g, kBlock, 0, s>>>(p);
+            if (nt)        reduce_rows_kernel<T, Tr, VEC, kSplitRow, true, kSplitU><<<g, kBlock, 0, s>>>(p);
+            else if (deep) reduce_rows_kernel<T, Tr, VEC, kSplitRow, false, kSplitU><<<g, kBlock, 0, s>>>(p);
+            else if (vec)  reduce_rows_kernel<T, Tr, VEC, kSplitRow, false, kRowsU><<<g, kBlock, 0, s>>>(p);
+            else           reduce_rows_kernel<T, Tr, 1, kSplitRow, false, kRowsU><<<g, kBlock, 0, s>>>(p);
         } else {
             if (nt)       reduce_rows_kernel<T, Tr, VEC, kBlockRow, true, kRowsU><<<(unsigned)grid, kBlock, 0, s>>>(p);
             else if (vec) reduce_rows_kernel<T, Tr, VEC, kBlockRow, false, kRowsU><<<(unsigned)grid, kBlock, 0, s>>>(p);
