@@ -413,3 +413,30 @@ def test_accumulators_of_shared_rows(hip, dtype, mbytes, accumulators):
         same((m.sum(1) if rows > 1 else m.sum_all()).to_numpy().reshape(rows), exp, ("sum", rows))
         if rows == 1:
             assert m.asum() == exp[0]
+
+
+# sources on both sides of the sizes from which a reduction streams its loads: 40 MB (f32), 64 MB with the ReLU gradient, 128 MB
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("mbytes", [39, 41, 63, 65, 126, 130])
+def test_reductions_of_large_sources_are_exact(hip, dtype, mbytes):
+    """small integers: every order of the sums gives the same value"""
+    cols = 2052
+    rows = mbytes * (1 << 20) // (cols * np.dtype(dtype).itemsize)
+    r = np.random.default_rng(mbytes)
+    a = r.integers(-4, 5, (rows, cols)).astype(dtype)
+    x = r.integers(-1, 2, (rows, cols)).astype(dtype)
+    for off in (0, 1):
+        m = offset_matrix(hip, a, off)
+        same(m.sum(0).to_numpy(), a.sum(0, dtype=np.float64), ("column sums", off))
+        same(m.sum(1).to_numpy(), a.sum(1, dtype=np.float64), ("row sums", off))
+        same(np.array(m.max_axis_idx_ravel(0)), a.argmax(0), ("rows of the column maxima", off))
+        same(np.array(m.max_axis_idx_ravel(1)), a.argmax(1), ("columns of the row maxima", off))
+        pieces = hip.Matrix(m.buf, m.offset, (rows, cols // 9, 9), (cols, 9, 1), dtype)
+        out = hip.Matrix.from_numpy(np.full((1, cols // 9, 1), 7, dtype))
+        hip.sum_to(pieces, out)
+        same(out.to_numpy().reshape(-1), a.reshape(rows, cols // 9, 9).sum((0, 2), dtype=np.float64), ("sums over pieces", off))
+        gx, gb = hip.Matrix.from_numpy(np.zeros((rows, cols), dtype)), hip.Matrix.from_numpy(np.zeros(cols, dtype))
+        gx.relu_backward_bias_grad(gb, m, offset_matrix(hip, x, off), 0.0)
+        g = np.where(x > 0, a, dtype(0))
+        same(gx.to_numpy(), g, ("ReLU gradient", off))
+        same(gb.to_numpy(), g.sum(0, dtype=np.float64), ("bias gradient", off))

@@ -1025,14 +1025,23 @@ __global__ __launch_bounds__(kBlock) void reduce_pieces_kernel(const T *src, T *
 
 // ---- host side ---------------------------------------------------------------------------------------------
 
-// A reduction writes next to nothing: a source of half the memory-side cache or less is loaded without the streaming hint
-// and stays there for the next reduction of the same tensor.  Column sums, row sums, two arg-maxima and the sum of
-// magnitudes of [10007,1003] f64 (80 MB) take 72.7 us, 76.3 with the hint, of [4000,4000] f32 61.8 / 63.1; of
-// [8192,4096] f32 (134 MB) 106.1 / 107.4, but there the first one, from memory, 24.8 / 23.8.
-constexpr int64_t kStreamSource = 4 * kStreamBytes;
+// A reduction writes next to nothing, so a source that is loaded without the streaming hint can stay in the caches for the
+// next reduction of the same tensor; a source that is read once is read faster with the hint.  us, plain / streaming, of a
+// tensor read once, read again by the same call, and by column sums, row sums, row maxima and sum of magnitudes in turn:
+//   f32  row sums [2075,4096] (34 MB) 7.5 / 7.2, 4.9 / 7.0; [2563,4096] (42 MB) 8.7 / 8.3, 8.0 / 8.1; [4882,4096] (80 MB) 14.5 /
+//        13.6, 13.5 / 13.4; column sums of these 11.6 / 10.9, 9.4 / 10.6; 12.0 / 11.7, 11.4 / 11.5; 17.6 / 16.8, 16.3 / 16.5; all four of
+//        [4000,4000] 51.2 / 51.2, of [6250,4000] (100 MB) 71.9 / 72.6: only the L2 keeps it, up to about 42 MB
+//   f64  row sums [2441,4096] (80 MB) 14.7 / 14.3, 13.6 / 14.0; column sums [9970,1003] 17.5 / 17.0, 16.4 / 16.8; all four of
+//        [2500,4000] 59.6 / 63.0, [9970,1003] 59.9 / 62.3, [3906,4000] (125 MB) 86.7 / 89.6
+//   sums over images and pixels f32 [398,256,196] (80 MB) 17.6 / 17.2, 15.9 / 17.1
+//   with the ReLU gradient (three times the source moved) f64 [15625,512] 38.0 / 34.9 once, between the calls that write
+//   its input and read its result 77.4 / 78.3; [21972,512] (90 MB) 51.2 / 46.9 and 105 / 106.3
+template <typename T> constexpr int64_t kStreamSource = sizeof(T) == 4 ? kStreamBytes / 4 * 5 : 4 * kStreamBytes;
+constexpr int64_t kStreamPieces = 4 * kStreamBytes, kStreamGradient = 2 * kStreamBytes;
+constexpr int64_t kRaggedBytes = 4 * kStreamBytes;   // see zenu_hip_relu_backward_bias_grad
 template <typename T> inline bool stream_source(const RedParams<T> &p)
 {
-    return p.nout * p.R * (int64_t)sizeof(T) >= kStreamSource;
+    return p.nout * p.R * (int64_t)sizeof(T) >= (p.pre_x ? kStreamGradient : kStreamSource<T>);
 }
 
 template <typename T, typename Tr>
@@ -1112,7 +1121,7 @@ int launch_cols(const RedParams<T> &p, hipStream_t s)
     const bool regular = g3 && p.cols_vec == VEC && shift == 5 && p.inner % per_tile == 0 && p.splits > 1 && p.fan >= p.splits && p.cstride == 1;
     if constexpr (!Tr::kHasIdx && std::is_same<Tr, SumTr<T>>::value) {
         if (p.pre_x) {
-            if (p.inner % VEC) {   // (below the streaming sizes: zenu_hip_relu_backward_bias_grad)
+            if (p.inner % VEC) {   // (no streaming instance: below kRaggedBytes)
                 reduce_cols_kernel<T, Tr, VEC, false, true, true><<<g, kBlock, 0, s>>>(p, ctl, shift, g3, banded);
             } else if (regular) {
                 if (nt) reduce_cols_regular_kernel<T, Tr, VEC, true, true><<<g, kBlock, 0, s>>>(p);
@@ -1393,7 +1402,7 @@ int sum_pieces(const T *src, int64_t N, int64_t C, int64_t I, T *out, hipStream_
     Workspace ws(splits > 1 ? (size_t)(C * splits) * sizeof(T) : 0, s);
     if (ws.status) return ws.status;
     T *const part = splits > 1 ? static_cast<T *>(ws.ptr) : out;
-    const bool nt = N * C * I * (int64_t)sizeof(T) >= kStreamSource;
+    const bool nt = N * C * I * (int64_t)sizeof(T) >= kStreamPieces;
     const unsigned grid = (unsigned)(C * splits);
     if (nt) reduce_pieces_kernel<T, VEC, true><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs, banded);
     else    reduce_pieces_kernel<T, VEC, false><<<grid, kBlock, 0, s>>>(src, part, (uint32_t)N, (uint32_t)C, I, (uint32_t)splits, (uint32_t)vecs, banded);
@@ -1747,14 +1756,14 @@ int zenu_hip_relu_backward_bias_grad(int dtype, const zenu_tensor_t *gx, const z
                  is_default_stride_strict(*gy) && is_default_stride_strict(*x) && is_default_stride_strict(*gbias);
     if (fused) {
         // Whole aligned vectors; or any rows of which the sums take vectors of columns as well (the bias gradient has the
-        // bits of sum_to, see kNarrowRows), below the streaming sizes, where lines shared by two rows cost more: f32, us
+        // bits of sum_to, see kNarrowRows), below kRaggedBytes, where lines shared by two rows cost more: f32, us
         // as two calls / in one launch, [402,1497] 7.5 / 5.4, [724,1397] 9.7 / 7.7, [1000,1499] 10.1 / 8.9, [500,301] 7.0 / 5.2;
         // f64 [1000,1499] 14.0 / 11.3; but f32 [30000,1499] 123 / 141.
         const int64_t n = gx->shape[gx->ndim - 1], vec = 16 / (int64_t)esz;
         const bool whole = n % vec == 0 && aligned16(gx->ptr) && aligned16(x->ptr) && aligned16(gy->ptr);
         // (sum_to has no sums to make, but a copy, where gbias has the shape of gx: it keeps the sign of a zero)
         int axes[kMaxDim * 2], keep[kMaxDim * 2], na;
-        const bool ragged = (n >= kColsTx * vec || (n >= vec && num_elm(*gy) / n > kNarrowRows)) && num_elm(*gy) * (int64_t)esz < kStreamSource &&
+        const bool ragged = (n >= kColsTx * vec || (n >= vec && num_elm(*gy) / n > kNarrowRows)) && num_elm(*gy) * (int64_t)esz < kRaggedBytes &&
                             sum_to_axes(*gx, *gbias, axes, keep, na) == ZENU_OK && na > 0;
         fused = gbias->shape[gbias->ndim - 1] == n && num_elm(*gbias) == n && (whole || ragged);
     }
