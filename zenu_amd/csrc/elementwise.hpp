@@ -252,19 +252,21 @@ template <typename T> struct CopyF {
 
 // ---- how a kernel's operands pass the caches --------------------------------------------------------
 // Below kStreamBytes: no hints.  Above, stores stream (a store that allocates pushes out what the next call reads), and
-//   kMemKeep    inputs are loaded plainly while the call's operands fit the 256 MB memory-side cache: they are often read
-//               again, a data matrix by the next statistic, a forward input by the backward pass.
+//   kMemKeep    inputs are loaded plainly while those of full size are below kKeepInputs: they are often read again, a data
+//               matrix by the next statistic, a forward input by the backward pass.
 //   kMemFeed    a layer's own step, whose result is what the next call reads: ReLU, its backward pass, a bias per channel
 //               or row.  Written through without the hint, it waits in the memory-side cache; the inputs stream.
 //   kMemStream  beyond that everything streams.
-// us with everything streaming / by these rules, three sets of operands in turn: bias, ReLU, NCHW -> NHWC, ReLU backward,
-// bias gradient of [64,512,14,14] f32 53.5 / 47.7 (257 MB moved), [64,256,28,28] 95.8 / 88.2, f64 [16,64,56,56] 54.8 /
-// 49.5; a + row, a * column, a + b^T, 0.5 a of [3001,2047] f32 43.2 / 38.6, [2000,4000] 55.0 / 46.3, [4096,4096] 102.1 /
-// 92.6; ReLU and its backward pass of 8 million 27.9 / 25.7; sigmoid's of 2^24 62.6 / 59.5.
-// Where the lines lie: keeping the inputs of 537 MB calls, ReLU of 2^26 80 / 86 us, backward 128 / 140; feeding from the
-// 201 MB of a ReLU backward of 2^24 31.7 / 33.6, from 154 MB 24.9 / 24.1.
+// us, plain loads / streaming, f32, operands used once and by three calls in turn: a + b of 36 MB 7.7 / 7.5, 4.7 / 7.2; 64 MB
+// 12.5 / 12.0, 11.0 / 11.7; 96 MB 17.7 / 16.9, 15.5 / 16.5; 128 MB 22.9 / 21.5, 20.2 / 21.2; 201 MB 34.9 / 32.2, 30.4 / 31.8; copy of 64 MB
+// 11.5 / 11.2, 9.3 / 9.9; 128 MB 21.5 / 20.7, 19.5 / 20.4; 160 MB 26.5 / 25.2, 24.0 / 25.1; 250 MB 40.4 / 38.3, 36.5 / 38.0; a + b^T 64 MB
+// 13.7 / 13.2, 11.7 / 12.9; 195 MB 35.0 / 32.9, 31.1 / 32.7.  Above 72 MB of inputs what is lost by the first use is more than a later one gains.
+// us with everything streaming / by these rules: bias, ReLU, NCHW -> NHWC, ReLU backward, bias gradient of [64,512,14,14]
+// f32 53.5 / 47.7 (257 MB moved), [64,256,28,28] 95.8 / 88.2, f64 [16,64,56,56] 54.8 / 49.5; a + row, a * column, a + b^T, 0.5 a
+// of [3001,2047] f32 45.5 / 42.5, [2000,4000] 54.6 / 49.3, [4096,4096] 102.4 / 92.8; ReLU and its backward pass of 8 million 27.9 / 25.7.
+// Feeding from the 201 MB of a ReLU backward of 2^24 on loses, 31.7 / 33.6; at 154 MB 24.9 / 24.1.
 enum { kMemCached, kMemKeep, kMemFeed, kMemStream };
-constexpr int64_t kKeepBytes = 8 * kStreamBytes, kFeedBytes = 6 * kStreamBytes;
+constexpr int64_t kKeepInputs = 72ll << 20, kFeedBytes = 6 * kStreamBytes;
 constexpr bool streams_loads(int mem) { return mem == kMemStream || mem == kMemFeed; }
 
 // ONE_IN: one input streams beside the output (the written-through streaming store, vecmem.hpp)
@@ -1128,11 +1130,13 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
     const int nin = F::NIN;
     const int64_t moved = p.numel * (int64_t)sizeof(T) * (nin + 1);
     const bool nt = moved >= kStreamBytes;
+    // whether inputs of which `full` have the size of the output stay in the caches, see kMemKeep
+    auto keeps = [&](int full) { return p.numel * (int64_t)sizeof(T) * full < kKeepInputs; };
     // calls go(mem) with the way past the caches as a constant; feed: see kMemFeed
-    auto with_mem = [&](auto feed, auto go) {
+    auto with_mem = [&](auto feed, int full, auto go) {
         constexpr bool FEED = decltype(feed)::value;
         if (!nt) go(std::integral_constant<int, kMemCached>());
-        else if (moved < (FEED ? kFeedBytes : kKeepBytes)) go(std::integral_constant<int, FEED ? kMemFeed : kMemKeep>());
+        else if (FEED ? moved < kFeedBytes : keeps(full)) go(std::integral_constant<int, FEED ? kMemFeed : kMemKeep>());
         else go(std::integral_constant<int, kMemStream>());
     };
     if (p.ndim == 0) {  // a single element
@@ -1160,7 +1164,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
         int64_t tile = (int64_t)cb * VEC * cu;
         int64_t grid = (n + tile - 1) / tile;
         if (grid > 0x7fffffffLL) return ZENU_ERR_UNSUPPORTED;
-        with_mem(std::integral_constant<bool, IsLayerStep<F>::value>(), [&](auto mem) {
+        with_mem(std::integral_constant<bool, IsLayerStep<F>::value>(), nin, [&](auto mem) {
             ew_contig_kernel<T, VEC, decltype(mem)::value, F><<<(unsigned)grid, cb, 0, stream>>>(out, a, b, n, f);
         });
         ZENU_LAUNCH_CHECK();
@@ -1214,7 +1218,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                         constexpr int B = small ? ZENU_EW1_BLOCK : 256, U = small ? ZENU_EW1_UNROLL : 2;
                         const int64_t tile = (int64_t)B * VEC * U;
                         const unsigned grid = (unsigned)((p.numel + tile - 1) / tile);
-                        with_mem(std::integral_constant<bool, IsAdd<F>::value && (MODE == 1 || MODE == 2)>(), [&](auto mem) {
+                        with_mem(std::integral_constant<bool, IsAdd<F>::value && (MODE == 1 || MODE == 2)>(), nin - 1, [&](auto mem) {
                             ew_periodic_kernel<T, VEC, decltype(mem)::value, F, YF, MODE, B, U><<<grid, B, 0, stream>>>(out, x, y, n32, in32, mid32, f);
                         });
                     };
@@ -1355,7 +1359,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                     if (tiles <= 0x7fffffffLL) {
                         const dim3 g((unsigned)tiles, (unsigned)tp.nbatch);
                         const size_t lds = (size_t)q.nshort * q.lds_pitch * sizeof(T);
-                        with_mem(std::false_type(), [&](auto mem) {
+                        with_mem(std::false_type(), 1, [&](auto mem) {
                             if (thin_out) ew_thin_kernel<T, decltype(mem)::value, true><<<g, kBlock, lds, stream>>>(out, a, q);
                             else          ew_thin_kernel<T, decltype(mem)::value, false><<<g, kBlock, lds, stream>>>(out, a, q);
                         });
@@ -1424,7 +1428,7 @@ template <typename T, typename F> int launch_ew(EwProblem &p, F f, hipStream_t s
                 const size_t lds = (size_t)(tp.trans_a + tp.trans_b) * kTile * (kTile + 1) * sizeof(T);
                 constexpr int kThreads = TileThreads<T, F, SMALL>::value;
                 if constexpr (!NT) ew_tile_kernel<T, kMemCached, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
-                else if (moved < kKeepBytes) ew_tile_kernel<T, kMemKeep, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
+                else if (keeps(nin)) ew_tile_kernel<T, kMemKeep, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
                 else ew_tile_kernel<T, kMemStream, F, SMALL><<<g, kThreads, lds, stream>>>(out, a, b, tp, f);
                 return ZENU_OK;
             };
