@@ -242,6 +242,91 @@ def test_softmax_staged_rows(hip, dtype, shape):
     assert np.array_equal(m.to_numpy(), out.to_numpy())
 
 
+def same_numbers(got, exp, what):
+    """the same bits, but for which of the NaNs a NaN is"""
+    nan = np.isnan(exp)
+    assert np.array_equal(np.isnan(got), nan), what
+    assert bits_equal(np.where(nan, 0, got), np.where(nan, 0, exp)), what
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", STAGED_SHAPES, ids=str)
+def test_softmax_staged_rows_have_the_bits_of_the_chain(hip, dtype, shape):
+    """the maximum, the sums and the division of the op-by-op chain, in its order, with every kind of number among them: NaN in
+    front of a line and elsewhere, infinities of either sign, lines of one value, of -inf only and with a single finite one"""
+    n = shape[1]
+    r = np.random.default_rng(n)
+    x = (r.standard_normal(shape, dtype=np.float32) * 4).astype(dtype)
+    gy = r.standard_normal(shape, dtype=np.float32).astype(dtype)
+    lines = np.moveaxis(x, 1, 2).reshape(-1, n).copy()
+    grads = np.moveaxis(gy, 1, 2).reshape(-1, n).copy()
+    put = [lambda l: l.__setitem__(0, np.nan), lambda l: l.__setitem__(n // 2, np.nan), lambda l: l.__setitem__(n - 1, np.inf),
+           lambda l: l.__setitem__(0, -np.inf), lambda l: l.fill(-np.inf), lambda l: l.fill(1.5), lambda l: l.__setitem__(slice(0, n - 1), -np.inf),
+           lambda l: l.__setitem__(slice(0, n, 2), -60), lambda l: None]
+    for i in range(0, len(lines), 3):                        # every third line, so that each has plain neighbours
+        put[i // 3 % len(put)](lines[i])
+    for i in range(1, len(grads), 7):
+        grads[i, i % n] = (np.inf, np.nan, -0.0)[i % 3]
+    outer, _, inner = shape
+    x, gy = (np.ascontiguousarray(np.moveaxis(l.reshape(outer, inner, n), 2, 1)) for l in (lines, grads))
+    with np.errstate(all="ignore"):
+        ref = CpuMatrix.zeros(shape, dtype)
+        ref.softmax_assign(CpuMatrix.from_numpy(x), 1)
+        out = hip.Matrix.zeros(shape, dtype)
+        out.softmax_assign(hip.Matrix.from_numpy(x), 1)
+        y = out.to_numpy()
+        same_numbers(y, ref.a, "softmax")
+        exp = cpu_matrix.softmax_backward(CpuMatrix.from_numpy(y), CpuMatrix.from_numpy(gy), 1).a
+        same_numbers(hip.softmax_backward(out, hip.Matrix.from_numpy(gy), 1).to_numpy(), exp, "backward")
+
+
+# Streamed rows by the way they are stored, see softmax_forward_launch: whole aligned rows beyond 4096 elements (written
+# through), many ragged rows with a result of 32 MB or more (plainly), few ragged rows (past the caches); whole aligned rows of
+# up to 4096 elements (a kernel of their own)
+STREAMED_ROWS = [(1100, 8192), (300, 16384), (270, 32768), (1100, 4100), (2100, 4099), (1030, 8195), (600, 8191), (150, 32735), (4200, 4096), (9000, 1020)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", STREAMED_ROWS, ids=str)
+def test_softmax_streamed_rows(hip, dtype, shape):
+    """against 80-bit sums with the bounds of test_softmax_kernel_edges, every operand at a 16-byte boundary, nothing written
+    around the result, and the same bits in place"""
+    print(f"[case] streamed softmax {shape} {np.dtype(dtype).name}", flush=True)
+    rows, n = shape
+    r = np.random.default_rng(n)
+    x = (r.standard_normal(shape, dtype=np.float32) * 3).astype(dtype)
+    gy = r.standard_normal(shape, dtype=np.float32).astype(dtype)
+    eps, tiny = np.finfo(dtype).eps, np.finfo(dtype).tiny
+
+    def framed(a):
+        m = hip.Matrix.from_numpy(np.concatenate([np.full(4, 7, dtype), a.reshape(-1), np.full(5, 7, dtype)]))
+        return hip.Matrix(m.buf, 4, shape, hip.default_stride(shape), dtype)
+
+    def frame_is_whole(m):
+        ends = hip.Matrix(m.buf, 0, (m.num_elm() + 9,), (1,), dtype).to_numpy()
+        return np.all(ends[:4] == 7) and np.all(ends[-5:] == 7)
+
+    X, out, gx = framed(x), framed(np.zeros_like(x)), framed(np.zeros_like(x))
+    out.softmax_assign(X, 1)
+    y = out.to_numpy()
+    hip._lib.check(hip.lib().zenu_hip_softmax_backward(hip._lib.F32 if dtype == np.float32 else hip._lib.F64, C.byref(gx.desc()),
+                   C.byref(out.desc()), C.byref(framed(gy).desc()), 1, None), "softmax_backward")
+    got = gx.to_numpy()
+    X.softmax_assign(X, 1)
+    assert bits_equal(X.to_numpy(), y)
+    assert frame_is_whole(X) and frame_is_whole(out) and frame_is_whole(gx)
+    for i in range(0, rows, 512):                            # (80-bit copies of some rows at a time)
+        at = slice(i, i + 512)
+        d = x[at].astype(np.longdouble) - x[at].max(axis=1, keepdims=True)
+        e = np.exp(d)
+        exact = e / e.sum(axis=1, keepdims=True)
+        assert np.all(np.abs(y[at] - exact) <= (n + 3 + 2 * np.abs(d)) * eps * exact + tiny)
+        t = y[at].astype(np.longdouble) * gy[at]
+        exact = t - y[at] * t.sum(axis=1, keepdims=True)
+        bound = (n + 2) * eps * np.abs(t).sum(axis=1, keepdims=True) * y[at] + 3 * eps * np.abs(t)
+        assert np.all(np.abs(got[at] - exact) <= bound + tiny)
+
+
 # Rows for the exact test below: few and many, around each limit of a wavefront, of 256 threads (single elements and
 # vectors) and of larger workgroups, totals below and above the streaming size.  Powers of two of them, see below.
 EXACT_ROWS = [(4, 65), (512, 127), (1024, 128), (2048, 255), (512, 256), (1024, 300), (512, 511), (2048, 512), (2048, 513), (4, 600),
