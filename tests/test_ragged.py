@@ -440,3 +440,139 @@ def test_reductions_of_large_sources_are_exact(hip, dtype, mbytes):
         g = np.where(x > 0, a, dtype(0))
         same(gx.to_numpy(), g, ("ReLU gradient", off))
         same(gb.to_numpy(), g.sum(0, dtype=np.float64), ("bias gradient", off))
+
+
+# Copies with a short side by the positions a workgroup takes, 2^7 to 2^11 of them (see the rule where ew_thin_kernel is
+# launched), last workgroups that are not full, 16 KB of a workgroup filled and not, and sizes on both sides of those from
+# which the stores stream and from which the loads do
+THIN = [(128, 3, 12545), (600, 2, 1027), (300, 2, 20001), (200, 8, 3137), (64, 8, 3137), (16, 24, 12547), (90, 5, 9001), (150, 16, 2051), (128, 3, 32769), (270, 3, 32771)]
+
+
+def thin_log_run(n, short, long, size):
+    log_run = 6
+    while short * size << (log_run + 1) <= 16384:
+        log_run += 1
+    while log_run > 6 and n * -(-long // (1 << log_run)) < 4 * 256:
+        log_run -= 1
+    return log_run
+
+
+def test_short_sides_reach_every_length_of_run():
+    assert {thin_log_run(*s, 4) for s in THIN} >= {7, 8, 9, 10, 11} and {thin_log_run(*s, 8) for s in THIN} >= {6, 7, 8, 9, 10}
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("shape", THIN, ids=str)
+def test_copies_with_one_short_side_and_long_runs(hip, dtype, shape):
+    n, short, long = shape
+    a = np.random.default_rng(long).standard_normal(shape, dtype=np.float32).astype(dtype)
+    flipped = np.ascontiguousarray(a.transpose(0, 2, 1))
+    for off, end in ((0, 0), (1, 2)):
+        def framed(x):
+            m = hip.Matrix.from_numpy(np.concatenate([np.full(off, 7, dtype), x.reshape(-1), np.full(9, 7, dtype)]))
+            return hip.Matrix(m.buf, off, x.shape, hip.default_stride(x.shape), dtype)
+
+        def frame_is_whole(m):
+            ends = hip.Matrix(m.buf, 0, (off + a.size + 9,), (1,), dtype).to_numpy()
+            return np.all(ends[:off] == 7) and np.all(ends[-9:] == 7)
+        A, out, back = framed(a), framed(np.zeros_like(flipped)), framed(np.zeros_like(a))
+        out.copy_from(A.transpose())
+        same(out.to_numpy(), flipped, ("into the short side", off))
+        back.copy_from(out.transpose())
+        same(back.to_numpy(), a, ("out of it", off))
+        assert frame_is_whole(out) and frame_is_whole(back)
+
+
+# Elementwise kernels by the way their operands pass the caches: megabytes of one operand such that one and two inputs are
+# cached, kept, fed to the next call and streamed (32 MB moved; 72 MB of inputs; 192 MB moved)
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("mbytes", [13, 20, 38, 80, 105])
+def test_elementwise_calls_of_every_size_class(hip, dtype, mbytes):
+    cols = 2052
+    rows = mbytes * (1 << 20) // (cols * np.dtype(dtype).itemsize) // 9 * 9 + 9
+    r = np.random.default_rng(mbytes)
+    shape, (n, c, hw) = (rows, cols), (rows // 9, 12, 9 * cols // 12)
+    a, b = (r.standard_normal(shape, dtype=np.float32).astype(dtype) for _ in range(2))
+    row, column, channel = (r.standard_normal(k, dtype=np.float32).astype(dtype) for k in ((cols,), (rows, 1), (1, c, 1)))
+    for off in (0, 1):
+        out = hip.Matrix.from_numpy(np.full(rows * cols + 16, 7, dtype))
+
+        def into(s):
+            return hip.Matrix(out.buf, off, s, hip.default_stride(s), dtype)
+
+        def check(fn, exp, what):
+            m = into(exp.shape)
+            fn(m)
+            same(m.to_numpy(), exp, (what, off))
+            ends = hip.Matrix(out.buf, 0, (off + exp.size + 8,), (1,), dtype).to_numpy()
+            assert np.all(ends[:off] == 7) and np.all(ends[-8:] == 7), (what, off)
+        A, B = offset_matrix(hip, a, off), offset_matrix(hip, b, off)
+        Row, Column, Channel = (hip.Matrix.from_numpy(x) for x in (row, column, channel))
+        images = hip.Matrix(A.buf, off, (n, c, hw), hip.default_stride((n, c, hw)), dtype)
+        check(lambda m: m.add_array(A, B), a + b, "a + b")
+        check(lambda m: m.copy_from(A), a, "copy")
+        check(lambda m: m.abs_array(A), np.abs(a), "abs")
+        check(lambda m: m.relu(A, 0.5), np.where(a > 0, a, a * dtype(0.5)), "relu")
+        check(lambda m: m.relu_backward(B, A, 0.5), b * np.where(a > 0, dtype(1), dtype(-0.5)), "relu backward")
+        check(lambda m: m.add_array(A, Row), a + row, "a + row")
+        check(lambda m: m.mul_array(A, Column), a * column, "a * column")
+        check(lambda m: m.add_array(images, Channel), a.reshape(n, c, hw) + channel, "images + channel")
+        check(lambda m: m.broadcast(Row), np.broadcast_to(row, shape), "broadcast")
+        turned = hip.Matrix(B.buf, off, (cols, rows), (rows, 1), dtype)
+        check(lambda m: m.add_array(A, turned.transpose()), a + b.reshape(cols, rows).T, "a + b^T")
+        check(lambda m: m.copy_from(turned.transpose()), np.ascontiguousarray(b.reshape(cols, rows).T), "transposed copy")
+        check(lambda m: m.abs_array(turned.transpose()), np.abs(b.reshape(cols, rows).T), "transposed abs")
+        check(lambda m: m.add_array(m, B), into(shape).to_numpy() + b, "in place")
+
+
+def in_steps(x, lanes):
+    """the lanes' sums added as the column kernels add them: lanes 0 .. 7 first take every eighth, then lane 0 the rest"""
+    x = [x[i] for i in range(lanes)]
+    if lanes > 8:
+        for i in range(8):
+            for w in range(i + 8, lanes, 8):
+                x[i] = x[i] + x[w]
+    for w in range(1, min(lanes, 8)):
+        x[0] = x[0] + x[w]
+    return x[0]
+
+
+def column_sums_in_order(a, lanes, splits):
+    """every `lanes` rows of a chunk of four times as many go to the lanes, the chunks to the splits in turn"""
+    rows, cols = a.shape
+    partial = []
+    for s in range(splits):
+        acc = np.zeros((lanes, cols), a.dtype)
+        for b in range(s * 4 * lanes, rows, splits * 4 * lanes):
+            for r in range(b, min(b + 4 * lanes, rows), lanes):
+                part = a[r:r + lanes]
+                acc[:len(part)] = acc[:len(part)] + part
+        partial.append(in_steps(acc, lanes))
+    if splits == 1:
+        return partial[0]
+    acc = np.zeros((lanes, cols), a.dtype)
+    for s in range(splits):
+        acc[s % lanes] = acc[s % lanes] + partial[s]
+    return in_steps(acc, lanes)
+
+
+# The order of column sums, with and without a launch of their own for the splits: (rows, columns, log2 of the lanes along a
+# row, splits), lanes and splits as the rule of the dispatch has them on 256 CUs
+ORDERS = {np.float32: [(1000, 640, 5, 16), (3000, 400, 5, 47), (3000, 200, 3, 12), (1100, 1500, 5, 18), (520, 2100, 5, 9), (30000, 65, 3, 118), (3001, 65, 3, 12)],
+          np.float64: [(1000, 300, 5, 16), (3000, 400, 5, 47), (1100, 1500, 5, 18), (520, 2100, 5, 9), (30000, 33, 3, 118)]}
+
+
+@pytest.mark.parametrize("dtype,geometry", [(d, g) for d in DTYPES for g in ORDERS[d]], ids=str)
+def test_order_of_column_sums(hip, dtype, geometry):
+    rows, cols, shift, splits = geometry
+    r = np.random.default_rng(rows)
+    a = (r.standard_normal((rows, cols)) * 10.0 ** r.integers(-3, 4, (rows, 1))).astype(dtype)
+    a[5] = -0.0
+    exp = column_sums_in_order(a, 256 >> shift, splits)
+    m, out = hip.Matrix.from_numpy(a), hip.Matrix.zeros((cols,), dtype)
+    hip.sum_to(m, out)
+    got = out.to_numpy()
+    same(got.view(np.uint8), exp.view(np.uint8), "column sums")
+    gx, gb = hip.Matrix.zeros(a.shape, dtype), hip.Matrix.zeros((cols,), dtype)
+    gx.relu_backward_bias_grad(gb, m, hip.Matrix.from_numpy(np.ones_like(a)), 0.0)
+    same(gb.to_numpy().view(np.uint8), exp.view(np.uint8), "with the ReLU gradient")
