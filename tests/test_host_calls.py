@@ -2,6 +2,12 @@
 results, the same errors, and what it does not take goes the ctypes way unchanged."""
 import ctypes as C
 import gc
+import glob
+import os
+import shutil
+import subprocess
+import sys
+import sysconfig
 import weakref
 
 import numpy as np
@@ -55,6 +61,32 @@ def test_transposed_view():
     assert _pyhost.transpose(Derived(Memory(4096), 0, (2, 3), (3, 1), np.float32)) is None
     u = Derived(Memory(4096), 0, (2, 3), (3, 1), np.float32).transpose()
     assert (u.shape, u.stride) == ((3, 2), (1, 3))
+
+
+def test_module_is_built_for_this_interpreter_alone(tmp_path):
+    """its name carries the interpreter's tag, and an interpreter that there is none for imports the package all the same"""
+    package = os.path.dirname(zenu_amd.__file__)
+    assert _pyhost.__file__ == os.path.join(package, "_pyhost" + sysconfig.get_config_var("EXT_SUFFIX")) and zenu_amd.matrix._pyhost is _pyhost
+    assert not os.path.exists(os.path.join(package, "_pyhost.so"))
+    copy = tmp_path / "zenu_amd"
+    copy.mkdir()
+    for f in glob.glob(os.path.join(package, "*.py")):
+        shutil.copy(f, copy)
+    os.symlink(os.path.join(package, "lib"), copy / "lib")
+    program = """
+import numpy as np, zenu_amd as z
+class Memory: ptr = 4096
+m = z.Matrix(Memory(), 0, (2, 3), (3, 1), np.float32)
+t = m.transpose()
+assert (t.shape, t.stride) == ((3, 2), (1, 3)) and t.desc().ptr == 4096
+z.lib()
+try:
+    m.add_array(z.Matrix(Memory(), 0, (4, 5), (5, 1), np.float32), m)
+except z.ZenuHipError:
+    print("refused")
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout == "refused\n", done.stderr
 
 
 def test_optimizer_operands_are_held_while_they_are_read():

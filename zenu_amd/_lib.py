@@ -1,15 +1,34 @@
 """ctypes binding of libzenu_hip.so (the C ABI declared in include/zenu_hip.h).
 
-The library is built in-tree by zenu_amd/csrc/Makefile.  There is no CPU fallback: if the
-shared object is missing, loading fails loudly.
+The library is built in-tree by zenu_amd/csrc/Makefile.  There is no CPU fallback: if
+libzenu_hip.so is missing, loading fails loudly.
 """
 import ctypes as C
+import importlib.util
 import os
 
-try:
-    from . import _pyhost
-except ImportError as e:
-    raise ImportError("zenu_amd/_pyhost.so is missing: build it with `make -C zenu_amd/csrc` (or __graft_entry__.build())") from e
+
+class _CtypesOnly:
+    """in place of _pyhost for an interpreter that none is built for: declines every call"""
+
+    def __getattr__(self, name):
+        return _decline if name in ("pack", "transpose", "setup", "bind") else _decline_call
+
+
+def _decline(*_):
+    return None
+
+
+def _decline_call(*_):
+    return False
+
+
+# The native host side of calls (csrc/pyhost.cpp).  Where there is none every call goes through ctypes, with the same results
+# and 2 us more; one that does not load is an error.
+if importlib.util.find_spec(__package__ + "._pyhost") is None:
+    pyhost = _CtypesOnly()
+else:
+    from . import _pyhost as pyhost
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libzenu_hip.so")
@@ -164,7 +183,7 @@ def lib():
     l.zenu_hip_validated_libm.restype = C.c_char_p
     l.zenu_hip_last_hip_error_string.argtypes = []
     l.zenu_hip_last_hip_error_string.restype = C.c_char_p
-    _pyhost.bind(l._handle)
+    pyhost.bind(l._handle)
     _lib = l
     return l
 

@@ -25,8 +25,8 @@ import struct
 
 import numpy as np
 
-from . import _lib, _pyhost
-from ._lib import ZenuHipError, Tensor, check
+from . import _lib
+from ._lib import ZenuHipError, Tensor, check, pyhost as _pyhost
 
 _stream = None  # hipStream_t as int / None = null stream
 

@@ -13,8 +13,8 @@ import ctypes as C
 
 import numpy as np
 
-from . import _lib, _pyhost
-from ._lib import check
+from . import _lib
+from ._lib import check, pyhost as _pyhost
 from .matrix import Matrix, get_stream, _dt
 
 
