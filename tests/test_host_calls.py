@@ -89,6 +89,19 @@ except z.ZenuHipError:
     assert done.returncode == 0 and done.stdout == "refused\n", done.stderr
 
 
+def test_a_module_without_a_tag_is_taken_away(tmp_path):
+    """such as builds left before modules were named after their interpreter: any interpreter would load it"""
+    package = os.path.dirname(zenu_amd.__file__)
+    (tmp_path / "zenu_amd" / "csrc").mkdir(parents=True)
+    for f in ("Makefile", "pyhost.cpp"):
+        shutil.copy(os.path.join(package, "csrc", f), tmp_path / "zenu_amd" / "csrc")
+    os.symlink(os.path.join(os.path.dirname(package), "include"), tmp_path / "include")
+    (tmp_path / "zenu_amd" / "_pyhost.so").write_bytes(b"")
+    module = "_pyhost" + sysconfig.get_config_var("EXT_SUFFIX")
+    subprocess.run(["make", "-C", str(tmp_path / "zenu_amd" / "csrc"), "../" + module, "PYTHON=" + sys.executable], check=True, capture_output=True, timeout=100)
+    assert [f for f in os.listdir(tmp_path / "zenu_amd") if f.endswith(".so")] == [module]
+
+
 def test_optimizer_operands_are_held_while_they_are_read():
     """reading a buffer's address can run code that takes the entry, its moments and its name away"""
     zenu_amd.lib()
