@@ -325,10 +325,13 @@ int zenu_hip_bias_add_relu(int dtype, const zenu_tensor_t *pre, const zenu_tenso
  * sums (the bias gradient: zenu-layer/src/layers/linear.rs:27-31 through the `sum_to` of
  * zenu-autograd/src/lib.rs:466-486).  Both in one pass over the incoming gradient:
  *   gx = gy * relu'(x)   (zenu_hip_relu_backward),   gbias[j] = sum over every leading index of gx[.., j]
- * gx, gy, x have the same shape [.., N]; gbias holds N elements ([N], [1, N], ..).  One launch (the
- * column-reduction kernel with the ReLU gradient applied to its loads) when the tensors are whole,
- * 16-byte aligned and N is a multiple of the vector width and at least 16; otherwise the two calls it
- * stands for.  gx is bit-identical to zenu_hip_relu_backward's and, for a 2-d gradient, gbias to
+ * gx, gy, x have the same shape [.., N]; gbias holds N elements ([N], [1, N], ..).  One pass (the
+ * column-reduction kernel with the ReLU gradient applied to its loads, behind it a second launch that
+ * folds the sums where a source of 4 MB or more is split over many workgroups) when the tensors are whole, N is at least 16 and either
+ *   - the tensors are 16-byte aligned and N is a multiple of the vector width (4 f32, 2 f64), or
+ *   - they hold less than 128 MiB each and N is at least 32 vectors, or there are more than 1024 rows;
+ * otherwise the two calls it stands for.  gx may be gy or x itself, but share memory with neither in
+ * another way.  gx is bit-identical to zenu_hip_relu_backward's and, for a 2-d gradient, gbias to
  * zenu_hip_sum_to(gbias, gx).
  * No counterpart in the reference (two autograd nodes there). */
 int zenu_hip_relu_backward_bias_grad(int dtype, const zenu_tensor_t *gx, const zenu_tensor_t *gbias,

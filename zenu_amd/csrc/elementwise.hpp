@@ -764,7 +764,7 @@ __global__ __launch_bounds__((TileThreads<T, F, SMALL>::value)) void ew_tile_ker
         constexpr bool EDGE = decltype(edge_c)::value;
         // vector e = k * kBlock + tid of the tile: eight consecutive ones form a segment, the segments
         // of one segment column follow each other along the other dim
-        constexpr int K = kTile * SEG * VPS / kBlock;   // vectors per thread and operand (1 or 4)
+        constexpr int K = kTile * SEG * VPS / kBlock;   // vectors per thread and operand (1 or 2)
         const int seg_v = (tid % VPS) * VEC;            // vector position inside the segment
         auto other_of = [&](int k) { return ((k * kBlock + tid) / VPS) % kTile; };                  // position along the other dim
         auto vec_of = [&](int k) { return seg_v + (((k * kBlock + tid) / VPS) / kTile) * VPS * VEC; };  // element position along the vector dim

@@ -1167,8 +1167,11 @@ inline bool staged_rows(const Geometry &g)
 // How the lines kernels write (us, left in the L2 / written through): all wavefronts of a launch store at about the same
 // time, and what is dirty in the L2 then is written back behind the last of them.  Softmax [16,21,16384] f32 14.8 / 12.5,
 // [2,32,16083] 5.4 / 4.7, [32,120,3136] 25.9 / 23.7, f64 [16,21,8000] 15.6 / 13.7; backward 11.4 / 10.9, 4.1 / 3.6, f64 11.4 /
-// 10.9, but larger results stream better through the L2 ([8,21,50000] 17.5 / 17.8).  Staged rows: [65536,64] 16.3 / 14.1 and
-// 15.8 / 13.6.  Where neighbouring lanes do not write neighbouring elements the L2 has to collect them ([65536,3] 3.0 / 3.2).
+// 10.9, but a larger result of the same operands again and again streams better through the L2 ([8,21,50000] 17.5 / 17.8).  Forward
+// there is no such size; operands used once, softmax alone and with its backward pass behind it: f32 [32,21,65536] (176 MB)
+// 67.7 / 65.7 and 163.5 / 160.9, [2048,5,12544] (514 MB) 222 / 215 and 489 / 484, [16,150,65536] (629 MB) 257 / 255 and 632 / 630, f64
+// [32,21,65536] 130.1 / 128.6 and 319 / 317.  Staged rows: [65536,64] 16.3 / 14.1 and 15.8 / 13.6, used once [1048576,64] (268 MB)
+// 113.0 / 112.7 and, backward, 153.8 / 153.6.  Where neighbouring lanes do not write neighbouring elements the L2 has to collect them ([65536,3] 3.0 / 3.2).
 inline int line_mode(const Geometry &g, bool forward, size_t size)
 {
     if (staged_rows(g)) return kLinesStaged;

@@ -254,8 +254,10 @@ template <typename T> struct RedParams {
     // optional transform of the source on its way in (column kernels, vector path, sums only):
     // the reduced value is in[i] * (pre_x[i] > 0 ? 1 : pre_alpha * -1), the gradient of ReLU
     // (zenu-autograd/src/activation/relu.rs:35-44), which is also stored to pre_out[i]; the three
-    // arrays share the source's layout.  Every source element is loaded by exactly one thread of
-    // the launch, so every element of pre_out is written once.
+    // arrays share the source's layout, and pre_out may be the source or pre_x.  Every element of pre_out is
+    // written by one thread.  Where rows are no whole number of vectors (RAGGED) a row's last vector reaches back
+    // into columns of its neighbour, which may have written them already: what is loaded there may enter neither
+    // a sum nor an output.
     const T *pre_x;
     T *pre_out;
     T pre_alpha;

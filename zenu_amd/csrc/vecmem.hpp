@@ -5,7 +5,7 @@
 // TB/s): the lines do not linger in L2 / the memory-side cache on their way through.  The hint
 // is used only when an op moves more than kStreamBytes; smaller operands keep normal caching so
 // that a following op can find them in L2.  Which of the loads and stores carry it then depends on who reads the operands
-// next: elementwise.hpp (kMemKeep, kMemFeed), fused.hip (softmax rows) and reduce.hip (kStreamSource) say so.
+// next: elementwise.hpp (kMemKeep, kMemFeed), fused.hip (softmax rows, line_mode) and reduce.hip (kStreamSource) say so.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
