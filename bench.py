@@ -309,7 +309,7 @@ def build_ops(z, workload, stream):
         row = r.standard_normal(n).astype(np.float32)
         nb = 4 * n * n
         sets = [(M.from_numpy(a), M.from_numpy(pos), M.from_numpy(unit), M.from_numpy(row), M.alloc((n, n)), M.alloc((n,)), M.alloc(()))
-                for _ in range(nsets(4 * nb))]
+                for _ in range(nsets(2 * nb))]   # (an op uses two of the four: its inputs alone are 512 MiB, twice the memory-side cache)
         out_h = np.empty_like(a)
         col_h = np.empty(n, dtype=np.float32)
 
